@@ -452,8 +452,8 @@ int vgpu_diag_stream(int32_t mode, const void* src, void* dst, uint64_t bytes, i
 int vgpu_scene_timing(vgpu_scene* scene, float* trace_ms, float* sort_ms, int32_t* launches);
 
 /* Traversal launch configuration (the autotuner's knobs).  Until the caller
- * sets one (or runs the autotuner), vgpu_scene_commit picks block 128, LDS
- * stack 12, 24 waves per CU, no sort for a static scene, and 64 / 8 / 20 /
+ * sets one (or runs the autotuner), vgpu_scene_commit picks block 64, LDS
+ * stack 12, 20 waves per CU, no sort for a static scene, and 64 / 8 / 20 /
  * no sort for a scene with motion keys. */
 typedef struct vgpu_trace_config {
     int32_t block;        /* threads per workgroup: 64, 128 or 256 */

@@ -194,8 +194,9 @@ __global__ __launch_bounds__(256) void k_pt_hit(PTView v, uint32_t pass, int cur
     const int prim = h0.x, g = h0.y;
     const float t = __int_as_float(h0.z), U = __int_as_float(h0.w), V = __int_as_float(h1.x), W = __int_as_float(h1.y);
     const DevGeom geo = v.sv.geoms[g];
-    const float4* tp = v.sv.tris + ((size_t)geo.tri_base + prim) * 3;
-    const F3 a = f3(tp[0]), bb = f3(tp[1]), c = f3(tp[2]);
+    const DevTri tp = v.sv.tris[(size_t)geo.tri_base + prim];
+    const F3 a = f3(tp.v[0][0], tp.v[0][1], tp.v[0][2]), bb = f3(tp.v[1][0], tp.v[1][1], tp.v[1][2]),
+             c = f3(tp.v[2][0], tp.v[2][1], tp.v[2][2]);
     const F3 P = f3((U * a.x + V * bb.x) + W * c.x, (U * a.y + V * bb.y) + W * c.y, (U * a.z + V * bb.z) + W * c.z);
     const F3 ng = cross(sub(bb, a), sub(c, a));
     const float nl = sqrtf(dot(ng, ng));

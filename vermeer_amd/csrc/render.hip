@@ -1048,8 +1048,9 @@ __device__ __forceinline__ int shade_pixel(int& next, const RenderView& rv, cons
         }
     } else {
         const float U = __int_as_float(h0.w), V = __int_as_float(h1.x), W = __int_as_float(h1.y);
-        const float4* tp = rv.sv.tris + ((size_t)geo.tri_base + prim) * 3;
-        const V3 a = from4(tp[0]), b = from4(tp[1]), c = from4(tp[2]);
+        const DevTri tp = rv.sv.tris[(size_t)geo.tri_base + prim];
+        const V3 a = v3(tp.v[0][0], tp.v[0][1], tp.v[0][2]), b = v3(tp.v[1][0], tp.v[1][1], tp.v[1][2]),
+                 c = v3(tp.v[2][0], tp.v[2][1], tp.v[2][2]);
         // hit attributes (builtin/geom/polymesh/trace.go:292-513)
         const float xs = fabs32(U * a.x) + fabs32(V * b.x) + fabs32(W * c.x);
         const float ys = fabs32(U * a.y) + fabs32(V * b.y) + fabs32(W * c.y);

@@ -213,26 +213,51 @@ int build_motion_mesh(MeshHost& m, int device) {
     return VGPU_OK;
 }
 
-void to_dev(const vgpu_qbvh_node& s, vgpu::DevNode& d) {
-    std::memcpy(d.lox, s.boxes, 24 * sizeof(float));   // rows lox, loy, loz, hix, hiy, hiz
-    for (int c = 0; c < 4; c++) d.children[c] = s.children[c];
-    d.axes[0] = (int32_t)s.axis0; d.axes[1] = (int32_t)s.axis1; d.axes[2] = (int32_t)s.axis2; d.axes[3] = 0;
+// A node in the device layout; false when a bound is NaN.
+bool to_dev(const vgpu_qbvh_node& s, vgpu::DevNode& d) {
+    constexpr int lo_row[3] = {vgpu::kRowLoX, vgpu::kRowLoY, vgpu::kRowLoZ};
+    constexpr int hi_row[3] = {vgpu::kRowHiX, vgpu::kRowHiY, vgpu::kRowHiZ};
+    int32_t swapped = 0;
+    bool ok = true;
+    for (int k = 0; k < 3; k++)
+        for (int c = 0; c < 4; c++) {
+            float lo = s.boxes[4 * k + c], hi = s.boxes[12 + 4 * k + c];
+            ok = ok && !std::isnan(lo) && !std::isnan(hi);
+            if (lo > hi) {
+                std::swap(lo, hi);
+                swapped |= 1 << (4 * k + c);
+            }
+            d.rows[lo_row[k]][c] = lo;
+            d.rows[hi_row[k]][c] = hi;
+        }
+    std::memcpy(d.rows[vgpu::kRowChildren], s.children, 16);
+    const int32_t ax[4] = {vgpu::kSignBit + (int32_t)s.axis0, vgpu::kSignBit + (int32_t)s.axis1,
+                           vgpu::kSignBit + (int32_t)s.axis2, swapped};
+    std::memcpy(d.rows[vgpu::kRowAxes], ax, 16);
+    return ok;
 }
 
-void append_motion_nodes(std::vector<float4>& out, const std::vector<vgpu_mqbvh_node>& topo, const std::vector<float>& boxes,
+// Appends a motion topology's nodes in the device layout; false when some box is not finite with lo <= hi.
+bool append_motion_nodes(std::vector<float4>& out, const std::vector<vgpu_mqbvh_node>& topo, const std::vector<float>& boxes,
                          int nkeys) {
     const size_t nn = topo.size();
+    bool ok = true;
     for (size_t i = 0; i < nn; i++) {
         float4 t0, t1;
         std::memcpy(&t0, topo[i].children, 16);
-        int32_t ax[4] = {topo[i].axis0, topo[i].axis1, topo[i].axis2, 0};
+        int32_t ax[4] = {vgpu::kSignBit + topo[i].axis0, vgpu::kSignBit + topo[i].axis1, vgpu::kSignBit + topo[i].axis2, 0};
         std::memcpy(&t1, ax, 16);
         out.push_back(t0); out.push_back(t1);
         for (int k = 0; k < nkeys; k++) {
             const float* b = &boxes[((size_t)k * nn + i) * 24];
-            for (int r = 0; r < 6; r++) out.push_back(make_float4(b[r * 4 + 0], b[r * 4 + 1], b[r * 4 + 2], b[r * 4 + 3]));
+            for (int r = 0; r < 6; r++) {
+                const float* row = b + 4 * (r % 2 == 0 ? r / 2 : 3 + r / 2);   // lo x, hi x, lo y, hi y, lo z, hi z
+                out.push_back(make_float4(row[0], row[1], row[2], row[3]));
+            }
+            for (int j = 0; j < 12; j++) ok = ok && std::isfinite(b[j]) && std::isfinite(b[12 + j]) && b[j] <= b[12 + j];
         }
     }
+    return ok;
 }
 
 template <class T>
@@ -786,28 +811,36 @@ int vgpu_scene_commit(vgpu_scene* s) {
         }
     }
     s->any_motion = maxKeys > 1;
-    // Default launch shape unless the caller chose one: static scenes run best at block 128 with a
-    // 12-entry LDS stack and 24 waves per CU; the motion kernel (about 120 VGPRs, four waves per
-    // SIMD) at block 256, 16 entries, 16 waves per CU.
-    if (!s->cfg_set) s->cfg = s->any_motion ? vgpu_trace_config{64, 8, 20, 0, 0} : vgpu_trace_config{128, 12, 24, 0, 0};
+    // Default launch shape unless the caller chose one: both kernels hold five waves per SIMD, so 20 waves
+    // per CU, with the LDS stack that measured fastest (figures at kExtLaunch and k_trace_wide_m5).
+    if (!s->cfg_set) s->cfg = s->any_motion ? vgpu_trace_config{64, 8, 20, 0, 0} : vgpu_trace_config{64, 12, 20, 0, 0};
 
     // Flatten into the device layout.
     std::vector<vgpu::DevNode> dnodes;
-    std::vector<float4> dtris, dmnodes, dmtris, dspheres;
+    std::vector<vgpu::DevTri> dtris;
+    std::vector<float4> dmnodes, dmtris, dspheres;
     std::vector<vgpu::DevGeom> dgeoms(nall);
+    bool near_far = true;
+    auto append_nodes = [&](const std::vector<vgpu_qbvh_node>& nodes) {
+        for (auto& nd : nodes) {
+            vgpu::DevNode d;
+            near_far = to_dev(nd, d) && near_far;
+            dnodes.push_back(d);
+        }
+    };
     {
-        size_t corners = 0;
+        size_t tris = 0;
         for (int slot = 0; slot < nall; slot++) {
             const MeshHost& m = s->meshes[s->order[slot]];
-            if (m.kind < vgpu::kXfInstance && !m.sphere && m.nkeys == 1) corners += (size_t)m.ntris * 3;
+            if (m.kind < vgpu::kXfInstance && !m.sphere && m.nkeys == 1) tris += m.ntris;
         }
-        dtris.reserve(corners);
+        dtris.reserve(tris);
     }
     if (!s->top_motion) {
-        for (auto& nd : s->top_nodes) { vgpu::DevNode d; to_dev(nd, d); dnodes.push_back(d); }
+        append_nodes(s->top_nodes);
     } else {
         s->view.top_mbase = 0;
-        append_motion_nodes(dmnodes, s->top_mnodes, s->top_mboxes, maxKeys);
+        near_far = append_motion_nodes(dmnodes, s->top_mnodes, s->top_mboxes, maxKeys) && near_far;
     }
     for (int slot = 0; slot < nall; slot++) {
         MeshHost& m = s->meshes[s->order[slot]];
@@ -825,20 +858,18 @@ int vgpu_scene_commit(vgpu_scene* s) {
             dspheres.push_back(make_float4(m.sphere_c[0], m.sphere_c[1], m.sphere_c[2], m.sphere_r));
         } else if (m.nkeys == 1) {
             g.node_base = (int32_t)dnodes.size();
-            for (auto& nd : m.nodes) { vgpu::DevNode d; to_dev(nd, d); dnodes.push_back(d); }
-            g.tri_base = (int32_t)(dtris.size() / 3);
+            append_nodes(m.nodes);
+            g.tri_base = (int32_t)dtris.size();
             const size_t base = dtris.size();
-            dtris.resize(base + (size_t)m.ntris * 3);
-            float4* out = dtris.data() + base;
-            parallel_ranges((size_t)m.ntris * 3, [&](size_t a, size_t b) {
-                for (size_t k = a; k < b; k++) {
-                    const float* v = m.vert(0, m.idxp_sorted[k]);
-                    out[k] = make_float4(v[0], v[1], v[2], 0.0f);
-                }
+            dtris.resize(base + m.ntris);
+            vgpu::DevTri* out = dtris.data() + base;
+            parallel_ranges(m.ntris, [&](size_t a, size_t b) {
+                for (size_t k = a; k < b; k++)
+                    for (int c = 0; c < 3; c++) std::memcpy(out[k].v[c], m.vert(0, m.idxp_sorted[3 * k + c]), 12);
             });
         } else {
             g.node_base = (int32_t)dmnodes.size();
-            append_motion_nodes(dmnodes, m.mnodes, m.mboxes, (int)m.nkeys);
+            near_far = append_motion_nodes(dmnodes, m.mnodes, m.mboxes, (int)m.nkeys) && near_far;
             g.tri_base = (int32_t)dmtris.size();
             const bool ref_idx = (m.flags & VGPU_MESH_MOTION_REFERENCE_INDEXING) != 0;
             for (uint32_t i = 0; i < m.ntris; i++) {
@@ -850,7 +881,7 @@ int vgpu_scene_commit(vgpu_scene* s) {
                     }
             }
         }
-        if (dtris.size() / 3 > 0x7fffffffull || dmtris.size() > 0x7fffffffull || dmnodes.size() > 0x7fffffffull)
+        if (dtris.size() > 0x7fffffffull || dmtris.size() > 0x7fffffffull || dmnodes.size() > 0x7fffffffull)
             return fail(VGPU_ERR_ARG, "scene too large for 32-bit offsets");
     }
     DeviceGuard dg(s->device);
@@ -982,13 +1013,8 @@ int vgpu_scene_commit(vgpu_scene* s) {
     s->view.spheres = s->d_spheres;
     s->view.top_motion = s->top_motion ? 1 : 0;
     s->view.top_keys = s->top_keys;
-    s->view.nan_free_boxes = 1;
-    for (const vgpu::DevNode& d : dnodes) {
-        float bx[24];
-        std::memcpy(bx, d.lox, sizeof(bx));
-        for (int k = 0; k < 24; k++)
-            if (std::isnan(bx[k])) s->view.nan_free_boxes = 0;
-    }
+    s->view.near_far = near_far && dnodes.size() * sizeof(vgpu::DevNode) < (1ull << 32) &&
+                       dmnodes.size() * sizeof(float4) < (1ull << 32);
     s->committed = true;
     return VGPU_OK;
 }

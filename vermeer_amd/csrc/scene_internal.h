@@ -112,7 +112,7 @@ struct vgpu_scene {
     bool any_motion = false;
 
     vgpu::DevNode* d_nodes = nullptr;
-    float4* d_tris = nullptr;
+    vgpu::DevTri* d_tris = nullptr;
     float4* d_mnodes = nullptr;
     float4* d_mtris = nullptr;
     vgpu::DevGeom* d_geoms = nullptr;

@@ -85,27 +85,12 @@ struct Box4 {
     bool h[4];
 };
 
-// FAST: every slab value is known not to be NaN (finite origin, finite non-zero 1/D, no NaN in
-// the node boxes).  MINPS/MAXPS then agree with IEEE min/max except for which zero of +0/-0
-// they return, and the entry distances are only ever compared, where +0 == -0, so the
-// hardware min/max (v_min3/v_max3) give the same hit flags and the same traversal.
-template <bool FAST>
 __device__ __forceinline__ void box4(const RayS& r, const float4& lx, const float4& ly, const float4& lz,
                                      const float4& hx, const float4& hy, const float4& hz, Box4& b) {
     const float lxa[4] = {lx.x, lx.y, lx.z, lx.w}, lya[4] = {ly.x, ly.y, ly.z, ly.w}, lza[4] = {lz.x, lz.y, lz.z, lz.w};
     const float hxa[4] = {hx.x, hx.y, hx.z, hx.w}, hya[4] = {hy.x, hy.y, hy.z, hy.w}, hza[4] = {hz.x, hz.y, hz.z, hz.w};
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        if (FAST) {
-            const float x1 = (lxa[c] - r.P[0]) * r.Dinv[0], x2 = (hxa[c] - r.P[0]) * r.Dinv[0];
-            const float y1 = (lya[c] - r.P[1]) * r.Dinv[1], y2 = (hya[c] - r.P[1]) * r.Dinv[1];
-            const float z1 = (lza[c] - r.P[2]) * r.Dinv[2], z2 = (hza[c] - r.P[2]) * r.Dinv[2];
-            const float tn = fmaxf(fmaxf(fmaxf(fminf(x1, x2), fminf(y1, y2)), fminf(z1, z2)), 0.0f);
-            const float tx = fminf(fminf(fmaxf(x1, x2), fmaxf(y1, y2)), fmaxf(z1, z2));
-            b.t[c] = tn;
-            b.h[c] = tn <= tx;
-            continue;
-        }
         float tmin, tmax;
         slab(lxa[c], hxa[c], r.P[0], r.Dinv[0], tmin, tmax, true);
         slab(lya[c], hya[c], r.P[1], r.Dinv[1], tmin, tmax, false);
@@ -113,6 +98,27 @@ __device__ __forceinline__ void box4(const RayS& r, const float4& lx, const floa
         const float tn = (0.0f > tmin) ? 0.0f : tmin;   // MAXPS X6,X0 with X0 = 0
         b.t[c] = tn;
         b.h[c] = tn <= tmax;                             // CMPPS $2 (ordered <=)
+    }
+}
+
+// The same four boxes given by their near and far planes: the lower or the upper bound of an axis,
+// whichever the direction's sign meets first.  For boxes with lo <= hi, a finite origin and a finite
+// non-zero 1/D no value is NaN, and rounding keeps the order of (lo - P) * Dinv and (hi - P) * Dinv, so
+// the near plane's value is intersectBoxes' smaller one.  MINPS/MAXPS then agree with IEEE min/max
+// except for which zero of +0/-0 they return, and the entry distances are only ever compared, where
+// +0 == -0: the same hit flags and the same traversal for 24 instructions less than sorting each pair.
+__device__ __forceinline__ void box4_near(const RayS& r, const float4& nx, const float4& ny, const float4& nz,
+                                          const float4& fx, const float4& fy, const float4& fz, Box4& b) {
+    const float nxa[4] = {nx.x, nx.y, nx.z, nx.w}, nya[4] = {ny.x, ny.y, ny.z, ny.w}, nza[4] = {nz.x, nz.y, nz.z, nz.w};
+    const float fxa[4] = {fx.x, fx.y, fx.z, fx.w}, fya[4] = {fy.x, fy.y, fy.z, fy.w}, fza[4] = {fz.x, fz.y, fz.z, fz.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const float tn = fmaxf(fmaxf(fmaxf((nxa[c] - r.P[0]) * r.Dinv[0], (nya[c] - r.P[1]) * r.Dinv[1]),
+                                     (nza[c] - r.P[2]) * r.Dinv[2]), 0.0f);
+        const float tx = fminf(fminf((fxa[c] - r.P[0]) * r.Dinv[0], (fya[c] - r.P[1]) * r.Dinv[1]),
+                               (fza[c] - r.P[2]) * r.Dinv[2]);
+        b.t[c] = tn;
+        b.h[c] = tn <= tx;
     }
 }
 
@@ -140,9 +146,20 @@ __device__ __forceinline__ int leaf_base(int32_t l) { return (int)((l & 0x7fffff
 __device__ __forceinline__ int leaf_count(int32_t l) { return (int)((l & 0xf) + 1); }
 
 // Ray quantities the watertight test reads: the shear constants and the permuted origin.
+// The axes are held as which of them is axis 0 and which is axis 1.
 struct TriRay {
     float S0, S1, S2, Pkx, Pky, Pkz;
-    int Kx, Ky, Kz;
+    bool x0, x1, y0, y1, z0, z1;
+    __device__ __forceinline__ float x(const float4& v) const { return x0 ? v.x : (x1 ? v.y : v.z); }
+    __device__ __forceinline__ float y(const float4& v) const { return y0 ? v.x : (y1 ? v.y : v.z); }
+    __device__ __forceinline__ float z(const float4& v) const { return z0 ? v.x : (z1 ? v.y : v.z); }
+    // from a pack_perm word; the three axes differ, so Kz's masks follow from the others without a compare
+    __device__ __forceinline__ void axes(int kp) {
+        const int Kx = (kp >> 7) & 3, Ky = (kp >> 9) & 3;
+        x0 = Kx == 0; x1 = Kx == 1;
+        y0 = Ky == 0; y1 = Ky == 1;
+        z0 = !(x0 || y0); z1 = !(x1 || y1);
+    }
 };
 
 
@@ -150,17 +167,21 @@ struct TriPre {
     float T, det, fU, fV, fW;
 };
 
-// The direction-sign bits and the permutation packed in one register: neg (bits 0-2, bit k set when
-// D[k] < 0), Kx (3-4), Ky (5-6), Kz (7-8).  The wide kernel keeps this instead of the separate fields
-// and the permuted origin, which it rebuilds from P when a leaf is tested.
-__device__ __forceinline__ int pack_perm(const RayS& r) { return r.neg | (r.Kx << 3) | (r.Ky << 5) | (r.Kz << 7); }
+// The direction-sign bits and the permutation packed in one register: bit kSignBit + k set when
+// D[k] < 0, then Kx, Ky, Kz in two bits each.  Nodes hold their split axes as kSignBit + axis, so the
+// sign bit of an axis is one bit-field extract; and the sign bits' values 16, 32 and 64 are the byte
+// offsets between a node's near and far rows (box4_near).
+__device__ __forceinline__ int pack_perm(const RayS& r) {
+    return (r.neg << kSignBit) | (r.Kx << 7) | (r.Ky << 9) | (r.Kz << 11);
+}
 __device__ __forceinline__ TriRay tri_ray_packed(const RayS& r, int kp) {
     TriRay q;
     q.S0 = r.S[0]; q.S1 = r.S[1]; q.S2 = r.S[2];
-    q.Kx = (kp >> 3) & 3; q.Ky = (kp >> 5) & 3; q.Kz = (kp >> 7) & 3;
-    q.Pkx = sel3(r.P[0], r.P[1], r.P[2], q.Kx);
-    q.Pky = sel3(r.P[0], r.P[1], r.P[2], q.Ky);
-    q.Pkz = sel3(r.P[0], r.P[1], r.P[2], q.Kz);
+    q.axes(kp);
+    const float4 P = make_float4(r.P[0], r.P[1], r.P[2], 0.0f);
+    q.Pkx = q.x(P);
+    q.Pky = q.y(P);
+    q.Pkz = q.z(P);
     return q;
 }
 
@@ -170,24 +191,25 @@ __device__ __forceinline__ TriRay tri_ray_packed(const RayS& r, int kp) {
 template <bool MOTION_BOUND>
 __device__ __forceinline__ bool tri_pre(const TriRay& q, const float4& v0, const float4& v1, const float4& v2, float bias,
                                         TriPre& p) {
-    const float AKz = sel3(v0.x, v0.y, v0.z, q.Kz) - q.Pkz;
-    const float BKz = sel3(v1.x, v1.y, v1.z, q.Kz) - q.Pkz;
-    const float CKz = sel3(v2.x, v2.y, v2.z, q.Kz) - q.Pkz;
-    const float Cx = (sel3(v2.x, v2.y, v2.z, q.Kx) - q.Pkx) - q.S0 * CKz;
-    const float By = (sel3(v1.x, v1.y, v1.z, q.Ky) - q.Pky) - q.S1 * BKz;
-    const float Cy = (sel3(v2.x, v2.y, v2.z, q.Ky) - q.Pky) - q.S1 * CKz;
-    const float Bx = (sel3(v1.x, v1.y, v1.z, q.Kx) - q.Pkx) - q.S0 * BKz;
-    const float Ax = (sel3(v0.x, v0.y, v0.z, q.Kx) - q.Pkx) - q.S0 * AKz;
-    const float Ay = (sel3(v0.x, v0.y, v0.z, q.Ky) - q.Pky) - q.S1 * AKz;
+    const float AKz = q.z(v0) - q.Pkz;
+    const float BKz = q.z(v1) - q.Pkz;
+    const float CKz = q.z(v2) - q.Pkz;
+    const float Cx = (q.x(v2) - q.Pkx) - q.S0 * CKz;
+    const float By = (q.y(v1) - q.Pky) - q.S1 * BKz;
+    const float Cy = (q.y(v2) - q.Pky) - q.S1 * CKz;
+    const float Bx = (q.x(v1) - q.Pkx) - q.S0 * BKz;
+    const float Ax = (q.x(v0) - q.Pkx) - q.S0 * AKz;
+    const float Ay = (q.y(v0) - q.Pky) - q.S1 * AKz;
     float fU = Cx * By - Cy * Bx;
     float fV = Ax * Cy - Ay * Cx;
     float fW = Bx * Ay - By * Ax;
-    if (fU == 0.0f || fV == 0.0f || fW == 0.0f) {
+    if (fminf(fminf(absf(fU), absf(fV)), absf(fW)) == 0.0f) {   // some edge function is zero (NaNs aside)
         fU = (float)((double)Cx * (double)By - (double)Cy * (double)Bx);
         fV = (float)((double)Ax * (double)Cy - (double)Ay * (double)Cx);
         fW = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
     }
-    if ((fU < 0.0f || fV < 0.0f || fW < 0.0f) && (fU > 0.0f || fV > 0.0f || fW > 0.0f)) return false;
+    // some edge function negative and another positive; fmin and fmax pass over NaNs as the comparisons do
+    if (fminf(fminf(fU, fV), fW) < 0.0f && fmaxf(fmaxf(fU, fV), fW) > 0.0f) return false;
     const float det = fU + fV + fW;
     if (det == 0.0f) return false;
     const float T = q.S2 * (fU * AKz + fV * BKz + fW * CKz);
@@ -228,6 +250,12 @@ __device__ __forceinline__ bool tri_test_q(RayS& r, const TriRay& q, const float
 
 
 
+__device__ __forceinline__ void load_tri(const DevTri* __restrict__ p, float4& v0, float4& v1, float4& v2) {
+    v0 = make_float4(p->v[0][0], p->v[0][1], p->v[0][2], 0.0f);
+    v1 = make_float4(p->v[1][0], p->v[1][1], p->v[1][2], 0.0f);
+    v2 = make_float4(p->v[2][0], p->v[2][1], p->v[2][2], 0.0f);
+}
+
 __device__ __forceinline__ float4 lerp4(const float4& a, const float4& b, float t) {
     const float s = 1.0f - t;
     return make_float4(s * a.x + t * b.x, s * a.y + t * b.y, s * a.z + t * b.z, s * a.w + t * b.w);
@@ -250,17 +278,35 @@ struct NodeData {
     int ax[3];
 };
 
+__device__ __forceinline__ void swap_lane(float& a, float& b, bool sw) {
+    const float t = a;
+    a = sw ? b : a;
+    b = sw ? t : b;
+}
+
+// A static node with its boxes as the reference holds them (the lanes that the upload put in order,
+// DevNode::axes[3], swapped back), for box4.
 __device__ __forceinline__ void fetch_static(const DevNode* __restrict__ nodes, int idx, NodeData& nd) {
     const float4* p = reinterpret_cast<const float4*>(nodes + idx);
-    nd.lx = p[0]; nd.ly = p[1]; nd.lz = p[2]; nd.hx = p[3]; nd.hy = p[4]; nd.hz = p[5];
-    const int4 c = reinterpret_cast<const int4*>(p)[6];
-    const int4 a = reinterpret_cast<const int4*>(p)[7];
+    nd.lx = p[kRowLoX]; nd.ly = p[kRowLoY]; nd.lz = p[kRowLoZ];
+    nd.hx = p[kRowHiX]; nd.hy = p[kRowHiY]; nd.hz = p[kRowHiZ];
+    const int4 c = reinterpret_cast<const int4*>(p)[kRowChildren];
+    const int4 a = reinterpret_cast<const int4*>(p)[kRowAxes];
     nd.ch[0] = c.x; nd.ch[1] = c.y; nd.ch[2] = c.z; nd.ch[3] = c.w;
     nd.ax[0] = a.x; nd.ax[1] = a.y; nd.ax[2] = a.z;
+    if (a.w != 0) {
+        const int m = a.w;
+        swap_lane(nd.lx.x, nd.hx.x, m & 1); swap_lane(nd.lx.y, nd.hx.y, m & 2);
+        swap_lane(nd.lx.z, nd.hx.z, m & 4); swap_lane(nd.lx.w, nd.hx.w, m & 8);
+        swap_lane(nd.ly.x, nd.hy.x, m & 16); swap_lane(nd.ly.y, nd.hy.y, m & 32);
+        swap_lane(nd.ly.z, nd.hy.z, m & 64); swap_lane(nd.ly.w, nd.hy.w, m & 128);
+        swap_lane(nd.lz.x, nd.hz.x, m & 256); swap_lane(nd.lz.y, nd.hz.y, m & 512);
+        swap_lane(nd.lz.z, nd.hz.z, m & 1024); swap_lane(nd.lz.w, nd.hz.w, m & 2048);
+    }
 }
 
 // Motion node (qbvh/motionintersect.go:47-49): the boxes lerped per key and tested one axis at a
-// time, in the slab order of box4<false>, so only one axis of both keys is live at once.
+// time, in the slab order of box4, so only one axis of both keys is live at once.
 __device__ __forceinline__ void box_motion(const RayS& r, const float4* __restrict__ mnodes, int base, int node,
                                            int nkeys, int key, int key2, float time, NodeData& nd, Box4& b) {
     const float4* p = mnodes + base + (size_t)node * (2 + 6 * nkeys);
@@ -273,7 +319,7 @@ __device__ __forceinline__ void box_motion(const RayS& r, const float4* __restri
     float tmin[4], tmax[4];
 #pragma unroll
     for (int ax = 0; ax < 3; ax++) {
-        const float4 lo = lerp4(b0[ax], b1[ax], time), hi = lerp4(b0[3 + ax], b1[3 + ax], time);
+        const float4 lo = lerp4(b0[2 * ax], b1[2 * ax], time), hi = lerp4(b0[2 * ax + 1], b1[2 * ax + 1], time);
         const float la[4] = {lo.x, lo.y, lo.z, lo.w}, ha[4] = {hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
         for (int ch = 0; ch < 4; ch++) slab(la[ch], ha[ch], r.P[ax], r.Dinv[ax], tmin[ch], tmax[ch], ax == 0);
@@ -283,6 +329,43 @@ __device__ __forceinline__ void box_motion(const RayS& r, const float4* __restri
         const float tn = (0.0f > tmin[ch]) ? 0.0f : tmin[ch];
         b.t[ch] = tn;
         b.h[ch] = tn <= tmax[ch];
+    }
+}
+
+// The same for a node whose boxes are finite and ordered, as near and far planes (box4_near): the lerp
+// keeps lo <= hi.  A row pair starts on 32 bytes, so the far plane's offset is the near one's with bit 4
+// flipped; byte offsets fit 32 bits (SceneView::near_far).
+__device__ __forceinline__ void box_motion_near(const RayS& r, int kp, const float4* __restrict__ mnodes, int base,
+                                                int node, int nkeys, int key, int key2, float time, int (&ch)[4],
+                                                int (&ax)[3], Box4& b) {
+    const char* mp = reinterpret_cast<const char*>(mnodes);
+    const uint32_t o = ((uint32_t)base + (uint32_t)node * (uint32_t)(2 + 6 * nkeys)) << 4;
+    const int4 c = *reinterpret_cast<const int4*>(mp + o);
+    const int4 a = *reinterpret_cast<const int4*>(mp + o + 16);
+    ch[0] = c.x; ch[1] = c.y; ch[2] = c.z; ch[3] = c.w;
+    ax[0] = a.x; ax[1] = a.y; ax[2] = a.z;
+    const uint32_t o0 = o + 96u * (uint32_t)key, o1 = o + 96u * (uint32_t)key2;
+    float tn[4], tx[4];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const uint32_t s = ((uint32_t)kp >> k) & 16u;
+        auto plane = [&](uint32_t flip) {
+            return lerp4(*reinterpret_cast<const float4*>(mp + ((o0 | s) ^ flip) + 32 + 32 * k),
+                         *reinterpret_cast<const float4*>(mp + ((o1 | s) ^ flip) + 32 + 32 * k), time);
+        };
+        const float4 nv = plane(0u), fv = plane(16u);
+        const float na[4] = {nv.x, nv.y, nv.z, nv.w}, fa[4] = {fv.x, fv.y, fv.z, fv.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float x = (na[j] - r.P[k]) * r.Dinv[k], y = (fa[j] - r.P[k]) * r.Dinv[k];
+            tn[j] = k == 0 ? x : fmaxf(tn[j], x);
+            tx[j] = k == 0 ? y : fminf(tx[j], y);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        b.t[j] = fmaxf(tn[j], 0.0f);
+        b.h[j] = b.t[j] <= tx[j];
     }
 }
 
@@ -345,15 +428,77 @@ __device__ __forceinline__ int next_geom(const SceneView& sv, const float4* __re
     return 0;
 }
 
-// The traversal, one ray per lane and one traversal step (a node or a leaf) per loop iteration.
-// The triangles of the leaves popped in a step are tested by the whole wavefront: lane l
-// owns a leaf of c_l triangles, the sum of the c_l triangle tests is dealt out over the 64
-// lanes (consecutive lanes take consecutive triangles of one leaf, so the loads coalesce),
-// and each lane reads the owning ray's shear constants with a cross-lane shuffle.  That part
-// of the watertight test does not read the closest distance; the owner then runs the full
-// test, in leaf order, on the triangles that passed it, which accepts the same triangles in
-// the same order as testing every triangle of the leaf in turn.  Lanes whose ray is finished
-// stay in the loop as workers until the whole wavefront is done.
+// ---- cross-lane helpers of the wavefront-wide leaf tests
+
+// Sums / maxima over lanes 0..lane on the DPP row shifts and broadcasts: six VALU operations with no
+// LDS round trip.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int x) {   // lanes without a source read 0
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_scan_add(int x) {
+    x += dpp0<0x111, 0xf>(x);
+    x += dpp0<0x112, 0xf>(x);
+    x += dpp0<0x114, 0xf>(x);
+    x += dpp0<0x118, 0xf>(x);
+    x += dpp0<0x142, 0xa>(x);
+    x += dpp0<0x143, 0xc>(x);
+    return x;
+}
+__device__ __forceinline__ int wave_scan_max(int x) {   // x >= 0
+    x = max(x, dpp0<0x111, 0xf>(x));
+    x = max(x, dpp0<0x112, 0xf>(x));
+    x = max(x, dpp0<0x114, 0xf>(x));
+    x = max(x, dpp0<0x118, 0xf>(x));
+    x = max(x, dpp0<0x142, 0xa>(x));
+    x = max(x, dpp0<0x143, 0xc>(x));
+    return x;
+}
+// LDS words that other lanes of the wavefront read or write (a wavefront's LDS operations stay in order;
+// relaxed atomics keep the compiler from assuming a lane's own stores).
+__device__ __forceinline__ void lds_put(int* p, int x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); }
+__device__ __forceinline__ int lds_get(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); }
+// x of lane (addr / 4); every lane of the wavefront takes part.
+__device__ __forceinline__ float lane_f(int addr, float x) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
+}
+__device__ __forceinline__ int lane_i(int addr, int x) { return __builtin_amdgcn_ds_bpermute(addr, x); }
+
+// What a lane does next, beside node indices (>= 0) and mesh leaves (< kIdle).
+constexpr int kPop = -1;    // take the next stack entry (also the encoding of an empty child)
+constexpr int kIdle = -2;   // no ray, or its traversal has ended
+
+// The wavefront tests the leaves its lanes hold once kLeafRatio times as many lanes hold a leaf as hold a
+// node: few waiting leaves cost less than a node step with idle lanes while most lanes hold nodes, more as
+// the node lanes run out.  Measured on the icosphere field (2.1M bounce rays) / the 1M-triangle room (one
+// plain 1024^2 pass) / the box of spheres (320 x 199, depth 5), in us: ratio 3: 703 / 8282 / 1780, 5: 705 /
+// 8448 / 1799, 8: 704 / 8713 / 1823; a fixed count of 2 lanes: 725 / 9044 / 1880, 4: 726 / 8564 / 1890, 10:
+// 743 / 8211 / 2030.
+constexpr int kLeafRatio = 3;
+
+// The traversal, one ray per lane.  A lane holds the node it visits next, a leaf of triangles it has
+// popped, or nothing; every turn of the loop the wavefront either steps all lanes that hold nodes (box
+// test, push) or tests all leaves held (kLeafRatio), so that neither runs for a few lanes while many wait;
+// lanes without either pop up to their next entry that is not culled.  The order of steps within each ray
+// is the reference's, whatever the other lanes do.
+//
+// What bounds it is VALU issue: 2.1M bounce rays in the icosphere field took 4.4e8 VALU instructions, 80%
+// of the issue slots of 902 us, when every turn ran both phases; now 3.0e8 and 65% of 703 us (2.98
+// Grays/s), the rest waiting for nodes and triangles beyond L2.  Hence the forms below: near and far planes
+// by address instead of sorted pairs (box4_near), stack positions as byte offsets summed from hit flags,
+// one 8-byte LDS entry per push, DPP scans, the workers' results handed to the owners instead of a second
+// test, and the geom changes kept out of the pop loop.
+//
+// Leaf tests are dealt out over the wavefront: an inclusive prefix sum of the leaf sizes runs over the
+// lanes, work item w belongs to the last lane whose items start at or before w (each owner marks its
+// first slot in LDS, a running maximum spreads the mark), and the lane working on it reads the owner's
+// ray with cross-lane shuffles.  Consecutive lanes take consecutive triangles of one leaf, so the loads
+// coalesce.  That part of the watertight test does not read the closest distance; the owner then accepts
+// the triangles that passed, in leaf order and with the values that the worker computed, which takes the
+// same triangles in the same order as the reference's loop.
+//
+// A lane whose ray has ended idles (and works in the leaf tests) until refill_min lanes are idle; then
+// the idle lanes write their results and take the next rays of the wavefront together.
 // MOTION: the scene has motion keys (a motion top level and/or moving meshes); node boxes
 // (qbvh/motionintersect.go:47-49) and triangles of moving meshes (trace.go:547-554) are
 // interpolated at the ray's time.
@@ -366,26 +511,30 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                                            const uint32_t* __restrict__ n_dev, const uint32_t* __restrict__ perm,
                                            int refill_min) {
     static_assert(BLOCK % 64 == 0, "whole wavefronts");
-    __shared__ float sT[LDS * BLOCK];
-    __shared__ int32_t sN[LDS * BLOCK];
+    static_assert(LDS >= 4, "a node step's pushes are checked against LDS - 3");
+    constexpr int kEntry = BLOCK * 8;             // bytes from one stack entry of a lane to the next
+    constexpr int kNoRay = -1;
+    __shared__ uint2 stack_lds[LDS * BLOCK];      // {T bits, node}, entry-major: lanes never conflict on a bank
+    __shared__ int owner[BLOCK];                  // written by one lane, read by another of its wavefront
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const uint64_t gtid = (uint64_t)blockIdx.x * BLOCK + tid;
     const uint64_t nthr = (uint64_t)gridDim.x * BLOCK;
-    Stack<BLOCK, LDS> st;
-    st.sT = sT + tid; st.sN = sN + tid;
-    st.gT = spT; st.gN = spN; st.gstride = nthr; st.gofs = (uint32_t)gtid;
+    const int bottom = tid * 8;                   // the lane's empty stack: entry i at bottom + i * kEntry
+
+    auto spill = [&](int sp) { return (uint64_t)((uint32_t)sp / kEntry - LDS) * nthr + (uint32_t)gtid; };
+    auto push = [&](int sp, float T, int32_t node) {
+        if (sp < LDS * kEntry) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + sp) = make_uint2(__float_as_uint(T), (uint32_t)node);
+        else { const uint64_t o = spill(sp); spT[o] = T; spN[o] = node; }
+    };
 
     if (n_dev) n = min(n, (uint64_t)*n_dev);
-    // Rays of this wavefront: v = 0, 1, 2, ... -> ray wave0 + (v / 64) * nthr + v % 64 (increasing
-    // in v).  A lane whose ray is finished idles (and serves as a worker in the leaf tests) until
-    // refill_min lanes are idle; then the idle lanes write their results and take the next rays
-    // of the wavefront together, so the ray set-up runs once for many lanes.
-    const uint64_t wave0 = gtid - (uint64_t)lane;
+    // Rays of this wavefront: v = 0, 1, 2, ... -> ray wave0 + (v / 64) * nthr + v % 64 (increasing in v).
+    const uint64_t wave0 = (uint64_t)blockIdx.x * BLOCK + (uint32_t)__builtin_amdgcn_readfirstlane(tid & ~63);
     uint32_t cursor = 0;
-    bool done = true, live = false, ok = true, fast = false;
-    uint32_t ri = 0;   // launches hold fewer than 2^32 rays
-    int kp = 0;   // pack_perm of the current ray
+    bool ok = true, fast = false;
+    int ri = kNoRay;                              // launches hold fewer than 2^32 rays; ~0 is never one
+    int kp = 0;                                   // pack_perm of the current ray
     RayS r;
     r.P[0] = 0.0f; r.P[1] = 0.0f; r.P[2] = 0.0f; r.tclosest = 0.0f; r.time = 0.0f;
     {
@@ -395,26 +544,27 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     int nodesT = 0, leafsT = 0, trisT = 0, maxDepth = 0;
     int best_geom = -1, best_prim = -1;
     float bu = 0.0f, bv = 0.0f, bw = 0.0f;
-    int mesh_base = 0, gcur = 0, gend = 0;   // mesh_base 0: in the scene level, else inside geom gcur
-    // A motion top level starts a geom's stack at the popped leaf's own slot, which can be 0, so
-    // motion scenes keep a separate flag (qbvh/motionintersect.go:99-103 against intersect.go:219-226).
+    // The level traversed: the scene's (base == bottom, in_mesh false) or geom gcur's, whose stack starts
+    // at base.  A motion top level starts it at the popped leaf's own slot, a static one above it
+    // (qbvh/motionintersect.go:99-103 against intersect.go:219-226).
     const bool top_motion = MOTION && sv.top_motion;
-    bool in_mesh_m = false;
-#define VGPU_IN_MESH (MOTION ? in_mesh_m : mesh_base != 0)
+    bool in_mesh = false;
+    int base = bottom, gcur = 0, gend = 0;
     DevGeom g = {0, 0, 1, 0.0f};
-    int sp = 0;
+    int sp = bottom;
+    int cur = kIdle;
     while (true) {
-        const uint64_t dm = __ballot(done);
+        const uint64_t dm = __ballot(cur == kIdle);
         const uint64_t next = wave0 + (uint64_t)(cursor >> 6) * nthr + (cursor & 63u);
         const bool more = next < n;
         if (more ? __popcll(dm) >= refill_min : dm == ~0ull) {
-            if (done) {
-                if (live) {
+            if (cur == kIdle) {
+                if (ri != kNoRay) {
                     if (best_prim == -2) {   // the stack overflowed
                         atomicOr(err, 1);
                         best_geom = -1; best_prim = -1;
                     }
-                    const uint64_t oi = perm ? (uint64_t)perm[ri] : (uint64_t)ri;
+                    const uint64_t oi = perm ? (uint64_t)perm[(uint32_t)ri] : (uint64_t)(uint32_t)ri;
                     if (EXT) {
                         hits[2 * oi] = make_int4(best_prim, best_geom, __float_as_int(r.tclosest), __float_as_int(bu));
                         hits[2 * oi + 1] = make_int4(__float_as_int(bv), __float_as_int(bw), 0, 0);
@@ -423,258 +573,238 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                         if (geoms_out) geoms_out[oi] = best_geom;
                     }
                     if (COUNTERS) counters[oi] = make_int4(nodesT, leafsT, trisT, maxDepth);
-                    live = false;
+                    ri = kNoRay;
                 }
                 if (more) {
                     const uint32_t v = cursor + (uint32_t)__popcll(dm & ((1ull << lane) - 1ull));
                     const uint64_t rnext = wave0 + (uint64_t)(v >> 6) * nthr + (v & 63u);
-                    live = rnext < n;
-                    ri = (uint32_t)rnext;
-                    if (live) {
-                        const float4 ra = rays[2 * ri], rb4 = rays[2 * ri + 1];
+                    ok = true;
+                    if (rnext < n) {
+                        ri = (int)(uint32_t)rnext;
+                        const float4 ra = rays[2 * rnext], rb4 = rays[2 * rnext + 1];
                         r.P[0] = ra.x; r.P[1] = ra.y; r.P[2] = ra.z; r.tclosest = ra.w;
                         const float D[3] = {rb4.x, rb4.y, rb4.z};
                         r.time = rb4.w;
                         ray_setup(r, D);
                         kp = pack_perm(r);
-                        ok = true;
                         for (int k = 0; k < 3; k++)
                             ok = ok && absf(r.P[k]) < INFINITY && absf(r.Dinv[k]) < INFINITY && r.Dinv[k] != 0.0f;
+                        if (MOTION) ok = ok && absf(r.time) < 1e20f;   // time * keys stays finite
                         nodesT = 0; leafsT = 0; trisT = 0; maxDepth = 0;
                         best_geom = -1; best_prim = -1;
                         bu = 0.0f; bv = 0.0f; bw = 0.0f;
-                        mesh_base = 0;
-                        in_mesh_m = false;
-                        st.store(0, r.tclosest, 0);
-                        sp = 1;
-                        done = false;
-                    } else {
-                        ok = true;
+                        in_mesh = false;
+                        base = bottom;
+                        sp = bottom;
+                        cur = 0;   // the root, whose entry distance is tclosest itself: never culled
                     }
                 }
             }
             if (!more) break;
             cursor += (uint32_t)__popcll(dm);
-            // motion boxes are interpolated, and 0 * inf there gives NaN: the exact form only
-            fast = !MOTION && sv.nan_free_boxes && __all(ok ? 1 : 0) != 0;
-        }
-        bool pend = false;   // this lane popped a triangle leaf: [lbase, lbase + lcount) of geom gcur
-        int lbase = 0, lcount = 0;
-        if (!done) {
-            do {
-                if (VGPU_IN_MESH && sp == mesh_base) {
-                    // PolyMesh.Trace returned; Scene.TraceElems moves to the leaf's next geom (scene.go:65-75)
-                    gcur++;
-                    const int ng = next_geom<SHADOW>(sv, rays, ri, r, gcur, gend, g, best_geom, best_prim, bu, bv, bw);
-                    if (ng == 2) { done = true; break; }
-                    if (ng == 1) {
-                        st.store(mesh_base, r.tclosest, 0);
-                        sp = mesh_base + 1;
-                        break;
-                    }
-                    sp = top_motion ? mesh_base : mesh_base - 1;
-                    mesh_base = 0;
-                    in_mesh_m = false;
-                }
-                if (sp == 0) { done = true; break; }
-                sp--;
-                float T; int32_t node;
-                st.load(sp, T, node);
-                if (r.tclosest < T || node == -1) break;
-                if (node >= 0) {
-                    if (COUNTERS) nodesT++;
-                    NodeData nd;
-                    Box4 b;
-                    if constexpr (MOTION) {
-                        const bool mnode = in_mesh_m ? g.nkeys > 1 : top_motion;
-                        if (mnode) {
-                            const int nk = in_mesh_m ? g.nkeys : sv.top_keys;
-                            int k0, k1;
-                            float t;
-                            motion_keys(r.time, nk, k0, k1, t);
-                            box_motion(r, sv.mnodes, in_mesh_m ? g.node_base : sv.top_mbase, node, nk, k0, k1, t, nd, b);
-                        } else {
-                            fetch_static(sv.nodes, in_mesh_m ? g.node_base + node : node, nd);
-                            box4<false>(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
-                        }
-                    } else {
-                        fetch_static(sv.nodes, mesh_base != 0 ? g.node_base + node : node, nd);
-                        if (fast) box4<true>(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
-                        else box4<false>(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
-                    }
-                    // Push order of qbvh/intersect.go:137-216 (same as motionintersect.go:53-97): the
-                    // children are pushed as two pairs; rank(c) is child c's position in that sequence.
-                    // Hit children are stored compacted in rank order, i.e. exactly the entries the
-                    // reference leaves below its stack top.
-                    const int n0 = (kp >> nd.ax[0]) & 1;
-                    const int n1 = (kp >> nd.ax[1]) & 1;
-                    const int n2 = (kp >> nd.ax[2]) & 1;
-                    const int gA = n0 ? 0 : 2, gB = 2 - gA;
-                    const int rk0 = gA + (n1 ^ 1), rk1 = gA + n1, rk2 = gB + (n2 ^ 1), rk3 = gB + n2;
-                    const int m = (b.h[0] ? 1 << rk0 : 0) | (b.h[1] ? 1 << rk1 : 0) | (b.h[2] ? 1 << rk2 : 0) |
-                                  (b.h[3] ? 1 << rk3 : 0);
-                    if (sp + 4 > VGPU_MAX_STACK) {   // conservative: the reference writes up to 4 slots here
-                        best_prim = -2;
-                        done = true;
-                        break;
-                    }
-                    if (b.h[0]) st.store(sp + __popc(m & ((1 << rk0) - 1)), b.t[0], nd.ch[0]);
-                    if (b.h[1]) st.store(sp + __popc(m & ((1 << rk1) - 1)), b.t[1], nd.ch[1]);
-                    if (b.h[2]) st.store(sp + __popc(m & ((1 << rk2) - 1)), b.t[2], nd.ch[2]);
-                    if (b.h[3]) st.store(sp + __popc(m & ((1 << rk3) - 1)), b.t[3], nd.ch[3]);
-                    sp += __popc(m);
-                    if (COUNTERS) maxDepth = max(maxDepth, sp);
-                } else {
-                    const int base = leaf_base(node), count = leaf_count(node);
-                    if (COUNTERS) leafsT++;
-                    if (VGPU_IN_MESH) {
-                        if (COUNTERS) trisT += count;
-                        pend = true;
-                        lbase = base;
-                        lcount = count;
-                    } else {
-                        // Scene.TraceElems: geoms [base, base+count) (scene.go:61-78)
-                        const int mb = top_motion ? sp : sp + 1;
-                        if (mb >= VGPU_MAX_STACK) { best_prim = -2; done = true; break; }
-                        gcur = base; gend = base + count;
-                        const int ng = next_geom<SHADOW>(sv, rays, ri, r, gcur, gend, g, best_geom, best_prim, bu, bv, bw);
-                        if (ng == 2) { done = true; break; }
-                        if (ng == 1) {
-                            mesh_base = mb;
-                            in_mesh_m = true;
-                            st.store(mesh_base, r.tclosest, 0);
-                            sp = mesh_base + 1;
-                        }
-                    }
-                }
-            } while (false);
+            fast = sv.near_far && __all(ok ? 1 : 0) != 0;
         }
 
-        const uint64_t pm = __ballot(pend);
-        if (pm != 0 && __ballot(pend && lcount > 2) == 0) {
-            // Leaves of one or two triangles only: each owner tests its own (dealing them out
-            // costs more than two tests).
-            if (pend) {
-                int idx = -1;
-                float U = 0.0f, V = 0.0f, W = 0.0f;
-                const TriRay q = tri_ray_packed(r, kp);
-                if (MOTION && g.nkeys > 1) {
-                    int k0, k1;
-                    float t;
-                    motion_keys(r.time, g.nkeys, k0, k1, t);
-                    const float4* tp = sv.mtris + g.tri_base + (size_t)lbase * 3 * g.nkeys;
-                    for (int i = 0; i < lcount; i++) {
-                        float4 v0, v1, v2;
-                        motion_tri(tp + (size_t)i * 3 * g.nkeys, k0, k1, t, v0, v1, v2);
-                        if (tri_test_q<true>(r, q, v0, v1, v2, g.ray_bias, U, V, W)) idx = lbase + i;
-                    }
+        // Pop: up to the next entry of the level that is not culled (a culled entry and an empty child both
+        // leave kPop).
+        while (cur == kPop && sp != base) {
+            sp -= kEntry;
+            float T; int32_t node;
+            if (sp < LDS * kEntry) {
+                const uint2 e = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(stack_lds) + sp);
+                T = __uint_as_float(e.x); node = (int32_t)e.y;
+            } else {
+                const uint64_t o = spill(sp);
+                T = spT[o]; node = spN[o];
+            }
+            cur = r.tclosest < T ? kPop : node;
+            if (COUNTERS && cur < kIdle) { leafsT++; if (in_mesh) trisT += leaf_count(cur); }
+        }
+        // Ends of levels, and the scene level's leaves: lanes that leave a mesh for the scene level pop there
+        // in the next turn.
+        const bool turn = cur == kPop || (cur < kIdle && !in_mesh);
+        if (__ballot(turn) != 0) {
+            if (turn) {
+                if (cur == kPop && !in_mesh) {
+                    cur = kIdle;
                 } else {
-                    const float4* tp = sv.tris + ((size_t)g.tri_base + lbase) * 3;
-                    for (int i = 0; i < lcount; i++)
-                        if (tri_test_q<false>(r, q, tp[3 * i], tp[3 * i + 1], tp[3 * i + 2], g.ray_bias, U, V, W))
-                            idx = lbase + i;
-                }
-                if (idx >= 0) {
-                    best_geom = gcur; best_prim = idx; bu = U; bv = V; bw = W;
-                    if (SHADOW) done = true;
-                }
-            }
-        } else if (pm != 0) {
-            // Deal the leaves' triangle tests out over the wavefront: inclusive prefix sum of the
-            // counts; work item w belongs to the first lane whose prefix exceeds w.
-            const int c = pend ? lcount : 0;
-            int pin = c;
-            for (int d = 1; d < 64; d <<= 1) {
-                const int y = __shfl_up(pin, d);
-                if (lane >= d) pin += y;
-            }
-            const int total = __shfl(pin, 63);
-            const int pex = pin - c;
-            // first triangle of the leaf: a triangle index (static) or a float4 offset (moving mesh)
-            const bool mv = MOTION && g.nkeys > 1;
-            const int tb = mv ? g.tri_base + lbase * 3 * g.nkeys : g.tri_base + lbase;
-            const TriRay q = tri_ray_packed(r, kp);
-            const int kpack = q.Kx | (q.Ky << 2) | (q.Kz << 4);
-            const float bias = g.ray_bias;
-            uint32_t cand = 0;   // owner: leaf triangles that passed the distance-free part of the test
-            for (int k0 = 0; k0 < total; k0 += 64) {
-                const int w = k0 + lane;
-                int o = 0;
-#pragma unroll
-                for (int s = 32; s >= 1; s >>= 1)
-                    if (__shfl(pin, o + s - 1) <= w) o += s;
-                const int i = w - __shfl(pex, o);
-                TriRay oq;
-                oq.S0 = __shfl(q.S0, o); oq.S1 = __shfl(q.S1, o); oq.S2 = __shfl(q.S2, o);
-                oq.Pkx = __shfl(q.Pkx, o); oq.Pky = __shfl(q.Pky, o); oq.Pkz = __shfl(q.Pkz, o);
-                const int ok = __shfl(kpack, o);
-                oq.Kx = ok & 3; oq.Ky = (ok >> 2) & 3; oq.Kz = (ok >> 4) & 3;
-                const float obias = __shfl(bias, o);
-                const int otb = __shfl(tb, o);
-                bool pass = false;
-                if constexpr (MOTION) {
-                    const int onk = __shfl(mv ? g.nkeys : 1, o);
-                    const float otime = __shfl(r.time, o);
-                    if (w < total) {
-                        TriPre pr;
-                        if (onk > 1) {
-                            int k0, k1;
-                            float t;
-                            motion_keys(otime, onk, k0, k1, t);
-                            float4 v0, v1, v2;
-                            motion_tri(sv.mtris + otb + (size_t)i * 3 * onk, k0, k1, t, v0, v1, v2);
-                            pass = tri_pre<true>(oq, v0, v1, v2, obias, pr);
-                        } else {
-                            const float4* tp = sv.tris + (size_t)(otb + i) * 3;
-                            pass = tri_pre<false>(oq, tp[0], tp[1], tp[2], obias, pr);
-                        }
+                    int mb = base;
+                    if (cur == kPop) {
+                        gcur++;   // PolyMesh.Trace returned; Scene.TraceElems moves to the leaf's next geom (scene.go:65-75)
+                    } else {      // Scene.TraceElems: the geoms of a top-level leaf (scene.go:61-78)
+                        mb = top_motion ? sp : sp + kEntry;
+                        gcur = leaf_base(cur); gend = gcur + leaf_count(cur);
                     }
-                } else if (w < total) {
-                    const float4* tp = sv.tris + (size_t)(otb + i) * 3;
-                    TriPre pr;
-                    pass = tri_pre<false>(oq, tp[0], tp[1], tp[2], obias, pr);
-                }
-                const uint64_t cm = __ballot(pass);
-                if (pend && cm != 0) {
-                    const int s0 = max(pex, k0), e0 = min(pin, k0 + 64);
-                    if (e0 > s0)
-                        cand |= (uint32_t)((cm >> (s0 - k0)) & ((1ull << (e0 - s0)) - 1ull)) << (s0 - pex);
-                }
-            }
-            if (cand != 0) {
-                // the owner's sequential pass over the candidates, in leaf order (trace.go:108-122)
-                int idx = -1;
-                float U = 0.0f, V = 0.0f, W = 0.0f;
-                if (mv) {
-                    int k0, k1;
-                    float t;
-                    motion_keys(r.time, g.nkeys, k0, k1, t);
-                    while (cand != 0) {
-                        const int i = __ffs(cand) - 1;
-                        cand &= cand - 1;
-                        float4 v0, v1, v2;
-                        motion_tri(sv.mtris + tb + (size_t)i * 3 * g.nkeys, k0, k1, t, v0, v1, v2);
-                        if (tri_test_q<true>(r, q, v0, v1, v2, g.ray_bias, U, V, W)) idx = lbase + i;
+                    if (mb >= VGPU_MAX_STACK * kEntry) {
+                        best_prim = -2;
+                        cur = kIdle;
+                    } else {
+                        const int ng = next_geom<SHADOW>(sv, rays, (uint32_t)ri, r, gcur, gend, g, best_geom, best_prim, bu, bv, bw);
+                        in_mesh = ng == 1;
+                        base = in_mesh ? mb : bottom;
+                        sp = in_mesh || top_motion ? mb : mb - kEntry;
+                        cur = ng == 2 ? kIdle : (ng == 1 ? 0 : kPop);
                     }
-                } else {
-                    const float4* tp = sv.tris + (size_t)tb * 3;
-                    while (cand != 0) {
-                        const int i = __ffs(cand) - 1;
-                        cand &= cand - 1;
-                        if (tri_test_q<false>(r, q, tp[3 * i], tp[3 * i + 1], tp[3 * i + 2], g.ray_bias, U, V, W))
-                            idx = lbase + i;
-                    }
-                }
-                if (idx >= 0) {
-                    best_geom = gcur; best_prim = idx; bu = U; bv = V; bw = W;
-                    if (SHADOW) done = true;   // qbvh/intersect.go:232-236 at both levels
                 }
             }
         }
+
+        const uint64_t leaves = __ballot(cur < kIdle);
+        const uint64_t nodes = __ballot(cur >= 0);
+        if (__popcll(leaves) * kLeafRatio < __popcll(nodes)) {
+            if (cur >= 0) {
+                if (COUNTERS) nodesT++;
+                Box4 b;
+                int ch[4], ax[3];
+                bool moving = false;
+                if constexpr (MOTION) moving = in_mesh ? g.nkeys > 1 : top_motion;
+                if (MOTION && moving) {
+                    const int nk = in_mesh ? g.nkeys : sv.top_keys;
+                    const int nb = in_mesh ? g.node_base : sv.top_mbase;
+                    int k0, k1;
+                    float t;
+                    motion_keys(r.time, nk, k0, k1, t);
+                    if (fast) {
+                        box_motion_near(r, kp, sv.mnodes, nb, cur, nk, k0, k1, t, ch, ax, b);
+                    } else {
+                        NodeData nd;
+                        box_motion(r, sv.mnodes, nb, cur, nk, k0, k1, t, nd, b);
+                        for (int c = 0; c < 4; c++) ch[c] = nd.ch[c];
+                        for (int k = 0; k < 3; k++) ax[k] = nd.ax[k];
+                    }
+                } else {
+                    const int idx = in_mesh ? g.node_base + cur : cur;
+                    if (fast) {
+                        // 32-bit byte offsets from the uniform base; a near plane's row is its axis's lower or
+                        // upper bound by the sign bit, the far plane's the other one (DevNode)
+                        const char* nbp = reinterpret_cast<const char*>(sv.nodes);
+                        const uint32_t o = (uint32_t)idx << 7;
+                        const uint32_t ox = (kp & 16) | o, oy = (kp & 32) | o, oz = (kp & 64) | o;
+                        auto row = [&](uint32_t ofs, int rr) { return *reinterpret_cast<const float4*>(nbp + ofs + 16 * rr); };
+                        const float4 nx = row(ox, kRowLoX), fx = row(ox ^ 16, kRowLoX);
+                        const float4 ny = row(oy, kRowLoY), fy = row(oy ^ 32, kRowLoY);
+                        const float4 nz = row(oz, kRowLoZ), fz = row(oz ^ 64, kRowLoZ);
+                        const int4 c = *reinterpret_cast<const int4*>(nbp + o + 16 * kRowChildren);
+                        const int4 a = *reinterpret_cast<const int4*>(nbp + o + 16 * kRowAxes);
+                        ch[0] = c.x; ch[1] = c.y; ch[2] = c.z; ch[3] = c.w;
+                        ax[0] = a.x; ax[1] = a.y; ax[2] = a.z;
+                        box4_near(r, nx, ny, nz, fx, fy, fz, b);
+                    } else {
+                        NodeData nd;
+                        fetch_static(sv.nodes, idx, nd);
+                        box4(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
+                        for (int c = 0; c < 4; c++) ch[c] = nd.ch[c];
+                        for (int k = 0; k < 3; k++) ax[k] = nd.ax[k];
+                    }
+                }
+                // Push order of qbvh/intersect.go:137-216 (same as motionintersect.go:53-97): the children
+                // are pushed as two pairs.  m0, m1, m2 are all ones when the ray's direction is negative on
+                // the node's axis: the first pair goes first when m0, child 0 before child 1 when m1, child 2
+                // before child 3 when m2.  A hit child's slot is the sum of the hits pushed before it, so the
+                // entries are exactly those the reference leaves below its stack top.
+                const int m0 = __builtin_amdgcn_sbfe(kp, ax[0], 1);
+                const int m1 = __builtin_amdgcn_sbfe(kp, ax[1], 1);
+                const int m2 = __builtin_amdgcn_sbfe(kp, ax[2], 1);
+                const int c0 = b.h[0] ? kEntry : 0, c1 = b.h[1] ? kEntry : 0;
+                const int c2 = b.h[2] ? kEntry : 0, c3 = b.h[3] ? kEntry : 0;
+                const int s01 = c0 + c1, s23 = c2 + c3;
+                const int pa = sp + (s23 & ~m0), pb = sp + (s01 & m0);
+                const int p0 = pa + (c1 & ~m1), p1 = pa + (c0 & m1);
+                const int p2 = pb + (c3 & ~m2), p3 = pb + (c2 & m2);
+                cur = kPop;
+                if (sp < (LDS - 3) * kEntry) {   // every slot of this step lies in LDS
+                    if (b.h[0]) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + p0) = make_uint2(__float_as_uint(b.t[0]), (uint32_t)ch[0]);
+                    if (b.h[1]) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + p1) = make_uint2(__float_as_uint(b.t[1]), (uint32_t)ch[1]);
+                    if (b.h[2]) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + p2) = make_uint2(__float_as_uint(b.t[2]), (uint32_t)ch[2]);
+                    if (b.h[3]) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + p3) = make_uint2(__float_as_uint(b.t[3]), (uint32_t)ch[3]);
+                    sp += s01 + s23;
+                } else if (sp >= (VGPU_MAX_STACK - 3) * kEntry) {   // conservative: the reference writes up to 4 slots here
+                    best_prim = -2;
+                    cur = kIdle;
+                } else {
+                    if (b.h[0]) push(p0, b.t[0], ch[0]);
+                    if (b.h[1]) push(p1, b.t[1], ch[1]);
+                    if (b.h[2]) push(p2, b.t[2], ch[2]);
+                    if (b.h[3]) push(p3, b.t[3], ch[3]);
+                    sp += s01 + s23;
+                }
+                if (COUNTERS && cur == kPop) maxDepth = max(maxDepth, (int)((uint32_t)sp / kEntry));
+            }
+            continue;
+        }
+        if (leaves == 0) continue;   // every lane popped its last entry
+
+        // ---- the leaves held, all of them
+        const bool mine = cur < kIdle;
+        const int cnt = mine ? leaf_count(cur) : 0;
+        const int lbase = leaf_base(cur);
+        const int pin = wave_scan_add(cnt);
+        const int pex = pin - cnt;
+        const int total = __builtin_amdgcn_readlane(pin, 63);
+        const TriRay own = tri_ray_packed(r, kp);
+        const bool mv = MOTION && g.nkeys > 1;
+        // what item w adds to reach its triangle: an index (static) or, scaled by the worker, a float4 offset
+        const int tb = mv ? g.tri_base + lbase * 3 * g.nkeys : g.tri_base + lbase - pex;
+        bool any = false;
+        for (int k0 = 0; k0 < total; k0 += 64) {
+            const int s0 = max(pex - k0, 0), e0 = min(pin - k0, 64);   // this lane's items of the chunk
+            const bool has = e0 > s0;
+            lds_put(&owner[tid], 0);
+            if (has) lds_put(&owner[(tid & ~63) + s0], lane);
+            const int o = wave_scan_max(lds_get(&owner[tid])) << 2;
+            const int w = k0 + lane;
+            TriRay q;
+            q.S0 = lane_f(o, own.S0); q.S1 = lane_f(o, own.S1); q.S2 = lane_f(o, own.S2);
+            q.Pkx = lane_f(o, own.Pkx); q.Pky = lane_f(o, own.Pky); q.Pkz = lane_f(o, own.Pkz);
+            q.axes(lane_i(o, kp));
+            const float obias = lane_f(o, g.ray_bias);
+            const int otb = lane_i(o, tb);
+            int onk = 1, oex = 0;
+            float otime = 0.0f;
+            if constexpr (MOTION) {
+                onk = lane_i(o, g.nkeys);
+                oex = lane_i(o, pex);
+                otime = lane_f(o, r.time);
+            }
+            bool pass = false;
+            TriPre pr;
+            if (w < total) {
+                if (MOTION && onk > 1) {
+                    int a0, a1;
+                    float t;
+                    motion_keys(otime, onk, a0, a1, t);
+                    float4 v0, v1, v2;
+                    motion_tri(sv.mtris + otb + (size_t)(w - oex) * 3 * onk, a0, a1, t, v0, v1, v2);
+                    pass = tri_pre<true>(q, v0, v1, v2, obias, pr);
+                } else {
+                    float4 v0, v1, v2;
+                    load_tri(sv.tris + (otb + w), v0, v1, v2);
+                    pass = tri_pre<false>(q, v0, v1, v2, obias, pr);
+                }
+            }
+            const uint64_t cm = __ballot(pass);
+            if (cm == 0) continue;
+            // the owners' passes over their candidates, in leaf order (trace.go:108-122)
+            uint32_t cand = has ? (uint32_t)(cm >> s0) & ((1u << (e0 - s0)) - 1u) : 0;
+            while (__ballot(cand != 0) != 0) {
+                const int src = s0 + __builtin_ctz(cand | 0x10000u);
+                const int sa = src << 2;
+                TriPre ow;
+                ow.T = lane_f(sa, pr.T); ow.det = lane_f(sa, pr.det);
+                ow.fU = lane_f(sa, pr.fU); ow.fV = lane_f(sa, pr.fV); ow.fW = lane_f(sa, pr.fW);
+                if (cand != 0) {
+                    cand &= cand - 1;
+                    if (tri_accept(r, ow, bu, bv, bw)) {
+                        best_geom = gcur;
+                        best_prim = lbase + k0 + src - pex;
+                        any = true;
+                    }
+                }
+            }
+        }
+        if (mine) cur = SHADOW && any ? kIdle : kPop;   // qbvh/intersect.go:232-236 at both levels
     }
 }
-
-#undef VGPU_IN_MESH
 
 #define VGPU_TRACE_PARAMS                                                                                      \
     SceneView sv, const float4 *__restrict__ rays, uint64_t n, int4 *__restrict__ hits,                       \
@@ -688,10 +818,9 @@ __global__ __launch_bounds__(BLOCK) void k_trace_wide(VGPU_TRACE_PARAMS) {
     trace_wide<BLOCK, LDS, SHADOW, MOTION, COUNTERS, EXT>(VGPU_TRACE_ARGS);
 }
 
-// Motion scenes with a short LDS stack (8 or 12 entries): the box and triangle interpolation leave
-// the plain kernel at 103-107 VGPRs, four waves per SIMD.  Held to 96 (a few dwords of spill), five
-// waves fit, and with a grid of five waves per SIMD (waves_per_cu 20) the 2000-moving-sphere camera
-// and shadow rays run 8-10% faster than the best four-wave shape.
+// Motion scenes with a short LDS stack (8 or 12 entries): the box and triangle interpolation leave the
+// plain kernel above 100 VGPRs, four waves per SIMD.  Held to 96 (a few dwords of spill), five waves fit;
+// 1M camera rays among 2000 moving spheres take 650 us at 64 / 8 / 20 against 738 us with a grid of four.
 template <int BLOCK, int LDS, bool SHADOW, bool COUNTERS, bool EXT>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_wide_m5(VGPU_TRACE_PARAMS) {
     static_assert(LDS <= 12, "the five-wave motion kernel is built for short LDS stacks");
@@ -759,7 +888,7 @@ __device__ bool trace_mesh(const SceneView& sv, const DevGeom& g, RayS& r, const
                 box_motion(r, sv.mnodes, g.node_base, node, g.nkeys, k0, k1, mt, nd, b);
             } else {
                 fetch_static(sv.nodes, g.node_base + node, nd);
-                box4<false>(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
+                box4(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
             }
             const int n0 = (kp >> nd.ax[0]) & 1, n1 = (kp >> nd.ax[1]) & 1, n2 = (kp >> nd.ax[2]) & 1;
             const int gA = n0 ? 0 : 2, gB = 2 - gA;
@@ -781,8 +910,9 @@ __device__ bool trace_mesh(const SceneView& sv, const DevGeom& g, RayS& r, const
                     motion_tri(sv.mtris + g.tri_base + (size_t)(lb + i) * 3 * g.nkeys, k0, k1, mt, v0, v1, v2);
                     ok = tri_test_q<true>(r, q, v0, v1, v2, g.ray_bias, U, V, W);
                 } else {
-                    const float4* tp = sv.tris + ((size_t)g.tri_base + lb + i) * 3;
-                    ok = tri_test_q<false>(r, q, tp[0], tp[1], tp[2], g.ray_bias, U, V, W);
+                    float4 v0, v1, v2;
+                    load_tri(sv.tris + (g.tri_base + lb + i), v0, v1, v2);
+                    ok = tri_test_q<false>(r, q, v0, v1, v2, g.ray_bias, U, V, W);
                 }
                 if (ok) { h.prim = lb + i; h.U = U; h.V = V; h.W = W; leaf_hit = true; }
             }
@@ -888,7 +1018,7 @@ __global__ __launch_bounds__(64) void k_trace_xform(SceneView sv, const float4* 
                     box_motion(r, sv.mnodes, sv.top_mbase, node, sv.top_keys, k0, k1, mt, nd, b);
                 } else {
                     fetch_static(sv.nodes, node, nd);
-                    box4<false>(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
+                    box4(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
                 }
                 const int n0 = (kp >> nd.ax[0]) & 1, n1 = (kp >> nd.ax[1]) & 1, n2 = (kp >> nd.ax[2]) & 1;
                 const int gA = n0 ? 0 : 2, gB = 2 - gA;

@@ -13,28 +13,38 @@ namespace vgpu {
 // fastest on incoherent bounce rays (64: refill only when the whole wavefront is idle).
 constexpr int kRefillDefault = 48;
 
-// Device node, 128 bytes = one cache line.  Same content as qbvh.Node
-// (qbvh/qbvh.go:31-36) re-laid for aligned 16-byte loads: the six box rows
-// (min x/y/z, max x/y/z; lane c = child c) are the reference's Boxes[24]
-// verbatim, followed by the children and the three split axes.
+// Direction-sign bit of axis 0 in the traversal's packed ray word, and the bias of the split axes that
+// nodes hold.
+constexpr int kSignBit = 4;
+
+// Device node, 128 bytes = one cache line: qbvh.Node (qbvh/qbvh.go:31-36) re-laid as eight 16-byte rows
+// (lane c = child c).  The two bounds of axis k lie in rows whose byte offsets differ in one bit, 16, 32
+// and 64 for x, y and z, so a ray's near and far planes are single loads at offsets made from its
+// direction signs.  The bounds are in order (lo <= hi): the upload swaps the lanes that are not, the
+// reference's empty box (+inf, -inf) above all, whose slab values are the same either way round.
+constexpr int kRowLoX = 0, kRowHiX = 1, kRowLoY = 4, kRowHiY = 6, kRowLoZ = 3, kRowHiZ = 7, kRowChildren = 2, kRowAxes = 5;
 struct alignas(16) DevNode {
-    float lox[4], loy[4], loz[4];
-    float hix[4], hiy[4], hiz[4];
-    int32_t children[4];   // reference encoding, node indices relative to the geom's node base
-    int32_t axes[4];       // axis0, axis1, axis2, 0
+    float rows[8][4];
+    // rows[kRowChildren]: int32, the reference's encoding, node indices relative to the geom's node base
+    // rows[kRowAxes]: int32 kSignBit + axis0, axis1, axis2; then bit 4 k + c set where the upload swapped
+    // axis k of child c
 };
 static_assert(sizeof(DevNode) == 128, "DevNode is one 128-byte line");
 
-// Motion node (qbvh.MotionNode + its per-key MotionNodeBoxes): a 32-byte
-// topology record followed by nkeys box blocks of 96 bytes (6 float4 rows as
-// above).  Stride in float4 units: 2 + 6*nkeys.
-struct alignas(16) DevMTopo {
-    int32_t children[4];
-    int32_t axes[4];
+// Motion node (qbvh.MotionNode + its per-key MotionNodeBoxes): a 32-byte topology record (children,
+// then axes as kSignBit + axis) followed by nkeys box blocks of 96 bytes: lo x, hi x, lo y, hi y, lo z,
+// hi z as float4 rows.  Stride in float4 units: 2 + 6*nkeys, so a row pair starts on 32 bytes.
+
+// A static triangle: three vertices without padding, 36 bytes.  Leaf tests read runs of consecutive
+// triangles, so the lines fetched shrink with the record (48 bytes as three float4 before: the 5.2M-triangle
+// field falls from 250 to 190 MB and, nodes included, under the 256 MB of the last-level cache).
+struct DevTri {
+    float v[3][3];
 };
+static_assert(sizeof(DevTri) == 36, "DevTri is nine floats");
 
 // Geom table entry.  Static geom: node_base indexes DevNode, tri_base indexes
-// triangles (3 float4 each: v0, v1, v2 with w unused).  Motion geom:
+// triangles (DevTri).  Motion geom:
 // node_base/tri_base are float4 offsets into the motion arrays; a motion
 // triangle is nkeys consecutive groups of 3 float4.
 struct alignas(16) DevGeom {
@@ -83,7 +93,7 @@ __device__ inline void xform_at(const DevXform& x, const float* xkeys, float tim
 
 struct SceneView {
     const DevNode* nodes;     // static nodes: top level at [0, ntop) when the top is static
-    const float4* tris;       // static triangles
+    const DevTri* tris;       // static triangles
     const float4* mnodes;     // motion nodes (topology + boxes)
     const float4* mtris;      // motion triangles
     const DevGeom* geoms;     // post-sort geom slots
@@ -91,7 +101,8 @@ struct SceneView {
     int32_t top_motion;       // 1: the top level is a motion QBVH at mnodes[top_mbase]
     int32_t top_keys;         // motion keys of the top level
     int32_t top_mbase;
-    int32_t nan_free_boxes;   // 1: no static node box holds a NaN bound
+    int32_t near_far;         // 1: box4_near's conditions hold for the nodes: no NaN bound, lo <= hi (motion
+                              // boxes: finite too), and both node arrays lie within 32-bit byte offsets
     int32_t any_xform;        // 1: some geom applies a transform (the per-lane kernel traces every ray)
     const DevXform* xforms;   // per geom slot (any_xform only)
     const float* xkeys;       // transform records
@@ -106,9 +117,10 @@ struct TraceLaunch {
 };
 
 // Launch shapes of launch_trace_ext (the shading passes' closest-hit traversal) for static and
-// motion scenes (the motion shape runs the four-wave kernel; the five-wave one measured 3% slower
-// in the motion-blur render); callers size the spill area for the larger grid.
-constexpr TraceLaunch kExtLaunch{128, 12, 24};
+// motion scenes; callers size the spill area for the larger grid.  The static kernel holds 88 VGPRs, five
+// waves per SIMD: a grid of 20 waves per CU fills them and leaves no workgroup waiting (2.1M bounce rays,
+// block 64: 725 us at 20 waves per CU, 786 at 16; block 128: 749 at 20, 780 at 24).
+constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 
 // Scratch of the ray sort (raysort.hip), sized for `capacity` rays.

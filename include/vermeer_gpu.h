@@ -251,7 +251,7 @@ int vgpu_scene_set_hidden(vgpu_scene* scene, int32_t geom, int32_t hidden);
  * interpolated at the ray's time; one key recomposed from its decomposition),
  * with bounds the box of bmin, bmax (BMin[0], BMax[0]; the reference ignores
  * later keys).  Hits report the instance's slot.  Scenes holding instances,
- * procs or mesh transforms are traced by a per-lane kernel without per-ray
+ * procs or mesh transforms are traced in a launch shape of their own, without per-ray
  * counters.  *geom_out: insertion index. */
 int vgpu_scene_add_instance(vgpu_scene* scene, int32_t geom, const float* matrices, uint32_t nkeys, const float* bmin,
                             const float* bmax, int32_t* geom_out);

@@ -105,3 +105,41 @@ def test_a_nan_bound_takes_the_exact_box_test():
     a, _, _ = g.trace(rays)
     b, _, _ = s.trace(rays)
     assert np.array_equal(_bits(a), _bits(b)) and (a["prim"] >= 0).any()
+
+
+@pytest.mark.parametrize("n", [1, 65, 4097])
+@pytest.mark.parametrize("count", [1, 7, 31])
+def test_transform_scenes_at_odd_sizes(count, n):
+    """Instances (still and moving), a proc and a moving
+    mesh; the allocation-free entry point gives the same hits."""
+    import torch
+    from vermeer_amd import render
+    desc = scenes.instance_scene(seed=count, count=count)
+    c = desc["camera"]
+    M, ttf = oracle.camera_lookat(c["from"], c["to"], c["up"], c["fov"], c["focal"])
+    R = render.Renderer(desc, 16, 16, render.lookat_camera(c["from"], c["to"], c["up"], c["fov"], c["focal"], 16, 16))
+    o = oracle.OracleRenderer(desc, 16, 16, M, ttf, c["focal"])
+    g = np.random.default_rng(n)
+    rays = np.zeros(n, va.RAY_DTYPE)
+    rays["P"] = g.uniform((-0.9, 0.1, -0.9), (0.9, 1.9, 0.9), (n, 3))
+    d = g.normal(size=(n, 3))
+    rays["D"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays["D"][::9, 2] = 0.0
+    rays["tmax"] = np.where(g.random(n) < 0.2, 0.7, np.inf)
+    rays["time"] = g.uniform(0, 1, n)
+    dr = torch.from_numpy(rays.view(np.uint8).copy()).cuda()
+    dh = torch.empty(n, 4, dtype=torch.int32, device="cuda")
+    dg = torch.empty(n, dtype=torch.int32, device="cuda")
+    lib = va._lib.load()
+    for shadow in (False, True):
+        hits, geoms, _ = R.scene.trace(rays, shadow=shadow)
+        ref, _ = o.scene.trace(rays, shadow=shadow)
+        for k in ("prim", "t", "u", "v"):
+            assert hits[k].tobytes() == ref[k].tobytes(), k
+        assert np.array_equal(geoms, ref["geom"])
+        va._lib.check(lib.vgpu_trace_noalloc(R.scene._h, va._lib.VGPU_TRACE_SHADOW if shadow else 0, dr.data_ptr(), n,
+                                             dh.data_ptr(), dg.data_ptr(), None, None, None))
+        torch.cuda.synchronize()
+        assert np.array_equal(dh.cpu().numpy().view(np.uint32), _bits(hits))
+        assert np.array_equal(dg.cpu().numpy(), geoms)
+    R.close()

@@ -359,7 +359,8 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
                   int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev) {
     if (d_counters && s->view.any_xform)
         return fail(VGPU_ERR_ARG, "per-ray counters are not kept for scenes with instances, procs or mesh transforms");
-    vgpu::TraceLaunch L{cfg.block, cfg.lds_stack, cfg.waves_per_cu, cfg.refill > 0 ? cfg.refill : vgpu::kRefillDefault};
+    const vgpu::TraceLaunch L = vgpu::scene_launch(
+        s->view, {cfg.block, cfg.lds_stack, cfg.waves_per_cu, cfg.refill > 0 ? cfg.refill : vgpu::kRefillDefault});
     const uint64_t threads = vgpu::trace_grid_threads(L, n, s->num_cus);
     int rc = ensure_spill(s, threads);
     if (rc) return rc;
@@ -1101,8 +1102,8 @@ int vgpu_trace_noalloc(vgpu_scene* s, uint32_t flags, const vgpu_ray* d_rays, ui
     DeviceGuard dg(s->device);
     // The scene's launch shape with fewer resident waves where its spill columns would not fit the
     // scratch array; never sorted (the sort's buffers grow with n).
-    vgpu::TraceLaunch L{s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu,
-                        s->cfg.refill > 0 ? s->cfg.refill : vgpu::kRefillDefault};
+    vgpu::TraceLaunch L = vgpu::scene_launch(s->view, {s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu,
+                                                       s->cfg.refill > 0 ? s->cfg.refill : vgpu::kRefillDefault});
     const uint64_t cap = vgpu::noalloc_max_threads(L.lds_depth);
     while (L.waves_per_cu > 1 && vgpu::trace_grid_threads(L, n, s->num_cus) > cap) L.waves_per_cu--;
     if (vgpu::trace_grid_threads(L, n, s->num_cus) > cap)

@@ -122,26 +122,6 @@ __device__ __forceinline__ void box4_near(const RayS& r, const float4& nx, const
     }
 }
 
-// The spill area is addressed from its (wavefront-uniform) bases plus one 32-bit per-lane offset,
-// so the lane keeps a single register for it.
-template <int BLOCK, int LDS>
-struct Stack {
-    float* sT;
-    int32_t* sN;
-    float* gT;          // spill bases (uniform)
-    int32_t* gN;
-    uint64_t gstride;
-    uint32_t gofs;      // this thread's column
-    __device__ __forceinline__ void store(int i, float T, int32_t node) {
-        if (i < LDS) { sT[i * BLOCK] = T; sN[i * BLOCK] = node; }
-        else { const uint64_t o = (uint64_t)(i - LDS) * gstride + gofs; gT[o] = T; gN[o] = node; }
-    }
-    __device__ __forceinline__ void load(int i, float& T, int32_t& node) const {
-        if (i < LDS) { T = sT[i * BLOCK]; node = sN[i * BLOCK]; }
-        else { const uint64_t o = (uint64_t)(i - LDS) * gstride + gofs; T = gT[o]; node = gN[o]; }
-    }
-};
-
 __device__ __forceinline__ int leaf_base(int32_t l) { return (int)((l & 0x7ffffff) >> 4); }
 __device__ __forceinline__ int leaf_count(int32_t l) { return (int)((l & 0xf) + 1); }
 
@@ -238,17 +218,6 @@ __device__ __forceinline__ bool tri_accept(RayS& r, const TriPre& p, float& U, f
     r.tclosest = p.T * rcp;
     return true;
 }
-
-// The whole test with the ray quantities given.
-template <bool MOTION_BOUND>
-__device__ __forceinline__ bool tri_test_q(RayS& r, const TriRay& q, const float4& v0, const float4& v1, const float4& v2,
-                                           float bias, float& U, float& V, float& W) {
-    TriPre p;
-    return tri_pre<MOTION_BOUND>(q, v0, v1, v2, bias, p) && tri_accept(r, p, U, V, W);
-}
-
-
-
 
 __device__ __forceinline__ void load_tri(const DevTri* __restrict__ p, float4& v0, float4& v1, float4& v2) {
     v0 = make_float4(p->v[0][0], p->v[0][1], p->v[0][2], 0.0f);
@@ -428,6 +397,97 @@ __device__ __forceinline__ int next_geom(const SceneView& sv, const float4* __re
     return 0;
 }
 
+// The ray in object space: P and D moved by Minv (D not renormalised).
+__device__ __forceinline__ void ray_to_object(const float* Minv, float* P, float* D) {
+    float p[3], d[3];
+    xf_point(Minv, P, p);
+    xf_vec(Minv, D, d);
+    for (int k = 0; k < 3; k++) { P[k] = p[k]; D[k] = d[k]; }
+}
+
+// Whether the near/far box tests hold for the ray (box4_near).
+template <bool MOTION>
+__device__ __forceinline__ bool ray_plain(const RayS& r) {
+    bool ok = !MOTION || absf(r.time) < 1e20f;   // time * keys stays finite
+    for (int k = 0; k < 3; k++) ok = ok && absf(r.P[k]) < INFINITY && absf(r.Dinv[k]) < INFINITY && r.Dinv[k] != 0.0f;
+    return ok;
+}
+
+// Where a lane stands among the geoms of a top-level leaf: child `child` of geom gcur (instances and
+// procs), whose mesh or sphere is `slot`; hit: gcur reported a hit.
+struct GeomWalk {
+    int slot, child;
+    bool hit;
+};
+
+// next_geom for scenes with transforms: the reference's recursion Scene.TraceElems -> Geom.Trace written
+// out.  first: the leaf has just been popped, gcur is its first geom; otherwise mesh w.slot has been
+// traced.  A geom with a transform moves the ray into its object space (P and D by the inverse transform
+// at the ray's time, then Setup) and restores it, Tclosest excepted (instance.go:78-104, proc.go:93-131,
+// polymesh/trace.go:20-74); a proc stops at the first geom reporting a hit unless the ray is a shadow ray
+// (proc.go:112-120), which leaves the scene after the geom that was hit.  Returns as next_geom.
+template <bool SHADOW>
+__device__ __forceinline__ int next_geom_xf(const SceneView& sv, const float4* __restrict__ rays, uint64_t ri, RayS& r,
+                                            int& kp, bool& ok, bool first, int& gcur, int gend, GeomWalk& w, DevGeom& g,
+                                            int& best_geom, int& best_prim, int& best_leaf, float& bu, float& bv,
+                                            float& bw) {
+    const float4 ra = rays[2 * ri], rb = rays[2 * ri + 1];
+    bool entered = !first;   // geom gcur has begun
+    while (true) {
+        if (entered) {
+            const DevXform x = sv.xforms[gcur];
+            if (x.kind >= kXfInstance && w.child + 1 < x.nchild && !(w.hit && (x.kind == kXfInstance || !SHADOW))) {
+                w.child++;
+            } else {
+                if (SHADOW && w.hit) return 2;
+                gcur++;
+                entered = false;
+            }
+        }
+        const bool end = !entered && gcur >= gend;
+        DevXform x{};
+        if (!end) {
+            x = sv.xforms[gcur];
+            if (!entered) {
+                entered = true;
+                w.child = 0;
+                w.hit = false;
+            }
+            if (x.kind >= kXfInstance) {
+                if (w.child >= x.nchild) continue;   // a proc without geoms
+                w.slot = sv.xchildren[x.child_base + w.child];
+            } else {
+                w.slot = gcur;
+            }
+            g = sv.geoms[w.slot];
+        }
+        float P[3] = {ra.x, ra.y, ra.z}, D[3] = {rb.x, rb.y, rb.z};
+        if (!end) {
+            // the instance's or proc's transform, then the mesh's own
+#pragma unroll 1
+            for (int level = x.kind >= kXfInstance ? 0 : 1; level < 2; level++) {
+                const DevXform xl = level == 0 ? x : sv.xforms[w.slot];
+                if (xl.kind == kXfNone) continue;
+                float M[16], Minv[16];
+                xform_at(xl, sv.xkeys, rb.w, M, Minv);
+                ray_to_object(Minv, P, D);
+            }
+        }
+        for (int k = 0; k < 3; k++) r.P[k] = P[k];
+        ray_setup(r, D);
+        kp = pack_perm(r);
+        ok = ray_plain<true>(r);
+        if (end) return 0;
+        if (g.nkeys != 0) return 1;
+        float t;
+        if (sphere_geom_hit(P, make_float4(D[0], D[1], D[2], 0.0f), sv.spheres[g.tri_base], r.tclosest, t)) {
+            r.tclosest = t;
+            w.hit = true;
+            best_geom = gcur; best_prim = 0; best_leaf = w.slot; bu = 0.0f; bv = 0.0f; bw = 0.0f;
+        }
+    }
+}
+
 // ---- cross-lane helpers of the wavefront-wide leaf tests
 
 // Sums / maxima over lanes 0..lane on the DPP row shifts and broadcasts: six VALU operations with no
@@ -463,6 +523,11 @@ __device__ __forceinline__ float lane_f(int addr, float x) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
 }
 __device__ __forceinline__ int lane_i(int addr, int x) { return __builtin_amdgcn_ds_bpermute(addr, x); }
+
+// In scenes with transforms, lanes at the end or the start of a geom wait until kTurnWait times as many
+// wait as hold a node or a leaf: the transform of a moving instance is a thousand instructions.  262,144
+// rays in a room of 60 instances: 712 us when half as many sufficed, 674 at 1, 656 at 2, 646 at 6.
+constexpr int kTurnWait = 4;
 
 // What a lane does next, beside node indices (>= 0) and mesh leaves (< kIdle).
 constexpr int kPop = -1;    // take the next stack entry (also the encoding of an empty child)
@@ -503,7 +568,10 @@ constexpr int kLeafRatio = 3;
 // (qbvh/motionintersect.go:47-49) and triangles of moving meshes (trace.go:547-554) are
 // interpolated at the ray's time.
 // EXT: hits are 32-byte records {prim, geom, t, U, V, W, 0, 0} for the shading kernels.
-template <int BLOCK, int LDS, bool SHADOW, bool MOTION, bool COUNTERS, bool EXT>
+// XFORM: the scene holds instances, procs or transformed meshes (MOTION is set too); a lane's ray is the
+// one in the space of the geom it traverses, and EXT records hold the slot of the mesh or sphere hit in
+// place of the first 0.
+template <int BLOCK, int LDS, bool SHADOW, bool MOTION, bool COUNTERS, bool EXT, bool XFORM = false>
 __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restrict__ rays, uint64_t n,
                                            int4* __restrict__ hits, int32_t* __restrict__ geoms_out,
                                            int4* __restrict__ counters, float* __restrict__ spT,
@@ -548,6 +616,9 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     // at base.  A motion top level starts it at the popped leaf's own slot, a static one above it
     // (qbvh/motionintersect.go:99-103 against intersect.go:219-226).
     const bool top_motion = MOTION && sv.top_motion;
+    const bool reuse_slot = XFORM || top_motion;
+    GeomWalk walk = {0, 0, false};
+    int best_leaf = 0;
     bool in_mesh = false;
     int base = bottom, gcur = 0, gend = 0;
     DevGeom g = {0, 0, 1, 0.0f};
@@ -563,11 +634,12 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                     if (best_prim == -2) {   // the stack overflowed
                         atomicOr(err, 1);
                         best_geom = -1; best_prim = -1;
+                        if (XFORM) best_leaf = -1;
                     }
                     const uint64_t oi = perm ? (uint64_t)perm[(uint32_t)ri] : (uint64_t)(uint32_t)ri;
                     if (EXT) {
                         hits[2 * oi] = make_int4(best_prim, best_geom, __float_as_int(r.tclosest), __float_as_int(bu));
-                        hits[2 * oi + 1] = make_int4(__float_as_int(bv), __float_as_int(bw), 0, 0);
+                        hits[2 * oi + 1] = make_int4(__float_as_int(bv), __float_as_int(bw), best_leaf, 0);
                     } else {
                         hits[oi] = make_int4(best_prim, __float_as_int(r.tclosest), __float_as_int(bu), __float_as_int(bv));
                         if (geoms_out) geoms_out[oi] = best_geom;
@@ -587,11 +659,10 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                         r.time = rb4.w;
                         ray_setup(r, D);
                         kp = pack_perm(r);
-                        for (int k = 0; k < 3; k++)
-                            ok = ok && absf(r.P[k]) < INFINITY && absf(r.Dinv[k]) < INFINITY && r.Dinv[k] != 0.0f;
-                        if (MOTION) ok = ok && absf(r.time) < 1e20f;   // time * keys stays finite
+                        ok = ray_plain<MOTION>(r);
                         nodesT = 0; leafsT = 0; trisT = 0; maxDepth = 0;
                         best_geom = -1; best_prim = -1;
+                        if (XFORM) best_leaf = -1;
                         bu = 0.0f; bv = 0.0f; bw = 0.0f;
                         in_mesh = false;
                         base = bottom;
@@ -623,33 +694,46 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
         // Ends of levels, and the scene level's leaves: lanes that leave a mesh for the scene level pop there
         // in the next turn.
         const bool turn = cur == kPop || (cur < kIdle && !in_mesh);
-        if (__ballot(turn) != 0) {
+        const uint64_t turns = __ballot(turn);
+        if (XFORM ? turns != 0 && __popcll(turns) >= kTurnWait * __popcll(__ballot(!turn && cur != kIdle)) : turns != 0) {
             if (turn) {
                 if (cur == kPop && !in_mesh) {
                     cur = kIdle;
                 } else {
+                    const bool first = cur != kPop;   // else PolyMesh.Trace returned: on to the leaf's next geom (scene.go:65-75)
                     int mb = base;
-                    if (cur == kPop) {
-                        gcur++;   // PolyMesh.Trace returned; Scene.TraceElems moves to the leaf's next geom (scene.go:65-75)
-                    } else {      // Scene.TraceElems: the geoms of a top-level leaf (scene.go:61-78)
-                        mb = top_motion ? sp : sp + kEntry;
+                    if (first) {   // Scene.TraceElems: the geoms of a top-level leaf (scene.go:61-78)
+                        mb = reuse_slot ? sp : sp + kEntry;
                         gcur = leaf_base(cur); gend = gcur + leaf_count(cur);
+                    } else if (!XFORM) {
+                        gcur++;
                     }
                     if (mb >= VGPU_MAX_STACK * kEntry) {
                         best_prim = -2;
                         cur = kIdle;
                     } else {
-                        const int ng = next_geom<SHADOW>(sv, rays, (uint32_t)ri, r, gcur, gend, g, best_geom, best_prim, bu, bv, bw);
+                        int ng;
+                        if constexpr (XFORM)
+                            ng = next_geom_xf<SHADOW>(sv, rays, (uint32_t)ri, r, kp, ok, first, gcur, gend, walk, g, best_geom,
+                                                      best_prim, best_leaf, bu, bv, bw);
+                        else
+                            ng = next_geom<SHADOW>(sv, rays, (uint32_t)ri, r, gcur, gend, g, best_geom, best_prim, bu, bv, bw);
                         in_mesh = ng == 1;
                         base = in_mesh ? mb : bottom;
-                        sp = in_mesh || top_motion ? mb : mb - kEntry;
+                        sp = in_mesh || reuse_slot ? mb : mb - kEntry;
                         cur = ng == 2 ? kIdle : (ng == 1 ? 0 : kPop);
                     }
                 }
             }
+            if (XFORM) {
+                if (cur == kIdle) ok = true;
+                fast = sv.near_far && __all(ok ? 1 : 0) != 0;
+                if (turns != 0) continue;
+            }
         }
 
-        const uint64_t leaves = __ballot(cur < kIdle);
+        const bool leaf = XFORM ? cur < kIdle && in_mesh : cur < kIdle;
+        const uint64_t leaves = __ballot(leaf);
         const uint64_t nodes = __ballot(cur >= 0);
         if (__popcll(leaves) * kLeafRatio < __popcll(nodes)) {
             if (cur >= 0) {
@@ -735,7 +819,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
         if (leaves == 0) continue;   // every lane popped its last entry
 
         // ---- the leaves held, all of them
-        const bool mine = cur < kIdle;
+        const bool mine = leaf;
         const int cnt = mine ? leaf_count(cur) : 0;
         const int lbase = leaf_base(cur);
         const int pin = wave_scan_add(cnt);
@@ -797,12 +881,18 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                     if (tri_accept(r, ow, bu, bv, bw)) {
                         best_geom = gcur;
                         best_prim = lbase + k0 + src - pex;
+                        if (XFORM) best_leaf = walk.slot;
                         any = true;
                     }
                 }
             }
         }
-        if (mine) cur = SHADOW && any ? kIdle : kPop;   // qbvh/intersect.go:232-236 at both levels
+        // a shadow ray's hit ends both levels (qbvh/intersect.go:232-236); under a transform, the mesh
+        if (mine) cur = SHADOW && any && !XFORM ? kIdle : kPop;
+        if (XFORM && any) {
+            walk.hit = true;
+            if (SHADOW) sp = base;
+        }
     }
 }
 
@@ -827,243 +917,28 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
     trace_wide<BLOCK, LDS, SHADOW, true, COUNTERS, EXT>(VGPU_TRACE_ARGS);
 }
 
+// Scenes holding GeomInstances, Procs or meshes with their own Transform.  Four waves per SIMD: the
+// transforms take registers, and their lanes wait for one another (kTurnWait).
+// 262,144 rays in rooms of 60 instances: 988 us, against 1,898 us for one ray per lane with the recursion
+// inside it (the leaf triangles of a lane tested by that lane alone).
+template <int BLOCK, int LDS, bool SHADOW, bool EXT>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_trace_xform(VGPU_TRACE_PARAMS) {
+    trace_wide<BLOCK, LDS, SHADOW, true, false, EXT, true>(VGPU_TRACE_ARGS);
+}
+
 #undef VGPU_TRACE_PARAMS
 #undef VGPU_TRACE_ARGS
 
-
-// ---------------------------------------------------------------- scenes with transforms
-//
-// Scenes holding GeomInstances, Procs or meshes with their own Transform run this kernel: one ray
-// per lane, the reference's recursion written out (Scene.Trace -> Geom.Trace -> qbvh.Trace ->
-// TraceElems), each level on the same stack above the level that called it.  A geom with a
-// transform moves the ray into its object space (P and D by the inverse transform at the ray's time,
-// D not renormalised, then Setup), traces what it holds and restores the ray, Tclosest excepted
-// (instance.go:78-104, proc.go:93-131, polymesh/trace.go:20-74).
-
-// The ray in object space: P and D moved by Minv, then Ray.Setup.
-__device__ __forceinline__ void ray_to_object(const RayS& r, const float* D, const float* Minv, RayS& o, float* Do) {
-    xf_point(Minv, r.P, o.P);
-    xf_vec(Minv, D, Do);
-    ray_setup(o, Do);
-    o.time = r.time;
-    o.tclosest = r.tclosest;
-}
-
-struct XHit {
-    int prim;
-    float U, V, W;
-};
-
-// qbvh.Trace / TraceMotion over one mesh (or the analytic sphere test) with the ray in the mesh's
-// space, its stack starting at entry `base`; true when it improved the hit.  -1 in *over: the stack
-// overflowed.
-template <bool SHADOW>
-__device__ bool trace_mesh(const SceneView& sv, const DevGeom& g, RayS& r, const float* D, Stack<64, 8>& st, int base,
-                           XHit& h, int* over) {
-    if (g.nkeys == 0) {   // analytic sphere (builtin/geom/sphere/trace.go:13-52)
-        float t;
-        const float4 d = make_float4(D[0], D[1], D[2], 0.0f);
-        if (!sphere_geom_hit(r.P, d, sv.spheres[g.tri_base], r.tclosest, t)) return false;
-        r.tclosest = t;
-        h.prim = 0; h.U = 0.0f; h.V = 0.0f; h.W = 0.0f;
-        return true;
-    }
-    const int kp = pack_perm(r);
-    const TriRay q = tri_ray_packed(r, kp);
-    int k0 = 0, k1 = 0;
-    float mt = 0.0f;
-    if (g.nkeys > 1) motion_keys(r.time, g.nkeys, k0, k1, mt);
-    bool hit = false;
-    st.store(base, r.tclosest, 0);
-    int sp = base + 1;
-    while (sp > base) {
-        sp--;
-        float T; int32_t node;
-        st.load(sp, T, node);
-        if (r.tclosest < T || node == -1) continue;
-        if (node >= 0) {
-            NodeData nd;
-            Box4 b;
-            if (g.nkeys > 1) {
-                box_motion(r, sv.mnodes, g.node_base, node, g.nkeys, k0, k1, mt, nd, b);
-            } else {
-                fetch_static(sv.nodes, g.node_base + node, nd);
-                box4(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
-            }
-            const int n0 = (kp >> nd.ax[0]) & 1, n1 = (kp >> nd.ax[1]) & 1, n2 = (kp >> nd.ax[2]) & 1;
-            const int gA = n0 ? 0 : 2, gB = 2 - gA;
-            const int rk[4] = {gA + (n1 ^ 1), gA + n1, gB + (n2 ^ 1), gB + n2};
-            if (sp + 4 > VGPU_MAX_STACK) { *over = 1; return hit; }
-            int m = 0;
-            for (int c = 0; c < 4; c++) if (b.h[c]) m |= 1 << rk[c];
-            for (int c = 0; c < 4; c++)
-                if (b.h[c]) st.store(sp + __popc(m & ((1 << rk[c]) - 1)), b.t[c], nd.ch[c]);
-            sp += __popc(m);
-        } else {
-            const int lb = leaf_base(node), lc = leaf_count(node);
-            bool leaf_hit = false;
-            for (int i = 0; i < lc; i++) {
-                float U, V, W;
-                bool ok;
-                if (g.nkeys > 1) {
-                    float4 v0, v1, v2;
-                    motion_tri(sv.mtris + g.tri_base + (size_t)(lb + i) * 3 * g.nkeys, k0, k1, mt, v0, v1, v2);
-                    ok = tri_test_q<true>(r, q, v0, v1, v2, g.ray_bias, U, V, W);
-                } else {
-                    float4 v0, v1, v2;
-                    load_tri(sv.tris + (g.tri_base + lb + i), v0, v1, v2);
-                    ok = tri_test_q<false>(r, q, v0, v1, v2, g.ray_bias, U, V, W);
-                }
-                if (ok) { h.prim = lb + i; h.U = U; h.V = V; h.W = W; leaf_hit = true; }
-            }
-            if (leaf_hit) {
-                hit = true;
-                if (SHADOW) return true;   // qbvh/intersect.go:232-236
-            }
-        }
-    }
-    return hit;
-}
-
-// Geom.Trace of a mesh or sphere slot, through its own Transform when it has one.
-template <bool SHADOW>
-__device__ bool trace_leaf_geom(const SceneView& sv, int slot, RayS& r, const float* D, Stack<64, 8>& st, int base,
-                                XHit& h, int* over) {
-    const DevGeom g = sv.geoms[slot];
-    const DevXform x = sv.xforms[slot];
-    if (x.kind != kXfMesh) return trace_mesh<SHADOW>(sv, g, r, D, st, base, h, over);
-    float M[16], Minv[16];
-    xform_at(x, sv.xkeys, r.time, M, Minv);
-    RayS o;
-    float Do[3];
-    ray_to_object(r, D, Minv, o, Do);
-    const bool hit = trace_mesh<SHADOW>(sv, g, o, Do, st, base, h, over);
-    r.tclosest = o.tclosest;
-    return hit;
-}
-
-// Geom.Trace of a top-level slot: a mesh or sphere, or an instance or proc over its geoms.  *leaf:
-// the slot whose element was hit.  A proc stops at the first geom reporting a hit unless the ray is
-// a shadow ray (proc.go:112-120).
-template <bool SHADOW>
-__device__ bool trace_geom(const SceneView& sv, int slot, RayS& r, const float* D, Stack<64, 8>& st, int base, XHit& h,
-                           int& leaf, int* over) {
-    const DevXform x = sv.xforms[slot];
-    if (x.kind != kXfInstance && x.kind != kXfProc) {
-        const bool hit = trace_leaf_geom<SHADOW>(sv, slot, r, D, st, base, h, over);
-        if (hit) leaf = slot;
-        return hit;
-    }
-    float M[16], Minv[16];
-    xform_at(x, sv.xkeys, r.time, M, Minv);
-    RayS o;
-    float Do[3];
-    ray_to_object(r, D, Minv, o, Do);
-    bool hit = false;
-    for (int c = 0; c < x.nchild && !*over; c++) {
-        const int child = sv.xchildren[x.child_base + c];
-        if (trace_leaf_geom<SHADOW>(sv, child, o, Do, st, base, h, over)) {
-            hit = true;
-            leaf = child;
-            if (x.kind == kXfInstance || !SHADOW) break;
-        }
-    }
-    r.tclosest = o.tclosest;
-    return hit;
-}
-
-// The whole traversal for one ray per lane.  EXT: 32-byte records {prim, geom, t, U, V, W, leaf slot, 0}.
 template <bool SHADOW, bool EXT>
-__global__ __launch_bounds__(64) void k_trace_xform(SceneView sv, const float4* __restrict__ rays, uint64_t n,
-                                                    int4* __restrict__ hits, int32_t* __restrict__ geoms_out,
-                                                    float* __restrict__ spT, int32_t* __restrict__ spN,
-                                                    int32_t* __restrict__ err, const uint32_t* __restrict__ n_dev,
-                                                    const uint32_t* __restrict__ perm) {
-    __shared__ float sT[8 * 64];
-    __shared__ int32_t sN[8 * 64];
-    const int tid = threadIdx.x;
-    const uint64_t gtid = (uint64_t)blockIdx.x * 64 + tid;
-    const uint64_t nthr = (uint64_t)gridDim.x * 64;
-    Stack<64, 8> st;
-    st.sT = sT + tid; st.sN = sN + tid;
-    st.gT = spT; st.gN = spN; st.gstride = nthr; st.gofs = (uint32_t)gtid;
-    if (n_dev) n = min(n, (uint64_t)*n_dev);
-    for (uint64_t ri = gtid; ri < n; ri += nthr) {
-        const float4 ra = rays[2 * ri], rb = rays[2 * ri + 1];
-        RayS r;
-        r.P[0] = ra.x; r.P[1] = ra.y; r.P[2] = ra.z;
-        r.tclosest = ra.w;
-        r.time = rb.w;
-        const float D[3] = {rb.x, rb.y, rb.z};
-        ray_setup(r, D);
-        const int kp = pack_perm(r);
-        XHit h{-1, 0.0f, 0.0f, 0.0f};
-        int best_geom = -1, best_leaf = -1, over = 0;
-        const bool top_motion = sv.top_motion != 0;
-        int k0 = 0, k1 = 0;
-        float mt = 0.0f;
-        if (top_motion) motion_keys(r.time, sv.top_keys, k0, k1, mt);
-        st.store(0, r.tclosest, 0);
-        int sp = 1;
-        bool done = false;
-        while (sp > 0 && !done && !over) {
-            sp--;
-            float T; int32_t node;
-            st.load(sp, T, node);
-            if (r.tclosest < T || node == -1) continue;
-            if (node >= 0) {
-                NodeData nd;
-                Box4 b;
-                if (top_motion) {
-                    box_motion(r, sv.mnodes, sv.top_mbase, node, sv.top_keys, k0, k1, mt, nd, b);
-                } else {
-                    fetch_static(sv.nodes, node, nd);
-                    box4(r, nd.lx, nd.ly, nd.lz, nd.hx, nd.hy, nd.hz, b);
-                }
-                const int n0 = (kp >> nd.ax[0]) & 1, n1 = (kp >> nd.ax[1]) & 1, n2 = (kp >> nd.ax[2]) & 1;
-                const int gA = n0 ? 0 : 2, gB = 2 - gA;
-                const int rk[4] = {gA + (n1 ^ 1), gA + n1, gB + (n2 ^ 1), gB + n2};
-                if (sp + 4 > VGPU_MAX_STACK) { over = 1; break; }
-                int m = 0;
-                for (int c = 0; c < 4; c++) if (b.h[c]) m |= 1 << rk[c];
-                for (int c = 0; c < 4; c++)
-                    if (b.h[c]) st.store(sp + __popc(m & ((1 << rk[c]) - 1)), b.t[c], nd.ch[c]);
-                sp += __popc(m);
-            } else {
-                // Scene.TraceElems over the leaf's geoms (scene.go:61-78)
-                const int lb = leaf_base(node), lc = leaf_count(node);
-                for (int gi = lb; gi < lb + lc && !over; gi++) {
-                    int leaf = -1;
-                    if (trace_geom<SHADOW>(sv, gi, r, D, st, sp, h, leaf, &over)) {
-                        best_geom = gi;
-                        best_leaf = leaf;
-                        if (SHADOW) { done = true; break; }
-                    }
-                }
-            }
-        }
-        if (over) {
-            atomicOr(err, 1);
-            best_geom = -1; best_leaf = -1; h.prim = -1;
-        }
-        if (best_geom < 0) h.prim = -1;
-        const uint64_t oi = perm ? (uint64_t)perm[ri] : ri;
-        if (EXT) {
-            hits[2 * oi] = make_int4(h.prim, best_geom, __float_as_int(r.tclosest), __float_as_int(h.U));
-            hits[2 * oi + 1] = make_int4(__float_as_int(h.V), __float_as_int(h.W), best_leaf, 0);
-        } else {
-            hits[oi] = make_int4(h.prim, __float_as_int(r.tclosest), __float_as_int(h.U), __float_as_int(h.V));
-            if (geoms_out) geoms_out[oi] = best_geom;
-        }
-    }
-}
-
-template <bool SHADOW, bool EXT>
-hipError_t launch_xform(const SceneView& sv, const void* rays, uint64_t n, void* hits, int32_t* geoms, float* spT,
-                        int32_t* spN, uint64_t threads, int32_t* err, const uint32_t* n_dev, const uint32_t* perm,
-                        hipStream_t stream) {
-    hipLaunchKernelGGL((k_trace_xform<SHADOW, EXT>), dim3((unsigned)(threads / 64)), dim3(64), 0, stream, sv,
-                       (const float4*)rays, n, (int4*)hits, geoms, spT, spN, err, n_dev, perm);
+hipError_t launch_xform(const SceneView& sv, const TraceLaunch& cfg, const void* rays, uint64_t n, void* hits,
+                        int32_t* geoms, float* spT, int32_t* spN, uint64_t spill_threads, int32_t* err, int num_cus,
+                        const uint32_t* n_dev, const uint32_t* perm, hipStream_t stream) {
+    constexpr int kB = kXformLaunch.block, kL = kXformLaunch.lds_depth;
+    const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
+    if (cfg.block != kB || cfg.lds_depth != kL || threads > spill_threads) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_trace_xform<kB, kL, SHADOW, EXT>), dim3((unsigned)(threads / kB)), dim3(kB), 0, stream, sv,
+                       (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err, n_dev, perm,
+                       cfg.refill_min);
     return hipGetLastError();
 }
 
@@ -1117,12 +992,13 @@ hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, 
     // the block size is the kernel's launch bound: each shape is a template constant
     constexpr int kB = kExtLaunch.block, kL = kExtLaunch.lds_depth;
     constexpr int kBM = kExtLaunchMotion.block, kLM = kExtLaunchMotion.lds_depth;
+    if (sv.any_xform)
+        return launch_xform<false, true>(sv, kXformLaunch, rays, n, hits32, nullptr, spT, spN, spill_threads, err, num_cus,
+                                         n_dev, nullptr, stream);
     const TraceLaunch cfg = motion ? kExtLaunchMotion : kExtLaunch;
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
     if (threads > spill_threads) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(threads / cfg.block);
-    if (sv.any_xform)
-        return launch_xform<false, true>(sv, rays, n, hits32, nullptr, spT, spN, threads, err, n_dev, nullptr, stream);
     if (motion)
         hipLaunchKernelGGL((k_trace_wide<kBM, kLM, false, true, false, true>), dim3(grid), dim3(kBM), 0, stream, sv,
                            (const float4*)rays, n, (int4*)hits32, (int32_t*)nullptr, (int4*)nullptr, spT, spN, err, n_dev,
@@ -1148,14 +1024,16 @@ hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const Tra
                         int32_t* err, int num_cus, hipStream_t stream, const uint32_t* n_dev, const uint32_t* perm) {
     if (n == 0) return hipSuccess;
     if (n > 0xffffffffull) return hipErrorInvalidValue;
+    if (sv.any_xform) {   // no counters
+        if (counters) return hipErrorInvalidValue;
+        return shadow ? launch_xform<true, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
+                                                  n_dev, perm, stream)
+                      : launch_xform<false, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
+                                                   n_dev, perm, stream);
+    }
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
     if (threads > spill_threads) return hipErrorInvalidValue;
     const uint64_t grid = threads / cfg.block;
-    if (sv.any_xform) {   // the per-lane kernel (block 64; threads is a multiple of 64); no counters
-        if (counters) return hipErrorInvalidValue;
-        return shadow ? launch_xform<true, false>(sv, rays, n, hits, geoms, spT, spN, threads, err, n_dev, perm, stream)
-                      : launch_xform<false, false>(sv, rays, n, hits, geoms, spT, spN, threads, err, n_dev, perm, stream);
-    }
 #define VGPU_CASE(B, L)                                                                                         \
     if (cfg.block == B && cfg.lds_depth == L)                                                                   \
         return launch_mode<B, L>(sv, shadow, motion, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, \

@@ -103,7 +103,7 @@ struct SceneView {
     int32_t top_mbase;
     int32_t near_far;         // 1: box4_near's conditions hold for the nodes: no NaN bound, lo <= hi (motion
                               // boxes: finite too), and both node arrays lie within 32-bit byte offsets
-    int32_t any_xform;        // 1: some geom applies a transform (the per-lane kernel traces every ray)
+    int32_t any_xform;        // 1: some geom applies a transform (k_trace_xform traces every ray)
     const DevXform* xforms;   // per geom slot (any_xform only)
     const float* xkeys;       // transform records
     const int32_t* xchildren; // geom slots held by instances and procs
@@ -122,6 +122,18 @@ struct TraceLaunch {
 // block 64: 725 us at 20 waves per CU, 786 at 16; block 128: 749 at 20, 780 at 24).
 constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
+
+// Launch shape of the traversals of a scene with transforms (block and LDS depth are its kernel's): the
+// scene's refill threshold in that shape.
+constexpr TraceLaunch kXformLaunch{64, 12, 16};
+static_assert(kXformLaunch.waves_per_cu <= kExtLaunch.waves_per_cu && kXformLaunch.waves_per_cu <= kExtLaunchMotion.waves_per_cu,
+              "the shading passes' spill areas cover it");
+inline TraceLaunch scene_launch(const SceneView& sv, const TraceLaunch& cfg) {
+    if (!sv.any_xform) return cfg;
+    TraceLaunch l = kXformLaunch;
+    l.refill_min = cfg.refill_min;
+    return l;
+}
 
 // Scratch of the ray sort (raysort.hip), sized for `capacity` rays.
 struct RaySortBuffers {
@@ -143,7 +155,7 @@ hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_
 // hold (VGPU_MAX_STACK - lds_depth) entries per launched thread; the launch
 // uses at most spill_threads threads.  n_dev (nullable): a device-resident
 // ray count; the kernel traces min(n, *n_dev) rays (n sizes the grid).  perm (nullable):
-// ray i's results go to slot perm[i] (rays reordered by launch_ray_sort).
+// ray i's results go to slot perm[i] (rays reordered by launch_ray_sort).  cfg: a scene_launch shape.
 // Returns hipSuccess or the launch error.
 hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg,
                         const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,

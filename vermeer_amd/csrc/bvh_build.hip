@@ -18,16 +18,18 @@
 //   counted from n - 1); for p >= s a right element goes to p - 1 and the k-th left element counted
 //   from n - 1 goes to rl[k-1], the position of the k-th right element counted from 0.
 //
-// Box arithmetic follows MINSS / MAXSS (math/dim_amd64.s): x < y ? x : y.  The reference grows boxes
-// element by element; reductions here combine partial boxes in element order with the operand order
-// that keeps the same element on ties, so the sign of zero bounds matches as well.
+// Box arithmetic follows MINSS / MAXSS (math/dim_amd64.s): x < y ? x : y.  The boxes that reach the
+// nodes (leaf boxes, unions of child boxes) are grown in the reference's order, so the sign of zero
+// bounds matches as well.  The centroid bounds and bin boxes of a split decide only through subtractions,
+// products and comparisons, which give the same split whichever zero a bound is, so those folds run in
+// any order, as integer minima and maxima of order-preserving keys.
 //
 // Schedule.  Ranges above kSubtreeMax elements are split level by level with device-wide kernels
-// over 4096-element chunks (all nodes of a level in one batch of launches; the host reads the pivots
+// over chunks (all nodes of a level in one batch of launches; the host reads the pivots
 // back after each batch).  A range of at most kSubtreeMax elements becomes a subtree that one
-// wavefront builds completely, depth first with an explicit stack, into a scratch node area at its
-// element offset.  The host then numbers the nodes in the reference's depth-first pre-order and one
-// kernel moves every subtree into place.
+// workgroup builds completely in LDS, its wavefronts taking nodes from a queue (k_subtree), into a
+// scratch node area at its element offset.  The host then numbers the nodes in the reference's
+// depth-first pre-order and one kernel moves every subtree into place.
 
 #include <hip/hip_runtime.h>
 
@@ -46,9 +48,10 @@ namespace vgpu {
 namespace {
 
 constexpr int kSegThreads = 256;                 // threads of a chunk kernel
-constexpr int kSegPer = 16;                      // contiguous elements per thread
-constexpr int kChunk = kSegThreads * kSegPer;    // elements per chunk
-constexpr int kSubtreeMax = 2048;                // largest range one wavefront builds
+// Elements per chunk: small chunks fill the chip (300,001 elements: 293 workgroups instead of 73; the kernels
+// of a batch take 51 us instead of 85), large ones keep the per-task folds over chunks short.
+constexpr int kChunkSmall = 1024, kChunkLarge = 4096, kChunkLargeFrom = 1 << 20;
+constexpr int kSubtreeMax = 2048;                // largest range one workgroup builds in LDS
 constexpr int kStackMax = 192;                   // subtree depth limit
 
 // One element: a = (lo xyz, index bits), b = (hi xyz, 0), c = (centroid xyz, 0).
@@ -67,19 +70,9 @@ __device__ __forceinline__ Box box_empty() {
     const float inf = __builtin_inff();
     return Box{{inf, inf, inf}, {-inf, -inf, -inf}};
 }
-// BoundingBox.GrowBox (math/boundingbox.go:99-104): Min(acc, b), Max(acc, b); ties take b.  Two
-// partial folds L (earlier elements) and R (later) combine as grow_box(L, R).
+// BoundingBox.GrowBox (math/boundingbox.go:99-104): Min(acc, b), Max(acc, b); ties take b.
 __device__ __forceinline__ void grow_box(Box& acc, const Box& b) {
     for (int k = 0; k < 3; k++) { acc.lo[k] = mins(acc.lo[k], b.lo[k]); acc.hi[k] = maxs(acc.hi[k], b.hi[k]); }
-}
-// BoundingBox.Grow (math/boundingbox.go:107-116): Min(p, acc), Max(p, acc); ties keep acc.
-__device__ __forceinline__ void grow_point(Box& acc, const float4& p) {
-    const float q[3] = {p.x, p.y, p.z};
-    for (int k = 0; k < 3; k++) { acc.lo[k] = mins(q[k], acc.lo[k]); acc.hi[k] = maxs(q[k], acc.hi[k]); }
-}
-// Two partial point folds, L earlier and R later: the earlier one wins ties.
-__device__ __forceinline__ void join_points(Box& L, const Box& R) {
-    for (int k = 0; k < 3; k++) { L.lo[k] = mins(R.lo[k], L.lo[k]); L.hi[k] = maxs(R.hi[k], L.hi[k]); }
 }
 __device__ __forceinline__ float dim(const Box& b, int a) { return b.hi[a] - b.lo[a]; }
 __device__ __forceinline__ float area(const Box& b) {
@@ -101,114 +94,165 @@ struct Cut {
     __device__ __forceinline__ bool right(const float4& c) const { return !((int)(k1 * (cen(c, axis) - k0)) < best); }
 };
 
-// ---------------------------------------------------------------- wavefront and block reductions
+// ---------------------------------------------------------------- folds
 
-template <bool POINTS>
-__device__ __forceinline__ Box wave_fold(Box v) {
-    const int lane = threadIdx.x & 63;
-    for (int d = 1; d < 64; d <<= 1) {
-        Box o;
-        for (int k = 0; k < 3; k++) { o.lo[k] = __shfl_down(v.lo[k], d); o.hi[k] = __shfl_down(v.hi[k], d); }
-        if ((lane & (2 * d - 1)) == 0) {
-            if (POINTS) join_points(v, o);
-            else grow_box(v, o);
+// Order-preserving integer keys of floats (no NaN): unsigned comparison of keys is comparison of values,
+// with -0 below +0.
+__device__ __forceinline__ uint32_t key_of(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ float of_key(uint32_t k) {
+    return __uint_as_float(k ^ (((k >> 31) - 1u) | 0x80000000u));
+}
+constexpr uint32_t kKeyInf = 0xff800000u, kKeyNegInf = 0x007fffffu;   // key_of(+inf), key_of(-inf)
+
+// DPP shifts: lanes without a source read `old`.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t dpp(uint32_t old, uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
+    x = min(x, dpp<0x111>(~0u, x));
+    x = min(x, dpp<0x112>(~0u, x));
+    x = min(x, dpp<0x114>(~0u, x));
+    x = min(x, dpp<0x118>(~0u, x));
+    x = min(x, dpp<0x142, 0xa>(~0u, x));
+    x = min(x, dpp<0x143, 0xc>(~0u, x));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) { return ~wave_min(~x); }
+
+// Keys of centroid bounds, folded over elements.
+struct KeyBox {
+    uint32_t lo[3], hi[3];
+    __device__ __forceinline__ void reset() {
+        for (int k = 0; k < 3; k++) { lo[k] = kKeyInf; hi[k] = kKeyNegInf; }
+    }
+    __device__ __forceinline__ void grow(float x, float y, float z) {
+        const float q[3] = {x, y, z};
+        for (int k = 0; k < 3; k++) {
+            const uint32_t u = key_of(q[k]);
+            lo[k] = min(lo[k], u);
+            hi[k] = max(hi[k], u);
         }
     }
-    for (int k = 0; k < 3; k++) { v.lo[k] = __shfl(v.lo[k], 0); v.hi[k] = __shfl(v.hi[k], 0); }
-    return v;
-}
-
-__device__ __forceinline__ int wave_scan(int x) {   // inclusive
-    const int lane = threadIdx.x & 63;
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d);
-        if (lane >= d) x += y;
+    __device__ __forceinline__ void join(const KeyBox& o) {
+        for (int k = 0; k < 3; k++) { lo[k] = min(lo[k], o.lo[k]); hi[k] = max(hi[k], o.hi[k]); }
     }
-    return x;
-}
-__device__ __forceinline__ int wave_sum(int x) { return __shfl(wave_scan(x), 63); }
+    __device__ __forceinline__ void over_wave() {
+        for (int k = 0; k < 3; k++) { lo[k] = wave_min(lo[k]); hi[k] = wave_max(hi[k]); }
+    }
+    __device__ __forceinline__ Box box() const {
+        Box b;
+        for (int k = 0; k < 3; k++) { b.lo[k] = of_key(lo[k]); b.hi[k] = of_key(hi[k]); }
+        return b;
+    }
+};
+
+// Orders one wavefront's LDS accesses for the compiler (the hardware keeps them in order).
+__device__ __forceinline__ void wave_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 constexpr int kWaves = kSegThreads / 64;
 
-template <bool POINTS>
-__device__ Box block_fold(Box v, Box* sh) {
-    v = wave_fold<POINTS>(v);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    Box r = sh[0];
-    for (int w = 1; w < kWaves; w++) {
-        if (POINTS) join_points(r, sh[w]);
-        else grow_box(r, sh[w]);
-    }
-    __syncthreads();
-    return r;
+// The split's axis and binning from the centroid bounds (build.go:40-58); false on a flat axis.
+__device__ __forceinline__ bool cut_of(const Box& cb, Cut& cut) {
+    cut.axis = longest(cb);
+    cut.best = 0;
+    const float lo = cut.axis == 0 ? cb.lo[0] : (cut.axis == 1 ? cb.lo[1] : cb.lo[2]);
+    const float hi = cut.axis == 0 ? cb.hi[0] : (cut.axis == 1 ? cb.hi[1] : cb.hi[2]);
+    cut.k1 = 7.99952f / (hi - lo);
+    cut.k0 = lo;
+    return !(hi == lo);
 }
 
-// Exclusive scan over the block (thread order); *total: the sum.
-__device__ int block_scan_excl(int x, int* sh, int* total) {
-    const int inc = wave_scan(x);
-    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = inc;
-    __syncthreads();
-    int base = 0, tot = 0;
-    for (int w = 0; w < kWaves; w++) {
-        if (w < (int)(threadIdx.x >> 6)) base += sh[w];
-        tot += sh[w];
-    }
-    __syncthreads();
-    *total = tot;
-    return base + inc - x;
+// Eight bins as kBinWords words: six keys (lo xyz, hi xyz) per bin, then the eight counts.
+constexpr int kBinWords = 56;
+__device__ __forceinline__ uint32_t bin_identity(int w) { return w >= 48 ? 0u : (w % 6 < 3 ? kKeyInf : kKeyNegInf); }
+__device__ __forceinline__ uint32_t bin_join(int w, uint32_t x, uint32_t y) {
+    return w >= 48 ? x + y : (w % 6 < 3 ? min(x, y) : max(x, y));
 }
-
-// Per-thread bins (counts and boxes grown in element order), updated without dynamic indexing.
-struct Bins {
-    Box b[8];
-    int n[8];
+// A wavefront's bins in LDS: COPIES copies, lane l adding to copy l % COPIES, since atomics on one address are
+// served one after another (about 8 cycles a lane).  Eight for the chunks of the device-wide splits (293 chunks
+// of 1024 elements: 25 us with one copy, 18 with eight), one for the subtrees, whose ranges are too short to
+// pay for more (147 subtrees: 220 us with one, 245 with eight).  Eight boxes per lane in registers cost 130
+// instructions an element and 288 shuffles a fold.
+constexpr int kBinStride = kBinWords + 1;   // the odd stride spreads the copies over the banks
+template <int COPIES>
+struct WaveBins {
+    uint32_t w[COPIES * kBinStride];
+    __device__ __forceinline__ uint32_t* mine() { return w + ((int)threadIdx.x % COPIES) * kBinStride; }
 };
-__device__ __forceinline__ void bins_init(Bins& B) {
-#pragma unroll
-    for (int k = 0; k < 8; k++) { B.b[k] = box_empty(); B.n[k] = 0; }
+template <int COPIES>
+__device__ __forceinline__ void bins_reset(WaveBins<COPIES>& B) {
+    for (int i = threadIdx.x & 63; i < COPIES * kBinStride; i += 64) B.w[i] = bin_identity(i % kBinStride);
 }
-// Adds e to its bin; sets err bit 1 for a bin outside [0, 7] (the reference's index panics there).
-__device__ __forceinline__ void bins_add(Bins& B, const GElem& e, const Cut& cut, int* err) {
-    const float f = cut.k1 * (cen(e.c, cut.axis) - cut.k0);
+// Folds the copies into the first one.
+template <int COPIES>
+__device__ __forceinline__ void bins_fold(WaveBins<COPIES>& B) {
+    const int w = threadIdx.x & 63;
+    if (COPIES == 1 || w >= kBinWords) return;
+    uint32_t x = B.w[w];
+#pragma unroll
+    for (int k = 1; k < COPIES; k++) x = bin_join(w, x, B.w[k * kBinStride + w]);
+    B.w[w] = x;
+}
+// Adds a box whose centroid coordinate on the cut's axis is c to a lane's copy; sets err bit 1 for a bin
+// outside [0, 7] (the reference's index panics there).
+__device__ __forceinline__ void bins_add(uint32_t* bins, const Cut& cut, float c, const float* b, int* err) {
+    const float f = cut.k1 * (c - cut.k0);
     const int bin = (int)f;
     if (f != f || bin < 0 || bin > 7) { atomicOr(err, 1); return; }
-    const Box eb = elem_box(e);
+    uint32_t* w = bins + bin * 6;
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-        if (bin == k) { grow_box(B.b[k], eb); B.n[k]++; }
+    for (int k = 0; k < 3; k++) {
+        __hip_atomic_fetch_min(w + k, key_of(b[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_max(w + 3 + k, key_of(b[3 + k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __hip_atomic_fetch_add(bins + 48 + bin, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// calcMinCost's SAH choice (qbvh/build.go:60-107) over the folded bins: left boxes and counts grown
-// from bin 0, right ones from bin 7, the first strict minimum of area(L) * nL + area(R) * nR.
-__device__ void sah(const Bins& B, int* best_out, int* nl_out) {
-    Box rb[8];
-    int rn[8];
-    Box acc = box_empty();
-    int m = 0;
+// calcMinCost's SAH choice (qbvh/build.go:60-107) over the folded bins, by one wavefront, lane b holding
+// bin b: left boxes and counts grown from bin 0, right ones from bin 7 (DPP scans), the first strict
+// minimum of area(L) * nL + area(R) * nR.
+__device__ void sah_wave(const uint32_t* bins, int* best_out, int* nl_out) {
+    const int lane = threadIdx.x & 63;
+    const bool in = lane < 8;
+    Box L, R;
 #pragma unroll
-    for (int b = 7; b >= 0; b--) { grow_box(acc, B.b[b]); m += B.n[b]; rb[b] = acc; rn[b] = m; }
-    acc = box_empty();
-    m = 0;
-    int best = -1;
-    float bestCost = __builtin_inff();
+    for (int j = 0; j < 6; j++) {
+        const bool lo = j < 3;
+        const uint32_t id = lo ? kKeyInf : kKeyNegInf;
+        const uint32_t v = in ? bins[lane * 6 + j] : id;
+        auto fold = [&](uint32_t x, uint32_t y) { return lo ? min(x, y) : max(x, y); };
+        uint32_t p = v, q = v;
+        p = fold(p, dpp<0x111>(id, p)); p = fold(p, dpp<0x112>(id, p)); p = fold(p, dpp<0x114>(id, p));
+        q = fold(q, dpp<0x101>(id, q)); q = fold(q, dpp<0x102>(id, q)); q = fold(q, dpp<0x104>(id, q));
+        p = dpp<0x111>(id, p);   // the bins before this one
+        (lo ? L.lo : L.hi)[j % 3] = of_key(p);
+        (lo ? R.lo : R.hi)[j % 3] = of_key(q);
+    }
+    const uint32_t n = in ? bins[48 + lane] : 0u;
+    uint32_t m = n, rn = n;
+    m += dpp<0x111>(0, m); m += dpp<0x112>(0, m); m += dpp<0x114>(0, m);
+    rn += dpp<0x101>(0, rn); rn += dpp<0x102>(0, rn); rn += dpp<0x104>(0, rn);
+    m = dpp<0x111>(0, m);
+    const float cost = area(L) * (float)(int)m + area(R) * (float)(int)rn;
+    int best = -1, nl = 0;
+    float best_cost = __builtin_inff();
 #pragma unroll
     for (int b = 1; b < 8; b++) {
-        grow_box(acc, B.b[b - 1]);
-        m += B.n[b - 1];
-        const float cost = area(acc) * (float)m + area(rb[b]) * (float)rn[b];
-        if (cost < bestCost) { best = b; bestCost = cost; }
+        const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), b));
+        if (c < best_cost) { best = b; best_cost = c; nl = __builtin_amdgcn_readlane((int)m, b); }
     }
-    int nl = 0;
-#pragma unroll
-    for (int b = 0; b < 8; b++) if (b < best) nl += B.n[b];
     *best_out = best;
     *nl_out = nl;
 }
 
 // Destination of position p (rank r = right elements in [0, p], inclusive) under the closed form;
 // -1 for an index outside [0, n), which only inconsistent bins (an error already flagged) produce.
-__device__ __forceinline__ int dest_of(int p, bool right, int r, int n, int nl, int s, const int* rl, const int* lr) {
+template <class I>
+__device__ __forceinline__ int dest_of(int p, bool right, int r, int n, int nl, int s, const I* rl, const I* lr) {
     int d;
     if (p < s) {
         if (!right) return p;
@@ -224,91 +268,119 @@ __device__ __forceinline__ int dest_of(int p, bool right, int r, int n, int nl, 
     return (d >= 0 && d < n) ? d : -1;
 }
 // Records position i in rl / lr (r: right elements in [0, i], inclusive); false if out of range.
-__device__ __forceinline__ bool record_rank(int i, bool right, int r, int n, int nl, int* rl, int* lr) {
+template <class I>
+__device__ __forceinline__ bool record_rank(int i, bool right, int r, int n, int nl, I* rl, I* lr) {
     if (right) {
         if (r - 1 >= n) return false;
-        rl[r - 1] = i;
+        rl[r - 1] = (I)i;
         return true;
     }
     const int k = nl - (i - r) - 1;
     if (k < 0 || k >= n) return false;
-    lr[k] = n - 1 - i;
+    lr[k] = (I)(n - 1 - i);
     return true;
 }
 
-// ---------------------------------------------------------------- one split by one wavefront
+// ---------------------------------------------------------------- subtrees in LDS
 
 struct SplitOut {
     int axis, pivot;
 };
 
-__device__ __forceinline__ void wave_copy(const GElem* src, GElem* dst, int n) {
-    for (int i = threadIdx.x; i < n; i += 64) dst[i] = src[i];
-}
+constexpr int kSubWaves = 8;
+constexpr int kSubThreads = 64 * kSubWaves;
+constexpr uint32_t kTaskReady = 0x80000000u;
+constexpr int kNoParent = 0x7ff;   // of node 0 only, which no node has as a child
 
-// binarySplit (qbvh/build.go:151-178) of src[0, n) into dst[0, n) by one wavefront (blockDim 64).
-// rl / lr: n ints each (LDS).  Lane l takes the contiguous slice [l * per, (l + 1) * per).
-__device__ SplitOut split_wave(const GElem* src, GElem* dst, int n, int leafMax, int* rl, int* lr, int* err) {
-    if (n <= leafMax) {
-        wave_copy(src, dst, n);
-        __syncthreads();
-        return SplitOut{0, n};
+// A subtree's elements (boxes and centroids, in the order they came) and the split's index lists, and its
+// nodes in the order they were found: node id's range, its place in the tree and what its completion needs.
+struct SubLds {
+    float box[6][kSubtreeMax];
+    float cen[3][kSubtreeMax];
+    uint16_t idx[2][kSubtreeMax];                // positions in split order; a split moves a range between the two
+    uint16_t rl[kSubtreeMax], lr[kSubtreeMax];
+    uint32_t task[kSubtreeMax];                  // kTaskReady | n << 16 | start, 0 until it is published
+    uint32_t link[kSubtreeMax];                  // parent | child slot << 11 | depth << 13
+    int pend[kSubtreeMax];                       // child nodes not yet complete
+    uint16_t child[kSubtreeMax][4];              // node ids, 0xffff: none
+    uint16_t size[kSubtreeMax], before[kSubtreeMax];   // nodes of the subtree; nodes of the siblings before it
+    WaveBins<1> bins[kSubWaves];
+    int head, tail, done;                        // next ticket; nodes found; 1: complete, 2: given up
+};
+static_assert(sizeof(SubLds) <= 160 * 1024, "one workgroup per CU");
+
+// binarySplit (qbvh/build.go:151-178) of positions [start, start + n) of L.idx[from] into L.idx[1 - from] by one
+// wavefront.
+__device__ __forceinline__ SplitOut split_lds(SubLds& L, int from, int start, int n, int leafMax, int* err) {
+    const int lane = threadIdx.x & 63;
+    const uint16_t* src = &L.idx[from][start];
+    uint16_t* dst = &L.idx[1 - from][start];
+    uint16_t* rl = L.rl + start;
+    uint16_t* lr = L.lr + start;
+    WaveBins<1>& B = L.bins[threadIdx.x >> 6];
+    Cut cut{0, 0, 0.0f, 0.0f};
+    bool split = n > leafMax;
+    if (split) {
+        KeyBox kb;
+        kb.reset();
+        for (int i = lane; i < n; i += 64) {
+            const int e = src[i];
+            kb.grow(L.cen[0][e], L.cen[1][e], L.cen[2][e]);
+        }
+        kb.over_wave();
+        split = cut_of(kb.box(), cut);
     }
-    const int lane = threadIdx.x;
-    const int per = (n + 63) >> 6;
-    const int a = min(n, lane * per), b = min(n, a + per);
-    Box cb = box_empty();
-    for (int i = a; i < b; i++) grow_point(cb, src[i].c);
-    cb = wave_fold<true>(cb);
-    const int axis = longest(cb);
-    if (cb.hi[axis] == cb.lo[axis]) {
-        wave_copy(src, dst, n);
-        __syncthreads();
-        return SplitOut{axis, n / 2 + 1};
+    if (!split) {
+        for (int i = lane; i < n; i += 64) dst[i] = src[i];
+        wave_order();
+        return SplitOut{cut.axis, n > leafMax ? n / 2 + 1 : n};
     }
-    Cut cut;
-    cut.axis = axis;
-    cut.k1 = 7.99952f / (cb.hi[axis] - cb.lo[axis]);
-    cut.k0 = cb.lo[axis];
-    Bins B;
-    bins_init(B);
-    for (int i = a; i < b; i++) bins_add(B, src[i], cut, err);
+    bins_reset(B);
+    wave_order();
+    uint32_t* bins = B.mine();
+    const float* cen = L.cen[cut.axis];
+    for (int i = lane; i < n; i += 64) {
+        const int e = src[i];
+        float b[6];
 #pragma unroll
-    for (int k = 0; k < 8; k++) { B.b[k] = wave_fold<false>(B.b[k]); B.n[k] = wave_sum(B.n[k]); }
+        for (int k = 0; k < 6; k++) b[k] = L.box[k][e];
+        bins_add(bins, cut, cen[e], b, err);
+    }
+    wave_order();
+    bins_fold(B);
+    wave_order();
     int nl;
-    sah(B, &cut.best, &nl);
-    int cnt = 0;
-    for (int i = a; i < b; i++) cnt += cut.right(src[i].c) ? 1 : 0;
-    const int base = wave_scan(cnt) - cnt;
-    int r = base;
-    for (int i = a; i < b; i++) {
-        const bool right = cut.right(src[i].c);
-        r += right ? 1 : 0;
-        if (!record_rank(i, right, r, n, nl, rl, lr)) atomicOr(err, 1);
+    sah_wave(B.w, &cut.best, &nl);
+    auto right = [&](int e) { return !((int)(cut.k1 * (cen[e] - cut.k0)) < cut.best); };
+    // rank: right elements at or before the position
+    const uint64_t upto = ~0ull >> (63 - lane);
+    int run = 0;
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        const int i = i0 + lane;
+        const bool rt = i < n && right(src[i]);
+        const uint64_t m = __ballot(rt);
+        if (i < n && !record_rank(i, rt, run + __popcll(m & upto), n, nl, rl, lr)) atomicOr(err, 1);
+        run += __popcll(m);
     }
-    __syncthreads();
-    const int s = nl + ((nl < n && cut.right(src[nl].c)) ? 1 : 0);
-    r = base;
-    for (int i = a; i < b; i++) {
-        const GElem e = src[i];
-        const bool right = cut.right(e.c);
-        r += right ? 1 : 0;
-        const int d = dest_of(i, right, r, n, nl, s, rl, lr);
-        if (d >= 0) dst[d] = e;
-        else atomicOr(err, 1);
+    wave_order();
+    const int s = nl + ((nl < n && right(src[nl])) ? 1 : 0);
+    run = 0;
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        const int i = i0 + lane;
+        const int e = i < n ? src[i] : 0;
+        const bool rt = i < n && right(e);
+        const uint64_t m = __ballot(rt);
+        if (i < n) {
+            const int d = dest_of(i, rt, run + __popcll(m & upto), n, nl, s, rl, lr);
+            if (d >= 0) dst[d] = (uint16_t)e;
+            else atomicOr(err, 1);
+        }
+        run += __popcll(m);
     }
-    __syncthreads();
-    return SplitOut{axis, nl};
+    wave_order();
+    return SplitOut{cut.axis, nl};
 }
 
-__device__ __forceinline__ void set_child_box(vgpu_qbvh_node& nd, int c, const Box& b) {
-    for (int k = 0; k < 3; k++) { nd.boxes[c + k * 4] = b.lo[k]; nd.boxes[c + 12 + k * 4] = b.hi[k]; }
-}
-__device__ __forceinline__ Box child_box(const vgpu_qbvh_node& nd, int c) {
-    Box b;
-    for (int k = 0; k < 3; k++) { b.lo[k] = nd.boxes[c + k * 4]; b.hi[k] = nd.boxes[c + 12 + k * 4]; }
-    return b;
-}
 __device__ __forceinline__ int32_t leaf_code(uint32_t first, uint32_t count) {
     return (int32_t)((1u << 31) | ((first << 4) & 0xfffffff0u) | ((count - 1) & 0xfu));
 }
@@ -320,124 +392,221 @@ __device__ Box leaf_box(const GElem* E, int n) {
     return b;
 }
 
-// SetBounds + SetLeaf; an empty leaf is child -1 with the InfBox (qbvh/qbvh.go:67-79).
-__device__ void set_leaf(vgpu_qbvh_node& nd, int c, uint32_t first, uint32_t count, const Box& b) {
-    if (count == 0) {
-        const float inf = __builtin_inff();
-        nd.children[c] = -1;
-        set_child_box(nd, c, Box{{inf, inf, inf}, {inf, inf, inf}});
-        return;
+// Node `me` is complete (its leaves' and child nodes' boxes are in its record): its box unions the
+// non-empty child boxes in order (qbvh/build.go:277-284) and fills its slot in the parent; the wavefront
+// that completes a node's last child completes the node too, up to the root.
+__device__ void complete_node(SubLds& L, int me, vgpu_qbvh_node* nodes, float* root_box) {
+    const int lane = threadIdx.x & 63;
+    while (true) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        const vgpu_qbvh_node& nd = nodes[me];
+        const bool lo = lane < 3;
+        float v = lo ? __builtin_inff() : -__builtin_inff();
+        if (lane < 6)
+            for (int c = 0; c < 4; c++)
+                if (nd.children[c] != -1) {
+                    const float b = nd.boxes[c + 4 * lane];
+                    v = lo ? mins(v, b) : maxs(v, b);
+                }
+        if (lane == 0) {
+            int sum = 0;
+            for (int c = 0; c < 4; c++) {
+                const int id = L.child[me][c];
+                if (id == 0xffff) continue;
+                L.before[id] = (uint16_t)sum;
+                sum += L.size[id];
+            }
+            L.size[me] = (uint16_t)(sum + 1);
+        }
+        const uint32_t link = L.link[me];
+        const int parent = (int)(link & 0x7ffu), slot = (int)((link >> 11) & 3u);
+        if (me == 0) {
+            if (lane < 6) root_box[lane] = v;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            if (lane == 0) __hip_atomic_store(&L.done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            return;
+        }
+        if (lane < 6) nodes[parent].boxes[slot + 4 * lane] = v;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        int left = 0;
+        if (lane == 0) left = __hip_atomic_fetch_add(&L.pend[parent], -1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (__builtin_amdgcn_readfirstlane(left) != 1) return;
+        me = parent;
     }
-    set_child_box(nd, c, b);
-    nd.children[c] = leaf_code(first, count);
 }
 
-struct Frame {
-    int start, n, node, next;   // next: -1 before the splits, then the child to visit
-    int p1, p0, p02;            // child c covers [lo(c), lo(c + 1)) with lo = {0, p1, p0, p02, n}
-};
-__device__ __forceinline__ int frame_lo(const Frame& f, int c) {
-    return c == 0 ? 0 : (c == 1 ? f.p1 : (c == 2 ? f.p0 : (c == 3 ? f.p02 : f.n)));
-}
-
-// buildAccelRec (qbvh/build.go:180-287) of one subtree per workgroup of one wavefront.  Elements of
-// subtree s: E[roots[s].x, + roots[s].y), built in place with T as the second buffer; nodes in local
-// pre-order at nodes[roots[s].x ..] (the subtree has at most max(n, 1) nodes); counts[s]: the node
-// count; root_boxes[s]: the root's box.  err bit 2: node area exceeded (only a range whose recursion
-// never ends, as two coincident centroids with leafMax 1); bit 8: deeper than kStackMax levels.
-__global__ __launch_bounds__(64) void k_subtree(GElem* E_all, GElem* T_all, const int2* roots,
-                                                vgpu_qbvh_node* nodes_all, int* counts, float* root_boxes,
-                                                int leafMax, int* err) {
-    __shared__ int rl[kSubtreeMax], lr[kSubtreeMax];
-    __shared__ Frame st[kStackMax];
-    __shared__ int sh_sp, sh_nn;
-    __shared__ float sh_box[6];
+// buildAccelRec (qbvh/build.go:180-287) of one subtree per workgroup.  Elements of subtree s: E[roots[s].x,
+// + roots[s].y), permuted in place; its nodes in the order they were found at nodes[roots[s].x ..] (at most
+// max(n, 1)), their pre-order numbers at pre[roots[s].x ..]; counts[s]: the node count; root_boxes[s]: the
+// root's box.  err bit 2: node area exceeded (only a range whose recursion never ends, as two coincident
+// centroids with leafMax 1); bit 8: deeper than kStackMax levels.
+//
+// The elements stay in LDS for the whole build and splits move 16-bit positions.  Wavefronts take nodes from
+// a queue in the order they were found: each takes a ticket and waits until that node is published or the
+// root is complete (or the build is given up), which some wavefront always reaches, since a published node
+// waits for no other.  Finding order puts parents before children; the numbers follow from the subtree sizes.
+// One wavefront per subtree splitting in global memory, with eight bin boxes per lane folded through
+// shuffles, took 2270 us for the 147 subtrees of 300,001 triangles (a chain of 270 nodes at 8 us each);
+// this takes 220 us.
+__global__ __launch_bounds__(kSubThreads) void k_subtree(GElem* E_all, const int2* roots, vgpu_qbvh_node* nodes_all,
+                                                         int* pre_all, int* counts, float* root_boxes, int leafMax,
+                                                         int* err) {
+    __shared__ SubLds L;
     const int2 root = roots[blockIdx.x];
     GElem* E = E_all + root.x;
-    GElem* T = T_all + root.x;
     vgpu_qbvh_node* nodes = nodes_all + root.x;
     const int cap = max(root.y, 1);
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63;
+    for (int i = t; i < kSubtreeMax; i += kSubThreads) {
+        L.task[i] = 0;
+        // every index a valid one, whatever a broken split leaves
+        L.idx[0][i] = (uint16_t)min(i, cap - 1);
+        L.idx[1][i] = (uint16_t)min(i, cap - 1);
+        if (i < root.y) {
+            const GElem e = E[i];
+            const float b[6] = {e.a.x, e.a.y, e.a.z, e.b.x, e.b.y, e.b.z};
+            for (int k = 0; k < 6; k++) L.box[k][i] = b[k];
+            L.cen[0][i] = e.c.x; L.cen[1][i] = e.c.y; L.cen[2][i] = e.c.z;
+        }
+    }
     if (t == 0) {
-        st[0] = Frame{0, root.y, -1, -1, 0, 0, 0};
-        sh_sp = 1;
-        sh_nn = 0;
-        const float inf = __builtin_inff();
-        for (int k = 0; k < 3; k++) { sh_box[k] = inf; sh_box[3 + k] = -inf; }
+        L.head = 0;
+        L.tail = 1;
+        L.done = 0;
+        L.link[0] = kNoParent;
     }
     __syncthreads();
+    if (t == 0)
+        __hip_atomic_store(&L.task[0], kTaskReady | ((uint32_t)root.y << 16), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     while (true) {
-        const int top = sh_sp - 1;
-        if (top < 0) break;
-        const Frame f = st[top];
-        __syncthreads();
-        if (f.next < 0) {
-            // the node's three binary splits: E -> T over the range, then each half T -> E
-            const SplitOut s0 = split_wave(E + f.start, T + f.start, f.n, leafMax, rl, lr, err);
-            const SplitOut s1 = split_wave(T + f.start, E + f.start, s0.pivot, leafMax, rl, lr, err);
-            const SplitOut s2 = split_wave(T + f.start + s0.pivot, E + f.start + s0.pivot, f.n - s0.pivot, leafMax, rl,
-                                           lr, err);
-            if (t == 0) {
-                const int me = sh_nn;
-                if (me >= cap) {
-                    atomicOr(err, 2);
-                    sh_sp = 0;
-                } else {
-                    sh_nn = me + 1;
-                    vgpu_qbvh_node& nd = nodes[me];
-                    for (int k = 0; k < 24; k++) nd.boxes[k] = 0.0f;
-                    for (int c = 0; c < 4; c++) nd.children[c] = 0;
-                    nd.parent = 0;
-                    nd.axis0 = (uint32_t)s0.axis;
-                    nd.axis1 = (uint32_t)s1.axis;
-                    nd.axis2 = (uint32_t)s2.axis;
-                    st[top] = Frame{f.start, f.n, me, 0, s1.pivot, s0.pivot, s0.pivot + s2.pivot};
+        int me = 0;
+        if (lane == 0) me = __hip_atomic_fetch_add(&L.head, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        me = __builtin_amdgcn_readfirstlane(me);
+        uint32_t task = 0;
+        int done = 0;
+        while (true) {
+            done = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&L.done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+            if (done) break;
+            if (me < kSubtreeMax)
+                task = (uint32_t)__builtin_amdgcn_readfirstlane(
+                    (int)__hip_atomic_load(&L.task[me], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+            if (task) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (done) break;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        const int start = (int)(task & 0xffffu), n = (int)((task >> 16) & 0x7fffu);
+        // the node's three binary splits: idx[0] -> idx[1] over the range, then each half back
+        SplitOut s0{}, s1{}, s2{};
+#pragma unroll 1
+        for (int k = 0; k < 3; k++) {
+            const SplitOut o = split_lds(L, k == 0 ? 0 : 1, k == 2 ? start + s0.pivot : start,
+                                         k == 0 ? n : (k == 1 ? s0.pivot : n - s0.pivot), leafMax, err);
+            if (k == 0) s0 = o;
+            else if (k == 1) s1 = o;
+            else s2 = o;
+        }
+        const int p1 = s1.pivot, p0 = s0.pivot, p02 = s0.pivot + s2.pivot;
+        auto lo_of = [&](int c) { return c == 0 ? 0 : (c == 1 ? p1 : (c == 2 ? p0 : (c == 3 ? p02 : n))); };
+        int cn[4], id[4], found = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            cn[c] = lo_of(c + 1) - lo_of(c);
+            id[c] = 0xffff;
+            if (cn[c] > leafMax) found++;
+        }
+        const int depth = (int)(L.link[me] >> 13);
+        int first = 0;
+        if (found) {
+            if (lane == 0) first = __hip_atomic_fetch_add(&L.tail, found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            first = __builtin_amdgcn_readfirstlane(first);
+            const int bad = first + found > cap ? 2 : (depth + 1 >= kStackMax ? 8 : 0);
+            if (bad) {
+                if (lane == 0) {
+                    atomicOr(err, bad);
+                    __hip_atomic_store(&L.done, 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-            }
-        } else if (f.next < 4) {
-            if (t == 0) {
-                const int c = f.next;
-                const int lo = frame_lo(f, c), cn = frame_lo(f, c + 1) - lo;
-                st[top].next = c + 1;
-                if (cn <= leafMax) {
-                    set_leaf(nodes[f.node], c, (uint32_t)(root.x + f.start + lo), (uint32_t)cn,
-                             leaf_box(E + f.start + lo, cn));
-                } else if (top + 1 >= kStackMax) {
-                    atomicOr(err, 8);
-                    sh_sp = 0;
-                } else {
-                    st[top + 1] = Frame{f.start + lo, cn, -1, -1, 0, 0, 0};
-                    sh_sp = top + 2;
-                }
-            }
-        } else if (t == 0) {
-            // the node is complete: its box unions the stored non-empty child boxes
-            // (qbvh/build.go:277-284), and it fills its slot in the parent
-            const vgpu_qbvh_node& nd = nodes[f.node];
-            Box nb = box_empty();
-            for (int c = 0; c < 4; c++)
-                if (nd.children[c] != -1) grow_box(nb, child_box(nd, c));
-            sh_sp = top;
-            if (top > 0) {
-                const Frame& p = st[top - 1];
-                const int c = p.next - 1;
-                set_child_box(nodes[p.node], c, nb);
-                nodes[p.node].children[c] = f.node;
-            } else {
-                for (int k = 0; k < 3; k++) { sh_box[k] = nb.lo[k]; sh_box[3 + k] = nb.hi[k]; }
+                break;
             }
         }
-        __syncthreads();
+        {
+            int k = first;
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                if (cn[c] > leafMax) id[c] = k++;
+        }
+        // the node's record, a word per lane: boxes (lane 4 j + c: bound j of child c), axes, children
+        const float inf = __builtin_inff();
+        uint32_t w = 0;
+        if (lane < 24) {
+            const int c = lane & 3, j = lane >> 2;
+            const int lo = start + lo_of(c), m = c == 0 ? cn[0] : (c == 1 ? cn[1] : (c == 2 ? cn[2] : cn[3]));
+            if (m == 0) {
+                w = __float_as_uint(inf);   // an empty leaf's InfBox (qbvh/qbvh.go:67-79)
+            } else if (m <= leafMax) {      // calcBox of a leaf: GrowBox in element order
+                const bool low = j < 3;
+                float v = low ? inf : -inf;
+                for (int i = 0; i < m; i++) {
+                    const float b = L.box[j][L.idx[0][lo + i]];
+                    v = low ? mins(v, b) : maxs(v, b);
+                }
+                w = __float_as_uint(v);
+            }
+        } else if (lane < 27) {
+            w = (uint32_t)(lane == 24 ? s0.axis : (lane == 25 ? s1.axis : s2.axis));
+        } else if (lane < 31) {
+            const int c = lane - 27;
+            const int m = c == 0 ? cn[0] : (c == 1 ? cn[1] : (c == 2 ? cn[2] : cn[3]));
+            const int k = c == 0 ? id[0] : (c == 1 ? id[1] : (c == 2 ? id[2] : id[3]));
+            w = (uint32_t)(m == 0 ? -1 : (m <= leafMax ? leaf_code((uint32_t)(root.x + start + lo_of(c)), (uint32_t)m) : k));
+            L.child[me][c] = (uint16_t)k;
+        }
+        if (lane < 32) reinterpret_cast<uint32_t*>(nodes + me)[lane] = w;
+        if (lane == 0) L.pend[me] = found;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (found == 0) {
+            complete_node(L, me, nodes, root_boxes + blockIdx.x * 6);
+        } else if (lane < 4) {
+            const int m = lane == 0 ? cn[0] : (lane == 1 ? cn[1] : (lane == 2 ? cn[2] : cn[3]));
+            const int k = lane == 0 ? id[0] : (lane == 1 ? id[1] : (lane == 2 ? id[2] : id[3]));
+            if (m > leafMax) {
+                L.link[k] = (uint32_t)me | ((uint32_t)lane << 11) | ((uint32_t)(depth + 1) << 13);
+                __hip_atomic_store(&L.task[k], kTaskReady | ((uint32_t)m << 16) | (uint32_t)(start + lo_of(lane)),
+                                   __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        }
     }
-    if (t == 0) counts[blockIdx.x] = sh_nn;
-    if (t < 6) root_boxes[blockIdx.x * 6 + t] = sh_box[t];
+    __syncthreads();
+    if (L.done != 1) return;
+    const int count = L.tail;
+    for (int i = t; i < count; i += kSubThreads) {
+        int p = 0;
+        for (int x = i; x != 0; x = (int)(L.link[x] & 0x7ffu)) p += 1 + L.before[x];
+        pre_all[root.x + i] = p;
+    }
+    if (t == 0) counts[blockIdx.x] = count;
+    constexpr int kPer = kSubtreeMax / kSubThreads;
+    if (root.y == 0) return;
+    float4 ea[kPer], eb[kPer], ec[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const GElem* p = E + L.idx[0][min(t + k * kSubThreads, root.y - 1)];
+        ea[k] = p->a; eb[k] = p->b; ec[k] = p->c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int i = t + k * kSubThreads;
+        if (i < root.y) E[i] = GElem{ea[k], eb[k], ec[k]};
+    }
 }
 
 // ---------------------------------------------------------------- device-wide splits of large ranges
 
-// A split of src[start, start + n) into dst, over chunks [chunk0, chunk0 + nchunk) of the batch.
+// A split of src[start, start + n) into dst, over chunks [chunk0, chunk0 + nchunk) of the batch, `chunk`
+// elements each.
 struct SegTask {
-    int start, n, chunk0, nchunk;
+    int start, n, chunk0, nchunk, chunk;
 };
 // mode 0: partition; 1: n <= leafMax (no binning); 2: flat axis.  pivot: the split's result.
 struct SegParam {
@@ -445,8 +614,7 @@ struct SegParam {
     float k0, k1;
 };
 struct BinPart {
-    Box b[8];
-    int n[8];
+    uint32_t w[kBinWords];
 };
 
 struct ChunkRange {
@@ -456,107 +624,138 @@ __device__ __forceinline__ ChunkRange chunk_range(const SegTask* tasks, const in
     ChunkRange c;
     c.task = chunk_task[blockIdx.x];
     const SegTask tk = tasks[c.task];
-    c.first = ((int)blockIdx.x - tk.chunk0) * kChunk;
-    c.end = min(tk.n, c.first + kChunk);
+    c.first = ((int)blockIdx.x - tk.chunk0) * tk.chunk;
+    c.end = min(tk.n, c.first + tk.chunk);
     return c;
 }
-// The thread's contiguous slice of a chunk.
-__device__ __forceinline__ void thread_slice(const ChunkRange& c, int* a, int* b) {
-    *a = min(c.end, c.first + (int)threadIdx.x * kSegPer);
-    *b = min(c.end, *a + kSegPer);
+// Right elements of the block's chunks before this one, then of its wavefronts before this one: the rank
+// base of a wavefront's quarter of the chunk.  part: right elements per chunk.  sh: kWaves ints each.
+__device__ int rank_base(const SegTask& tk, const int* part, int mine, int* sh_before, int* sh_mine) {
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int chunk = (int)blockIdx.x - tk.chunk0;
+    int before = 0;
+    for (int i = threadIdx.x; i < chunk; i += kSegThreads) before += part[tk.chunk0 + i];
+    for (int d = 32; d >= 1; d >>= 1) before += __shfl_xor(before, d);
+    if (lane == 0) { sh_before[wv] = before; sh_mine[wv] = mine; }
+    __syncthreads();
+    int base = 0;
+    for (int k = 0; k < kWaves; k++) {
+        base += sh_before[k];
+        if (k < wv) base += sh_mine[k];
+    }
+    return base;
 }
-// The thread's contiguous share of m items (the per-task folds over chunk partials).
-__device__ __forceinline__ void block_share(int m, int* a, int* b) {
-    const int per = (m + kSegThreads - 1) / kSegThreads;
-    *a = min(m, (int)threadIdx.x * per);
-    *b = min(m, *a + per);
+// A wavefront's quarter of the chunk, read 64 consecutive elements at a time.
+__device__ __forceinline__ void wave_range(const ChunkRange& c, int chunk, int* a, int* b) {
+    *a = min(c.end, c.first + (int)(threadIdx.x >> 6) * (chunk / kWaves));
+    *b = min(c.end, *a + chunk / kWaves);
+}
+// Right elements in a wavefront's range.
+__device__ __forceinline__ int wave_count(const GElem* E, const Cut& cut, int a, int b) {
+    int cnt = 0;
+    for (int i0 = a; i0 < b; i0 += 64) {
+        const int i = i0 + (int)(threadIdx.x & 63);
+        cnt += __popcll(__ballot(i < b && cut.right(E[i].c)));
+    }
+    return cnt;
 }
 
 __global__ __launch_bounds__(kSegThreads) void k_seg_cb(const GElem* src, const SegTask* tasks, const int* chunk_task,
-                                                         int leafMax, Box* part) {
-    __shared__ Box sh[kWaves];
+                                                         int leafMax, KeyBox* part) {
+    __shared__ KeyBox sh[kWaves];
     const ChunkRange c = chunk_range(tasks, chunk_task);
     if (tasks[c.task].n <= leafMax) return;
     const GElem* E = src + tasks[c.task].start;
-    int a, b;
-    thread_slice(c, &a, &b);
-    Box v = box_empty();
-    for (int i = a; i < b; i++) grow_point(v, E[i].c);
-    v = block_fold<true>(v, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = v;
+    KeyBox v;
+    v.reset();
+    for (int i = c.first + (int)threadIdx.x; i < c.end; i += kSegThreads) v.grow(E[i].c.x, E[i].c.y, E[i].c.z);
+    v.over_wave();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < kWaves; k++) v.join(sh[k]);
+        part[blockIdx.x] = v;
+    }
 }
 
-__global__ __launch_bounds__(kSegThreads) void k_seg_axis(const SegTask* tasks, const Box* part, int leafMax,
-                                                           SegParam* params) {
-    __shared__ Box sh[kWaves];
-    const SegTask tk = tasks[blockIdx.x];
+// The task's cut from its chunks' centroid bounds, by every block of the task (the bounds of a chunk are
+// 24 bytes; a launch of its own cost 6 us), and the chunk's bins.  The task's first block keeps the cut.
+__global__ __launch_bounds__(kSegThreads) void k_seg_bins(const GElem* src, const SegTask* tasks, const int* chunk_task,
+                                                           const KeyBox* cb_part, int leafMax, SegParam* params,
+                                                           BinPart* part, int* err) {
+    __shared__ KeyBox sh[kWaves];
+    __shared__ WaveBins<8> bins[kWaves];
+    const ChunkRange c = chunk_range(tasks, chunk_task);
+    const SegTask tk = tasks[c.task];
+    const bool owner = (int)blockIdx.x == tk.chunk0 && threadIdx.x == 0;
     SegParam P{};
     if (tk.n <= leafMax) {
         P.mode = 1;
         P.pivot = tk.n;
-        if (threadIdx.x == 0) params[blockIdx.x] = P;
+        if (owner) params[c.task] = P;
         return;
     }
-    int a, b;
-    block_share(tk.nchunk, &a, &b);
-    Box v = box_empty();
-    for (int i = a; i < b; i++) join_points(v, part[tk.chunk0 + i]);
-    const Box cb = block_fold<true>(v, sh);
-    P.axis = longest(cb);
-    if (cb.hi[P.axis] == cb.lo[P.axis]) {
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    KeyBox v;
+    v.reset();
+    for (int i = threadIdx.x; i < tk.nchunk; i += kSegThreads) v.join(cb_part[tk.chunk0 + i]);
+    v.over_wave();
+    if (lane == 0) sh[wv] = v;
+    bins_reset(bins[wv]);
+    __syncthreads();
+    v = sh[0];
+    for (int k = 1; k < kWaves; k++) v.join(sh[k]);
+    Cut cut;
+    const bool flat = !cut_of(v.box(), cut);
+    P.axis = cut.axis;
+    if (flat) {
         P.mode = 2;
         P.pivot = tk.n / 2 + 1;
     } else {
-        P.mode = 0;
-        P.k1 = 7.99952f / (cb.hi[P.axis] - cb.lo[P.axis]);
-        P.k0 = cb.lo[P.axis];
+        P.k1 = cut.k1;
+        P.k0 = cut.k0;
     }
-    if (threadIdx.x == 0) params[blockIdx.x] = P;
-}
-
-__global__ __launch_bounds__(kSegThreads) void k_seg_bins(const GElem* src, const SegTask* tasks, const int* chunk_task,
-                                                           const SegParam* params, BinPart* part, int* err) {
-    __shared__ Box sh[kWaves];
-    __shared__ int shi[kWaves];
-    const ChunkRange c = chunk_range(tasks, chunk_task);
-    const SegParam P = params[c.task];
-    if (P.mode != 0) return;
-    const GElem* E = src + tasks[c.task].start;
-    const Cut cut{P.axis, 0, P.k0, P.k1};
-    int a, b;
-    thread_slice(c, &a, &b);
-    Bins B;
-    bins_init(B);
-    for (int i = a; i < b; i++) bins_add(B, E[i], cut, err);
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const Box r = block_fold<false>(B.b[k], sh);
-        int tot;
-        (void)block_scan_excl(B.n[k], shi, &tot);
-        if (threadIdx.x == 0) { part[blockIdx.x].b[k] = r; part[blockIdx.x].n[k] = tot; }
+    if (owner) params[c.task] = P;
+    if (flat) return;
+    const GElem* E = src + tk.start;
+    for (int i = c.first + (int)threadIdx.x; i < c.end; i += kSegThreads) {
+        const GElem e = E[i];
+        const float b[6] = {e.a.x, e.a.y, e.a.z, e.b.x, e.b.y, e.b.z};
+        bins_add(bins[wv].mine(), cut, cen(e.c, cut.axis), b, err);
+    }
+    wave_order();
+    bins_fold(bins[wv]);
+    __syncthreads();
+    if (threadIdx.x < kBinWords) {
+        const int w = threadIdx.x;
+        uint32_t x = bins[0].w[w];
+        for (int k = 1; k < kWaves; k++) x = bin_join(w, x, bins[k].w[w]);
+        part[blockIdx.x].w[w] = x;
     }
 }
 
 __global__ __launch_bounds__(kSegThreads) void k_seg_sah(const GElem* src, const SegTask* tasks, const BinPart* part,
                                                           SegParam* params) {
-    __shared__ Box sh[kWaves];
-    __shared__ int shi[kWaves];
+    __shared__ uint32_t sh[kWaves][kBinWords];
     const SegTask tk = tasks[blockIdx.x];
     SegParam P = params[blockIdx.x];
     if (P.mode != 0) return;
-    int a, b;
-    block_share(tk.nchunk, &a, &b);
-    Bins B;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        Box v = box_empty();
-        int m = 0;
-        for (int i = a; i < b; i++) { grow_box(v, part[tk.chunk0 + i].b[k]); m += part[tk.chunk0 + i].n[k]; }
-        B.b[k] = block_fold<false>(v, sh);
-        (void)block_scan_excl(m, shi, &B.n[k]);
+    const int wv = threadIdx.x >> 6, w = threadIdx.x & 63;
+    if (w < kBinWords) {
+        uint32_t x = bin_identity(w);
+        for (int i = wv; i < tk.nchunk; i += kWaves) x = bin_join(w, x, part[tk.chunk0 + i].w[w]);
+        sh[wv][w] = x;
     }
+    __syncthreads();
+    if (wv != 0) return;
+    if (w < kBinWords) {
+        uint32_t x = sh[0][w];
+        for (int k = 1; k < kWaves; k++) x = bin_join(w, x, sh[k][w]);
+        sh[0][w] = x;
+    }
+    wave_order();
     Cut cut{P.axis, 0, P.k0, P.k1};
-    sah(B, &cut.best, &P.nl);
+    sah_wave(sh[0], &cut.best, &P.nl);
     P.best = cut.best;
     P.pivot = P.nl;
     P.s = P.nl + ((P.nl < tk.n && cut.right(src[tk.start + P.nl].c)) ? 1 : 0);
@@ -565,36 +764,19 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_sah(const GElem* src, const
 
 __global__ __launch_bounds__(kSegThreads) void k_seg_rcount(const GElem* src, const SegTask* tasks,
                                                              const int* chunk_task, const SegParam* params, int* part) {
-    __shared__ int shi[kWaves];
+    __shared__ int sh[kWaves];
     const ChunkRange c = chunk_range(tasks, chunk_task);
     const SegParam P = params[c.task];
     if (P.mode != 0) return;
-    const GElem* E = src + tasks[c.task].start;
-    const Cut cut{P.axis, P.best, P.k0, P.k1};
     int a, b;
-    thread_slice(c, &a, &b);
-    int cnt = 0;
-    for (int i = a; i < b; i++) cnt += cut.right(E[i].c) ? 1 : 0;
-    int tot;
-    (void)block_scan_excl(cnt, shi, &tot);
-    if (threadIdx.x == 0) part[blockIdx.x] = tot;
-}
-
-// Exclusive scan of a task's chunk counts, in place.
-__global__ __launch_bounds__(kSegThreads) void k_seg_rscan(const SegTask* tasks, const SegParam* params, int* part) {
-    __shared__ int shi[kWaves];
-    const SegTask tk = tasks[blockIdx.x];
-    if (params[blockIdx.x].mode != 0) return;
-    int a, b;
-    block_share(tk.nchunk, &a, &b);
-    int m = 0;
-    for (int i = a; i < b; i++) m += part[tk.chunk0 + i];
-    int tot;
-    int run = block_scan_excl(m, shi, &tot);
-    for (int i = a; i < b; i++) {
-        const int x = part[tk.chunk0 + i];
-        part[tk.chunk0 + i] = run;
-        run += x;
+    wave_range(c, tasks[c.task].chunk, &a, &b);
+    const int cnt = wave_count(src + tasks[c.task].start, Cut{P.axis, P.best, P.k0, P.k1}, a, b);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int k = 0; k < kWaves; k++) tot += sh[k];
+        part[blockIdx.x] = tot;
     }
 }
 
@@ -602,25 +784,25 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_rscan(const SegTask* tasks,
 __global__ __launch_bounds__(kSegThreads) void k_seg_rank(const GElem* src, const SegTask* tasks, const int* chunk_task,
                                                            const SegParam* params, const int* part, int* rl_all,
                                                            int* lr_all, int* err) {
-    __shared__ int shi[kWaves];
+    __shared__ int sh_before[kWaves], sh_mine[kWaves];
     const ChunkRange c = chunk_range(tasks, chunk_task);
     const SegParam P = params[c.task];
     if (P.mode != 0) return;
     const SegTask tk = tasks[c.task];
     const GElem* E = src + tk.start;
-    int* rl = rl_all + tk.start;
-    int* lr = lr_all + tk.start;
     const Cut cut{P.axis, P.best, P.k0, P.k1};
     int a, b;
-    thread_slice(c, &a, &b);
-    int cnt = 0;
-    for (int i = a; i < b; i++) cnt += cut.right(E[i].c) ? 1 : 0;
-    int tot;
-    int r = part[blockIdx.x] + block_scan_excl(cnt, shi, &tot);
-    for (int i = a; i < b; i++) {
-        const bool right = cut.right(E[i].c);
-        r += right ? 1 : 0;
-        if (!record_rank(i, right, r, tk.n, P.nl, rl, lr)) atomicOr(err, 1);
+    wave_range(c, tk.chunk, &a, &b);
+    int r = rank_base(tk, part, wave_count(E, cut, a, b), sh_before, sh_mine);
+    const int lane = threadIdx.x & 63;
+    const uint64_t upto = ~0ull >> (63 - lane);
+    for (int i0 = a; i0 < b; i0 += 64) {
+        const int i = i0 + lane;
+        const bool right = i < b && cut.right(E[i].c);
+        const uint64_t m = __ballot(right);
+        if (i < b && !record_rank(i, right, r + __popcll(m & upto), tk.n, P.nl, rl_all + tk.start, lr_all + tk.start))
+            atomicOr(err, 1);
+        r += __popcll(m);
     }
 }
 
@@ -628,7 +810,7 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_scatter(const GElem* src, G
                                                               const int* chunk_task, const SegParam* params,
                                                               const int* part, const int* rl_all, const int* lr_all,
                                                               int* err) {
-    __shared__ int shi[kWaves];
+    __shared__ int sh_before[kWaves], sh_mine[kWaves];
     const ChunkRange c = chunk_range(tasks, chunk_task);
     const SegParam P = params[c.task];
     const SegTask tk = tasks[c.task];
@@ -638,22 +820,23 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_scatter(const GElem* src, G
         for (int i = c.first + (int)threadIdx.x; i < c.end; i += kSegThreads) D[i] = S[i];
         return;
     }
-    const int* rl = rl_all + tk.start;
-    const int* lr = lr_all + tk.start;
     const Cut cut{P.axis, P.best, P.k0, P.k1};
     int a, b;
-    thread_slice(c, &a, &b);
-    int cnt = 0;
-    for (int i = a; i < b; i++) cnt += cut.right(S[i].c) ? 1 : 0;
-    int tot;
-    int r = part[blockIdx.x] + block_scan_excl(cnt, shi, &tot);
-    for (int i = a; i < b; i++) {
-        const GElem e = S[i];
-        const bool right = cut.right(e.c);
-        r += right ? 1 : 0;
-        const int d = dest_of(i, right, r, tk.n, P.nl, P.s, rl, lr);
-        if (d >= 0) D[d] = e;
-        else atomicOr(err, 1);
+    wave_range(c, tk.chunk, &a, &b);
+    int r = rank_base(tk, part, wave_count(S, cut, a, b), sh_before, sh_mine);
+    const int lane = threadIdx.x & 63;
+    const uint64_t upto = ~0ull >> (63 - lane);
+    for (int i0 = a; i0 < b; i0 += 64) {
+        const int i = i0 + lane;
+        const GElem e = S[min(i, b - 1)];
+        const bool right = i < b && cut.right(e.c);
+        const uint64_t m = __ballot(right);
+        if (i < b) {
+            const int d = dest_of(i, right, r + __popcll(m & upto), tk.n, P.nl, P.s, rl_all + tk.start, lr_all + tk.start);
+            if (d >= 0) D[d] = e;
+            else atomicOr(err, 1);
+        }
+        r += __popcll(m);
     }
 }
 
@@ -693,16 +876,17 @@ __global__ void k_leaf_boxes(const GElem* E, const int2* leaves, int n, float* o
     for (int k = 0; k < 3; k++) { out[i * 6 + k] = b.lo[k]; out[i * 6 + 3 + k] = b.hi[k]; }
 }
 
-// Moves subtree s's nodes from the scratch area (offset src[s]) to their pre-order place dst[s],
-// offsetting child node indices.
-__global__ void k_place(const vgpu_qbvh_node* scratch, const int* src, const int* dst, const int* counts,
-                        vgpu_qbvh_node* out) {
+// Moves subtree s's nodes from the scratch area (offset src[s], in the order they were found) to their
+// pre-order place from dst[s] on, renumbering child nodes.
+__global__ void k_place(const vgpu_qbvh_node* scratch, const int* pre_all, const int* src, const int* dst,
+                        const int* counts, vgpu_qbvh_node* out) {
     const int s = blockIdx.y;
+    const int* pre = pre_all + src[s];
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < counts[s]; i += gridDim.x * blockDim.x) {
         vgpu_qbvh_node nd = scratch[src[s] + i];
         for (int c = 0; c < 4; c++)
-            if (nd.children[c] >= 0) nd.children[c] += dst[s];
-        out[dst[s] + i] = nd;
+            if (nd.children[c] >= 0) nd.children[c] = dst[s] + pre[nd.children[c]];
+        out[dst[s] + pre[i]] = nd;
     }
 }
 
@@ -863,20 +1047,54 @@ hipError_t stage_d2h(const HostSeg* segs, int nseg, hipStream_t st) {
 }
 
 
+// The device memory of one build: carved from one allocation sized for the element arrays and the usual
+// small ones (a build made 28 allocations and as many frees, each a synchronisation: 0.6 ms of 3.8 at
+// 300,001 elements), with further slabs where it does not suffice.  Freed together.
+struct Arena {
+    std::vector<void*> slabs;
+    char* cur = nullptr;
+    size_t left = 0;
+    Arena() = default;
+    Arena(const Arena&) = delete;
+    Arena& operator=(const Arena&) = delete;
+    ~Arena() { for (void* p : slabs) (void)hipFree(p); }
+    static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+    hipError_t slab(size_t bytes) {
+        void* p = nullptr;
+        const hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess) return e;
+        slabs.push_back(p);
+        cur = (char*)p;
+        left = bytes;
+        return hipSuccess;
+    }
+    hipError_t take(size_t bytes, void** out) {
+        bytes = padded(bytes);
+        if (bytes > left) {
+            const hipError_t e = slab(std::max(bytes, (size_t)1 << 20));
+            if (e != hipSuccess) return e;
+        }
+        *out = cur;
+        cur += bytes;
+        left -= bytes;
+        return hipSuccess;
+    }
+};
+
 template <class T>
 struct DevBuf {
+    Arena& arena;
     T* p = nullptr;
     size_t cap = 0;
-    DevBuf() = default;
+    explicit DevBuf(Arena& a) : arena(a) {}
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    hipError_t alloc(size_t n) {
+    hipError_t alloc(size_t n) {   // contents are not kept when it grows
         n = std::max<size_t>(n, 1);
         if (n <= cap) return hipSuccess;
-        if (p) { (void)hipFree(p); p = nullptr; cap = 0; }
-        const hipError_t e = hipMalloc((void**)&p, n * sizeof(T));
-        if (e == hipSuccess) cap = n;
+        void* q = nullptr;
+        const hipError_t e = arena.take(n * sizeof(T), &q);
+        if (e == hipSuccess) { p = (T*)q; cap = n; }
         return e;
     }
 };
@@ -900,44 +1118,49 @@ struct TopNode {
 // into `out`.
 struct SegRunner {
     hipStream_t st;
-    int leafMax;
-    DevBuf<SegTask> d_tasks;
-    DevBuf<int> d_chunk_task, d_rpart;
+    int leafMax, chunk;
+    DevBuf<int> d_work, d_rpart;     // the tasks, then the task of every chunk
     DevBuf<SegParam> d_params;
-    DevBuf<Box> d_cbpart;
+    DevBuf<KeyBox> d_cbpart;
     DevBuf<BinPart> d_binpart;
     std::vector<SegTask> tasks;
-    std::vector<int> chunk_task;
+    std::vector<int> chunk_task, work;
     std::vector<SegParam> params;
+
+    SegRunner(Arena& a, hipStream_t s, int leaf_max, int chunk_elems)
+        : st(s), leafMax(leaf_max), chunk(chunk_elems), d_work(a), d_rpart(a), d_params(a), d_cbpart(a), d_binpart(a) {}
 
     int run(const GElem* src, GElem* dst, const std::vector<int2>& ranges, int* rl, int* lr, int* err,
             std::vector<int2>& out) {
         tasks.clear();
         chunk_task.clear();
         for (size_t i = 0; i < ranges.size(); i++) {
-            const int nch = std::max(1, (ranges[i].y + kChunk - 1) / kChunk);
-            tasks.push_back(SegTask{ranges[i].x, ranges[i].y, (int)chunk_task.size(), nch});
+            const int nch = std::max(1, (ranges[i].y + chunk - 1) / chunk);
+            tasks.push_back(SegTask{ranges[i].x, ranges[i].y, (int)chunk_task.size(), nch, chunk});
             for (int k = 0; k < nch; k++) chunk_task.push_back((int)i);
         }
         const unsigned nt = (unsigned)tasks.size(), nc = (unsigned)chunk_task.size();
-        BUILD_TRY(d_tasks.alloc(nt));
+        constexpr size_t kTaskInts = sizeof(SegTask) / sizeof(int);
+        work.resize(nt * kTaskInts + nc);
+        std::memcpy(work.data(), tasks.data(), nt * sizeof(SegTask));
+        std::memcpy(work.data() + nt * kTaskInts, chunk_task.data(), nc * sizeof(int));
+        BUILD_TRY(d_work.alloc(work.size()));
         BUILD_TRY(d_params.alloc(nt));
-        BUILD_TRY(d_chunk_task.alloc(nc));
         BUILD_TRY(d_rpart.alloc(nc));
         BUILD_TRY(d_cbpart.alloc(nc));
         BUILD_TRY(d_binpart.alloc(nc));
-        BUILD_TRY(hipMemcpyAsync(d_tasks.p, tasks.data(), nt * sizeof(SegTask), hipMemcpyHostToDevice, st));
-        BUILD_TRY(hipMemcpyAsync(d_chunk_task.p, chunk_task.data(), nc * sizeof(int), hipMemcpyHostToDevice, st));
+        BUILD_TRY(hipMemcpyAsync(d_work.p, work.data(), work.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        const SegTask* d_tasks = (const SegTask*)d_work.p;
+        const int* d_chunk_task = d_work.p + nt * kTaskInts;
         const dim3 blk(kSegThreads);
-        hipLaunchKernelGGL(k_seg_cb, dim3(nc), blk, 0, st, src, d_tasks.p, d_chunk_task.p, leafMax, d_cbpart.p);
-        hipLaunchKernelGGL(k_seg_axis, dim3(nt), blk, 0, st, d_tasks.p, d_cbpart.p, leafMax, d_params.p);
-        hipLaunchKernelGGL(k_seg_bins, dim3(nc), blk, 0, st, src, d_tasks.p, d_chunk_task.p, d_params.p, d_binpart.p, err);
-        hipLaunchKernelGGL(k_seg_sah, dim3(nt), blk, 0, st, src, d_tasks.p, d_binpart.p, d_params.p);
-        hipLaunchKernelGGL(k_seg_rcount, dim3(nc), blk, 0, st, src, d_tasks.p, d_chunk_task.p, d_params.p, d_rpart.p);
-        hipLaunchKernelGGL(k_seg_rscan, dim3(nt), blk, 0, st, d_tasks.p, d_params.p, d_rpart.p);
-        hipLaunchKernelGGL(k_seg_rank, dim3(nc), blk, 0, st, src, d_tasks.p, d_chunk_task.p, d_params.p, d_rpart.p, rl,
+        hipLaunchKernelGGL(k_seg_cb, dim3(nc), blk, 0, st, src, d_tasks, d_chunk_task, leafMax, d_cbpart.p);
+        hipLaunchKernelGGL(k_seg_bins, dim3(nc), blk, 0, st, src, d_tasks, d_chunk_task, d_cbpart.p, leafMax,
+                           d_params.p, d_binpart.p, err);
+        hipLaunchKernelGGL(k_seg_sah, dim3(nt), blk, 0, st, src, d_tasks, d_binpart.p, d_params.p);
+        hipLaunchKernelGGL(k_seg_rcount, dim3(nc), blk, 0, st, src, d_tasks, d_chunk_task, d_params.p, d_rpart.p);
+        hipLaunchKernelGGL(k_seg_rank, dim3(nc), blk, 0, st, src, d_tasks, d_chunk_task, d_params.p, d_rpart.p, rl,
                            lr, err);
-        hipLaunchKernelGGL(k_seg_scatter, dim3(nc), blk, 0, st, src, dst, d_tasks.p, d_chunk_task.p, d_params.p,
+        hipLaunchKernelGGL(k_seg_scatter, dim3(nc), blk, 0, st, src, dst, d_tasks, d_chunk_task, d_params.p,
                            d_rpart.p, rl, lr, err);
         BUILD_TRY(hipGetLastError());
         params.resize(nt);
@@ -964,18 +1187,23 @@ int build_qbvh_gpu(float* boxes, float* centroids, int32_t* idx, int32_t n, int3
     if (leafMax > 16) leafMax = 16;
     if (leafMax < 1) leafMax = 1;
     const size_t N = (size_t)std::max(n, 1);
-    DevBuf<float> d_boxes, d_cent, d_rootbox, d_leafbox;
-    DevBuf<int32_t> d_idx;
-    DevBuf<GElem> d_E, d_T;
-    DevBuf<int> d_rl, d_lr, d_err, d_counts, d_src, d_dst;
-    DevBuf<int2> d_roots, d_leaves;
-    DevBuf<vgpu_qbvh_node> d_scratch, d_nodes;
+    // boxes, centroids, indices, elements (twice with ranges to split), ranks, pre-order numbers, scratch
+    // nodes; and a 16th of those again for the final nodes (leafMax 16 makes one per 22 elements) and the small arrays
+    Arena arena;
+    const size_t per = 40 + sizeof(GElem) + 4 + sizeof(vgpu_qbvh_node) + (n > kSubtreeMax ? sizeof(GElem) + 8 : 0);
+    BUILD_TRY(arena.slab(N * per + N * sizeof(vgpu_qbvh_node) / 16 + ((size_t)1 << 18)));
+    DevBuf<float> d_boxes(arena), d_cent(arena), d_rootbox(arena), d_leafbox(arena);
+    DevBuf<int32_t> d_idx(arena);
+    DevBuf<GElem> d_E(arena), d_T(arena);
+    DevBuf<int> d_rl(arena), d_lr(arena), d_err(arena), d_counts(arena), d_src(arena), d_dst(arena), d_pre(arena);
+    DevBuf<int2> d_roots(arena), d_leaves(arena);
+    DevBuf<vgpu_qbvh_node> d_scratch(arena), d_nodes(arena);
     BUILD_TRY(d_boxes.alloc(N * 6));
     BUILD_TRY(d_cent.alloc(N * 3));
     BUILD_TRY(d_idx.alloc(N));
     BUILD_TRY(d_E.alloc(N));
-    BUILD_TRY(d_T.alloc(N));
     BUILD_TRY(d_err.alloc(1));
+    BUILD_TRY(d_pre.alloc(N));
     BUILD_TRY(d_scratch.alloc(N));
     BUILD_TRY(hipMemsetAsync(d_err.p, 0, sizeof(int), st));
     if (n > 0) {
@@ -1022,14 +1250,13 @@ int build_qbvh_gpu(float* boxes, float* centroids, int32_t* idx, int32_t n, int3
         r.n = n;
         top.push_back(r);
         level.push_back(0);
+        BUILD_TRY(d_T.alloc(N));
         BUILD_TRY(d_rl.alloc(N));
         BUILD_TRY(d_lr.alloc(N));
     } else {
         subtrees.push_back(make_int2(0, n));
     }
-    SegRunner seg;
-    seg.st = st;
-    seg.leafMax = leafMax;
+    SegRunner seg(arena, st, leafMax, n < kChunkLargeFrom ? kChunkSmall : kChunkLarge);
     std::vector<int2> ranges, r0, r12;
     while (!level.empty()) {
         const std::vector<int> cur = level;
@@ -1073,8 +1300,8 @@ int build_qbvh_gpu(float* boxes, float* centroids, int32_t* idx, int32_t n, int3
         BUILD_TRY(d_counts.alloc(nsub));
         BUILD_TRY(d_rootbox.alloc((size_t)nsub * 6));
         BUILD_TRY(hipMemcpyAsync(d_roots.p, subtrees.data(), nsub * sizeof(int2), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_subtree, dim3(nsub), dim3(64), 0, st, d_E.p, d_T.p, d_roots.p, d_scratch.p, d_counts.p,
-                           d_rootbox.p, leafMax, d_err.p);
+        hipLaunchKernelGGL(k_subtree, dim3(nsub), dim3(kSubThreads), 0, st, d_E.p, d_roots.p, d_scratch.p, d_pre.p,
+                           d_counts.p, d_rootbox.p, leafMax, d_err.p);
         BUILD_TRY(hipGetLastError());
         BUILD_TRY(hipMemcpyAsync(counts.data(), d_counts.p, nsub * sizeof(int), hipMemcpyDeviceToHost, st));
         BUILD_TRY(hipMemcpyAsync(rootbox.data(), d_rootbox.p, (size_t)nsub * 6 * sizeof(float), hipMemcpyDeviceToHost,
@@ -1125,8 +1352,8 @@ int build_qbvh_gpu(float* boxes, float* centroids, int32_t* idx, int32_t n, int3
         BUILD_TRY(d_dst.alloc(nsub));
         BUILD_TRY(hipMemcpyAsync(d_src.p, src.data(), nsub * sizeof(int), hipMemcpyHostToDevice, st));
         BUILD_TRY(hipMemcpyAsync(d_dst.p, sub_dst.data(), nsub * sizeof(int), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_place, dim3(8, nsub), dim3(256), 0, st, d_scratch.p, d_src.p, d_dst.p, d_counts.p,
-                           d_nodes.p);
+        hipLaunchKernelGGL(k_place, dim3(8, nsub), dim3(256), 0, st, d_scratch.p, d_pre.p, d_src.p, d_dst.p,
+                           d_counts.p, d_nodes.p);
         BUILD_TRY(hipGetLastError());
     }
     if (n > 0) {

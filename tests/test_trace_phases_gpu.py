@@ -1,7 +1,7 @@
 """Edges of the traversal kernel's box test, stack and leaf dealing.
 
 Workload: a 1,000-triangle sphere over a quad, and an icosphere field of 8 spheres; ray counts around
-whole wavefronts; accels whose child boxes hold their bounds the wrong way round or a NaN bound.
+whole wavefronts and around the counts where a wavefront takes more rays; accels whose child boxes hold their bounds the wrong way round or a NaN bound.
 Bar: every hit and per-ray counter bit-identical with the oracle, or with the scene whose boxes are in
 order: MINPS/MAXPS of the two slab values do not depend on which bound is which.
 """
@@ -25,7 +25,7 @@ def _bits(h):
     return h.view(np.uint32).reshape(len(h), -1)
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 4097])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 4097, 8193, 32769, 131071, 300001])
 @pytest.mark.parametrize("name", ["sphere", "field"])
 def test_ray_counts_around_wavefronts(name, n):
     g, o = va.Scene(0), oracle.OracleScene()
@@ -143,3 +143,33 @@ def test_transform_scenes_at_odd_sizes(count, n):
         assert np.array_equal(dh.cpu().numpy().view(np.uint32), _bits(hits))
         assert np.array_equal(dg.cpu().numpy(), geoms)
     R.close()
+
+
+@pytest.mark.parametrize("sort", [0, 3])
+@pytest.mark.parametrize("size", [(37, 29), (64, 33)])
+def test_shadow_rays_listed_per_pass(size, sort):
+    """Film, sample and shadow-ray count of the feature scene (mirrors, two lights) at pixel counts off whole
+    workgroups do not depend on the scene's ray sort, and the device counts the rays listed."""
+    from vermeer_amd import render
+    w, h = size
+    desc = scenes.feature_scene()
+    c = desc["camera"]
+    M, ttf = oracle.camera_lookat(c["from"], c["to"], c["up"], c["fov"], c["focal"])
+    cam = np.zeros((), va._lib.CAMERA_DTYPE)
+    cam["M"], cam["tan_theta_focal"], cam["aspect"], cam["focal"] = M, ttf, w / h, c["focal"]
+    R = render.Renderer(desc, w, h, cam)
+    R.scene.set_trace_config(64, 12, 20, sort=sort)
+    plain = render.Renderer(desc, w, h, cam)
+    scr = scenes.pixel_scrambles(w, h)
+    total = 0
+    for it in (1, 2):
+        n, samp = R.render_pass(scr, it, want_sample=True)
+        m, ref = plain.render_pass(scr, it, want_sample=True)
+        assert n == m > 0
+        total += n
+        assert samp.tobytes() == ref.tobytes()
+    assert R.film.tobytes() == plain.film.tobytes()
+    closest, shadow = R.stats()
+    assert shadow == total and closest >= 2 * w * h
+    R.close()
+    plain.close()

@@ -335,6 +335,7 @@ struct vgpu_render {
     float4* d_slot_rays = nullptr;
     float4* d_slot_rgb = nullptr;
     int4* d_slot_hits = nullptr;
+    uint32_t* d_list = nullptr;               // slots holding shadow rays, then (one entry) their number
     float4* d_groups = nullptr;
     float4* d_pixshade = nullptr;
     void* d_stage = nullptr;       // host-pointer mode: scrambles, film, samples
@@ -346,7 +347,7 @@ struct vgpu_render {
         int prev = 0;
         if (hipGetDevice(&prev) == hipSuccess && scene) (void)hipSetDevice(scene->device);
         void* ptrs[] = {d_materials, d_lights, d_rays, d_rays2, d_recs, d_filter, d_camkeys, d_pix, d_hits32, d_slot_rays,
-                        d_slot_rgb, d_slot_hits, d_groups, d_pixshade, d_stage, d_counts};
+                        d_slot_rgb, d_slot_hits, d_groups, d_pixshade, d_stage, d_counts, d_list};
         for (void* p : ptrs) if (p) (void)hipFree(p);
         (void)hipSetDevice(prev);
     }
@@ -443,6 +444,7 @@ int vgpu_render_create(vgpu_render** out, vgpu_scene* s, const vgpu_material* ma
     if (e == hipSuccess) e = alloc((void**)&r->d_slot_rays, ns * 32);
     if (e == hipSuccess) e = alloc((void**)&r->d_slot_rgb, ns * 16);
     if (e == hipSuccess) e = alloc((void**)&r->d_slot_hits, ns * 16);
+    if (e == hipSuccess) e = alloc((void**)&r->d_list, (ns + 1) * 4);
     if (e == hipSuccess) e = alloc((void**)&r->d_groups, np * (size_t)rv.groups * 16);
     if (e == hipSuccess) e = alloc((void**)&r->d_pixshade, np * 64);
     if (e == hipSuccess) e = alloc((void**)&r->d_counts, 2 * sizeof(unsigned long long));
@@ -503,7 +505,6 @@ int vgpu_render_pass(vgpu_render* r, uint32_t flags, const uint64_t* scrambles, 
     const bool graph = (flags & VGPU_GRAPH) != 0;
     if (graph && host) return fail(VGPU_ERR_ARG, "VGPU_GRAPH needs VGPU_TRACE_DEVICE_PTRS");
     if (graph && s->timing) return fail(VGPU_ERR_STATE, "VGPU_GRAPH with kernel timing enabled");
-    if (graph && s->cfg.sort > 0) { const int rc = ensure_sort(s, ns); if (rc) return rc; }
     uint64_t shadow_count = 0;
     // The pass's launches, on the caller's stream or on the capture stream of the pass's graph.
     auto enqueue = [&](hipStream_t st) -> int {
@@ -516,11 +517,11 @@ int vgpu_render_pass(vgpu_render* r, uint32_t flags, const uint64_t* scrambles, 
                                        s->num_cus, st);
             if (e != hipSuccess) return fail(VGPU_ERR_HIP, "closest hit: %s", hipGetErrorString(e));
             e = vgpu::launch_shade(r->rv, d_scr, iter, level, rin, r->d_hits32, r->d_pix, r->d_slot_rays, r->d_slot_rgb,
-                                   r->d_groups, r->d_pixshade, rout, r->d_recs, st);
+                                   r->d_groups, r->d_pixshade, rout, r->d_recs, r->d_list, r->d_list + ns, st);
             if (e != hipSuccess) return fail(VGPU_ERR_HIP, "shade: %s", hipGetErrorString(e));
             if (r->rv.groups > 0) {   // without lights no slot holds a shadow ray
                 const int rc = enqueue_trace(s, VGPU_TRACE_SHADOW | VGPU_TRACE_DEVICE_PTRS, r->d_slot_rays, ns,
-                                             r->d_slot_hits, nullptr, nullptr, st, s->cfg);
+                                             r->d_slot_hits, nullptr, nullptr, st, s->cfg, r->d_list + ns, r->d_list);
                 if (rc) return rc;
             }
             const bool direct = r->rv.max_level == 0;
@@ -528,11 +529,11 @@ int vgpu_render_pass(vgpu_render* r, uint32_t flags, const uint64_t* scrambles, 
                                      direct ? d_film : nullptr, direct ? d_samp : nullptr, st);
             if (e != hipSuccess) return fail(VGPU_ERR_HIP, "resolve: %s", hipGetErrorString(e));
             if (host && shadow_rays_out && r->rv.groups > 0) {
-                // count active slots (diagnostic, host mode only)
-                std::vector<float4> rgb(ns);
-                HIP_TRY(hipMemcpyAsync(rgb.data(), r->d_slot_rgb, ns * 16, hipMemcpyDeviceToHost, st));
+                // shadow rays of the level (diagnostic, host mode only)
+                uint32_t on = 0;
+                HIP_TRY(hipMemcpyAsync(&on, r->d_list + ns, sizeof(on), hipMemcpyDeviceToHost, st));
                 HIP_TRY(hipStreamSynchronize(st));
-                for (const float4& v : rgb) shadow_count += v.w != 0.0f;
+                shadow_count += on;
             }
         }
         if (r->rv.max_level > 0) {

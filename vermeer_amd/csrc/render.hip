@@ -12,7 +12,8 @@
 //              EvaluateLightSamples (core/shader.go:203-402).  Every sample that
 //              would trace a shadow ray gets a slot: the shadow ray and the
 //              colour it adds if unoccluded.
-//   (trace)    shadow any-hit over all slots (trace.hip)
+//   k_slots    lists the slots that hold shadow rays
+//   (trace)    shadow any-hit over the listed slots (trace.hip)
 //   k_resolve  sums the unoccluded slot colours in the reference's order,
 //              applies the per-light / per-lobe scales and updates the film as
 //              fb = (fb*iter + c)/(iter + 1) (core/render.go:127-129).
@@ -680,31 +681,26 @@ __device__ V3 offset_p(const SC& sc, int dir) {
 
 struct SlotOut {
     float4* rays;   // 2 float4 per slot
-    float4* rgb;    // 1 float4 per slot: colour if unoccluded, w = 1 when a shadow ray is traced
+    float4* rgb;    // 1 float4 per slot: colour if unoccluded
     float time;     // ray time of the shaded hit, inherited by its shadow rays (core/ray.go:65)
 };
 
-__device__ __forceinline__ void slot_off(const SlotOut& so, int s) {
-    so.rays[2 * s] = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
-    so.rays[2 * s + 1] = make_float4(0.0f, 0.0f, 1.0f, 0.0f);
-    so.rgb[s] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
 __device__ __forceinline__ void slot_on(const SlotOut& so, int s, V3 o, V3 d, RGB c) {
     so.rays[2 * s] = make_float4(o.x, o.y, o.z, 1.0f);   // tmax 1: D spans the distance to the light
     so.rays[2 * s + 1] = make_float4(d.x, d.y, d.z, so.time);
     so.rgb[s] = make_float4(c.r, c.g, c.b, 1.0f);
 }
 
-// EvaluateLightSamples (core/shader.go:203-402) up to the shadow tests: fills the group's slots
-// [base, base + sg_slots) and returns the group record {scale, mode}.  Not inlined: k_shade then
+// EvaluateLightSamples (core/shader.go:203-402) up to the shadow tests: fills the group's slots from
+// base on, one per shadow ray in the order of the samples, and returns the group record {scale, mode, shadow
+// rays}.  Not inlined: k_shade then
 // needs 214 instead of 256 VGPRs + 86 AGPRs, runs two waves per SIMD instead of one, and the
 // box-and-spheres pass is 5% faster.
 template <class B>
 __device__ __noinline__ float4 light_samples(const DevLight& L, const vgpu_material& lm, const SC& sc, const B& bsdf, int NS,
-                                const SlotOut& so, int base, int sg_slots) {
+                                const SlotOut& so, int base) {
     const float k = 1.0f - 0.0001f;   // 1 - ShadowRayEpsilon (core/ray.go:22)
-    int on = 0;                       // shadow rays set up (returned in .z)
-    for (int s = 0; s < sg_slots; s++) slot_off(so, base + s);
+    int on = 0;                       // shadow rays set up
     if (NS > 1) {
         const int half = NS / 2;
         int nB = 0, nL = 0;
@@ -732,8 +728,7 @@ __device__ __noinline__ float4 light_samples(const DevLight& L, const vgpu_mater
             if (c.r < 0) c.r = 0;
             if (c.g < 0) c.g = 0;
             if (c.b < 0) c.b = 0;
-            slot_on(so, base + i, o, scale(l.ldist * k, l.ld), c);
-            on++;
+            slot_on(so, base + on++, o, scale(l.ldist * k, l.ld), c);
         }
         for (int i = 0; i < half; i++) {
             const uint64_t idx = sc.I * (uint64_t)half + (uint64_t)i;
@@ -752,8 +747,7 @@ __device__ __noinline__ float4 light_samples(const DevLight& L, const vgpu_mater
             if (c.r < 0) c.r = 0;
             if (c.g < 0) c.g = 0;
             if (c.b < 0) c.b = 0;
-            slot_on(so, base + half + i, o, scale(b.ldist * k, b.ld), c);
-            on++;
+            slot_on(so, base + on++, o, scale(b.ldist * k, b.ld), c);
         }
         return make_float4(1.0f / (float)total, 1.0f, (float)on, 0.0f);
     }
@@ -764,8 +758,7 @@ __device__ __noinline__ float4 light_samples(const DevLight& L, const vgpu_mater
         Spec rho = bsdf.eval(l.ld);
         spec_mul(rho, l.liu);
         spec_scale(rho, 1.0f / l.pdf);
-        slot_on(so, base + i, o, scale(l.ldist * k, l.ld), spec_to_rgb(rho));
-        on++;
+        slot_on(so, base + on++, o, scale(l.ldist * k, l.ld), spec_to_rgb(rho));
     }
     return make_float4(1.0f, 2.0f, (float)on, 0.0f);
 }
@@ -965,7 +958,6 @@ __device__ __forceinline__ int shade_pixel(int& next, const RenderView& rv, cons
     }
     const bool path = rv.path_depth > 0;
     if (mat < 0) {   // a miss, or a geom without a shader: core.Trace reports no hit (trace.go:62-64)
-        for (int s = 0; s < rv.slots; s++) slot_off(so, s);
         for (int q = 0; q < rv.groups; q++) grp[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         ps[0] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         rec->a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1138,10 +1130,8 @@ __device__ __forceinline__ int shade_pixel(int& next, const RenderView& rv, cons
         const vgpu_material lm = rv.materials[L.material];
         const int b0 = (2 * l) * SGS, b1 = (2 * l + 1) * SGS;
         float4 g0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), g1 = g0;
-        if (!skip && diff_on) g0 = light_samples(L, lm, sc, on, NS, so, b0, SGS);
-        else for (int s = 0; s < SGS; s++) slot_off(so, b0 + s);
-        if (!skip && spec_on) g1 = light_samples(L, lm, sc, gx, NS, so, b1, SGS);
-        else for (int s = 0; s < SGS; s++) slot_off(so, b1 + s);
+        if (!skip && diff_on) g0 = light_samples(L, lm, sc, on, NS, so, b0);
+        if (!skip && spec_on) g1 = light_samples(L, lm, sc, gx, NS, so, b1);
         grp[2 * l] = g0;
         grp[2 * l + 1] = g1;
         nrays += (int)g0.z + (int)g1.z;
@@ -1247,8 +1237,9 @@ __global__ __launch_bounds__(128) void k_shade(RenderView rv, const uint64_t* __
                                                const float4* __restrict__ pix, float4* __restrict__ slot_rays,
                                                float4* __restrict__ slot_rgb, float4* __restrict__ groups,
                                                float4* __restrict__ pixshade, float4* __restrict__ rays_out,
-                                               LevelRec* __restrict__ recs) {
+                                               LevelRec* __restrict__ recs, uint32_t* __restrict__ nlist) {
     int next;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nlist = 0;   // for k_slots, the next launch
     const int nshadow = shade_pixel(next, rv, scr, iter, level, rays_in, hits32, pix, slot_rays, slot_rgb, groups, pixshade,
                                     rays_out, recs);
     if (rv.counts) {
@@ -1257,6 +1248,46 @@ __global__ __launch_bounds__(128) void k_shade(RenderView rv, const uint64_t* __
     }
 }
 
+
+// The slots holding shadow rays, as a list for the any-hit launch: most slots hold none (1.7 of 8 do per
+// pixel in the box of spheres), and tracing all of them spent the launch on lanes without work (512^2
+// pixels: 270 us for the launch, 214 with the list and 11 for making it; a frame 652 -> 593 us, unused slots
+// no longer written and read).  A wavefront lists its pixels' slots group by group and sample by sample, so neighbouring entries
+// are neighbouring pixels' rays to one light; one atomic per 1024 pixels.
+constexpr int kSlotsBlock = 1024;
+__global__ __launch_bounds__(kSlotsBlock) void k_slots(RenderView rv, const float4* __restrict__ groups,
+                                                       uint32_t* __restrict__ list, uint32_t* __restrict__ nlist) {
+    constexpr int kW = kSlotsBlock / 64;
+    __shared__ uint32_t sh[kW + 1];
+    const int p = blockIdx.x * kSlotsBlock + (int)threadIdx.x;
+    const bool in = p < rv.width * rv.height;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int SGS = 2 * rv.max_half;
+    const float4* grp = groups + (size_t)p * rv.groups;
+    uint32_t n = 0;
+    for (int q = 0; q < rv.groups; q++) n += in ? (uint32_t)(int)grp[q].z : 0u;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
+    if (lane == 0) sh[wv] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t run = 0;
+        for (int k = 0; k < kW; k++) { const uint32_t x = sh[k]; sh[k] = run; run += x; }
+        sh[kW] = run > 0 ? atomicAdd(nlist, run) : 0u;
+    }
+    __syncthreads();
+    uint32_t at = sh[kW] + sh[wv];
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int q = 0; q < rv.groups; q++) {
+        const int on = in ? (int)grp[q].z : 0;
+        for (int s = 0; s < SGS; s++) {
+            const uint64_t m = __ballot(s < on);
+            if (m == 0) break;
+            if (s < on) list[at + (uint32_t)__popcll(m & below)] = (uint32_t)p * (uint32_t)rv.slots + (uint32_t)(q * SGS + s);
+            at += (uint32_t)__popcll(m);
+        }
+    }
+}
 
 // Sums one level's unoccluded slot colours in the reference's order and applies the per-light / per-lobe
 // scales: a = (0 + emission) + diffuse, and for a rough specular lobe s = its direct lighting.
@@ -1302,9 +1333,10 @@ __global__ __launch_bounds__(256) void k_resolve(RenderView rv, int level, uint3
             RGB col = rgb0();
             if (gr.y != 0.0f) {
                 const int base = (2 * l + lobe) * SGS;
-                for (int s = 0; s < SGS; s++) {
+                const int on = (int)gr.z;
+                for (int s = 0; s < on; s++) {
                     const float4 c = rgb[base + s];
-                    if (c.w != 0.0f && hit[base + s].x < 0) rgb_add(col, RGB{c.x, c.y, c.z});
+                    if (hit[base + s].x < 0) rgb_add(col, RGB{c.x, c.y, c.z});
                 }
                 if (gr.y == 1.0f) rgb_scale(col, gr.x);
             }
@@ -1391,10 +1423,14 @@ hipError_t launch_camera(const RenderView& rv, const uint64_t* scr, uint32_t ite
 
 hipError_t launch_shade(const RenderView& rv, const uint64_t* scr, uint32_t iter, int level, const float4* rays_in,
                         const int4* hits32, const float4* pix, float4* slot_rays, float4* slot_rgb, float4* groups,
-                        float4* pixshade, float4* rays_out, LevelRec* recs, hipStream_t stream) {
+                        float4* pixshade, float4* rays_out, LevelRec* recs, uint32_t* list, uint32_t* nlist,
+                        hipStream_t stream) {
     const int n = rv.width * rv.height;
     hipLaunchKernelGGL(k_shade, dim3((n + 127) / 128), dim3(128), 0, stream, rv, scr, iter, level, rays_in, hits32, pix,
-                       slot_rays, slot_rgb, groups, pixshade, rays_out, recs);
+                       slot_rays, slot_rgb, groups, pixshade, rays_out, recs, nlist);
+    if (rv.groups > 0)
+        hipLaunchKernelGGL(k_slots, dim3((n + kSlotsBlock - 1) / kSlotsBlock), dim3(kSlotsBlock), 0, stream, rv,
+                           (const float4*)groups, list, nlist);
     return hipGetLastError();
 }
 

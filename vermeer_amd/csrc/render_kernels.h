@@ -75,12 +75,14 @@ constexpr int kMaxLevel = 3;       // ShaderStd.Eval returns at once above level
 constexpr int kMaxPathDepth = 16;  // path mode: segments per path
 
 // Launch wrappers (all enqueue on `stream`).  Levels: rays_in holds the level's rays (P, tmax; D,
-// time), rays_out receives the next level's mirror rays (inactive pixels get tmax -1).
+// time), rays_out receives the next level's mirror rays (inactive pixels get tmax -1).  launch_shade also lists
+// the slots that hold shadow rays: list (width * height * slots entries) and their number, *nlist.
 hipError_t launch_camera(const RenderView& rv, const uint64_t* scrambles, uint32_t iter, float4* rays, float4* pix,
                          hipStream_t stream);
 hipError_t launch_shade(const RenderView& rv, const uint64_t* scrambles, uint32_t iter, int level, const float4* rays_in,
                         const int4* hits32, const float4* pix, float4* slot_rays, float4* slot_rgb, float4* groups,
-                        float4* pixshade, float4* rays_out, LevelRec* recs, hipStream_t stream);
+                        float4* pixshade, float4* rays_out, LevelRec* recs, uint32_t* list, uint32_t* nlist,
+                        hipStream_t stream);
 // film null: record the level for launch_combine; otherwise (no mirrors) update the film directly.
 hipError_t launch_resolve(const RenderView& rv, int level, uint32_t iter, const float4* slot_rgb, const int4* slot_hits,
                           const float4* groups, const float4* pixshade, LevelRec* recs, float* film, float* sample_out,

@@ -356,7 +356,7 @@ hipEvent_t timing_event(vgpu_scene* s) {
 }
 
 int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n, void* d_hits, int32_t* d_geoms,
-                  int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev) {
+                  int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev, const uint32_t* list) {
     if (d_counters && s->view.any_xform)
         return fail(VGPU_ERR_ARG, "per-ray counters are not kept for scenes with instances, procs or mesh transforms");
     const vgpu::TraceLaunch L = vgpu::scene_launch(
@@ -370,8 +370,8 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
         if (!ev[0] || !ev[1] || !ev[2]) return fail(VGPU_ERR_HIP, "timing events");
         HIP_TRY(hipEventRecord(ev[0], st));
     }
-    const uint32_t* perm = nullptr;
-    if (cfg.sort > 0) {
+    const uint32_t* perm = list;
+    if (cfg.sort > 0 && !list) {
         if (n > 0xffffffffull) return fail(VGPU_ERR_ARG, "ray sorting handles at most 2^32-1 rays per call");
         if ((rc = ensure_sort(s, n))) return rc;
         hipError_t e = vgpu::launch_ray_sort(s->box, cfg.sort, d_rays, n, n_dev, s->sort, s->num_cus, st);
@@ -382,7 +382,7 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
     if (ev[1]) HIP_TRY(hipEventRecord(ev[1], st));
     hipError_t e = vgpu::launch_trace(s->view, (flags & VGPU_TRACE_SHADOW) != 0, s->any_motion, L, d_rays, n, d_hits,
                                       d_geoms, d_counters, s->d_spT, s->d_spN, s->spill_threads, s->d_err, s->num_cus, st,
-                                      n_dev, perm);
+                                      n_dev, perm, list != nullptr);
     if (e != hipSuccess) return fail(VGPU_ERR_HIP, "trace launch: %s", hipGetErrorString(e));
     if (ev[2]) HIP_TRY(hipEventRecord(ev[2], st));
     return VGPU_OK;

@@ -202,8 +202,9 @@ struct GraphCache {
     int run(hipStream_t st, const std::function<int(hipStream_t)>& body);
 };
 // Enqueues one traversal (device pointers) with configuration cfg.  n_dev (nullable): device-resident
-// count of rays to trace, at most n.
+// count of rays to trace, at most n.  list (nullable): the slots of d_rays and d_hits to trace, in order
+// (they are not sorted).
 int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n, void* d_hits, int32_t* d_geoms,
-                  int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev = nullptr);
+                  int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev = nullptr, const uint32_t* list = nullptr);
 
 }  // namespace vgpu_detail

@@ -22,6 +22,7 @@
 // Compiled with -ffp-contract=off: every float operation rounds as the
 // reference's unfused SSE code does.
 
+#include <algorithm>
 #include <mutex>
 
 #include "trace_kernels.h"
@@ -577,7 +578,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                                            int4* __restrict__ counters, float* __restrict__ spT,
                                            int32_t* __restrict__ spN, int32_t* __restrict__ err,
                                            const uint32_t* __restrict__ n_dev, const uint32_t* __restrict__ perm,
-                                           int refill_min) {
+                                           int gather, int ray_shift, int refill_min) {
     static_assert(BLOCK % 64 == 0, "whole wavefronts");
     static_assert(LDS >= 4, "a node step's pushes are checked against LDS - 3");
     constexpr int kEntry = BLOCK * 8;             // bytes from one stack entry of a lane to the next
@@ -588,6 +589,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     const int lane = tid & 63;
     const uint64_t gtid = (uint64_t)blockIdx.x * BLOCK + tid;
     const uint64_t nthr = (uint64_t)gridDim.x * BLOCK;
+    const uint64_t nwaves = nthr / 64;
     const int bottom = tid * 8;                   // the lane's empty stack: entry i at bottom + i * kEntry
 
     auto spill = [&](int sp) { return (uint64_t)((uint32_t)sp / kEntry - LDS) * nthr + (uint32_t)gtid; };
@@ -597,8 +599,12 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     };
 
     if (n_dev) n = min(n, (uint64_t)*n_dev);
-    // Rays of this wavefront: v = 0, 1, 2, ... -> ray wave0 + (v / 64) * nthr + v % 64 (increasing in v).
-    const uint64_t wave0 = (uint64_t)blockIdx.x * BLOCK + (uint32_t)__builtin_amdgcn_readfirstlane(tid & ~63);
+    // Rays of this wavefront: v = 0, 1, 2, ... -> ray_of(v), increasing in v: 2^ray_shift consecutive rays, then
+    // as many nwaves * 2^ray_shift further on (trace_ray_shift).
+    const uint64_t wave = (uint64_t)blockIdx.x * (BLOCK / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
+    auto ray_of = [&](uint32_t v) {
+        return (((uint64_t)(v >> ray_shift) * nwaves + wave) << ray_shift) + (v & ((1u << ray_shift) - 1u));
+    };
     uint32_t cursor = 0;
     bool ok = true, fast = false;
     int ri = kNoRay;                              // launches hold fewer than 2^32 rays; ~0 is never one
@@ -626,8 +632,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     int cur = kIdle;
     while (true) {
         const uint64_t dm = __ballot(cur == kIdle);
-        const uint64_t next = wave0 + (uint64_t)(cursor >> 6) * nthr + (cursor & 63u);
-        const bool more = next < n;
+        const bool more = ray_of(cursor) < n;
         if (more ? __popcll(dm) >= refill_min : dm == ~0ull) {
             if (cur == kIdle) {
                 if (ri != kNoRay) {
@@ -636,7 +641,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                         best_geom = -1; best_prim = -1;
                         if (XFORM) best_leaf = -1;
                     }
-                    const uint64_t oi = perm ? (uint64_t)perm[(uint32_t)ri] : (uint64_t)(uint32_t)ri;
+                    const uint64_t oi = perm && !gather ? (uint64_t)perm[(uint32_t)ri] : (uint64_t)(uint32_t)ri;
                     if (EXT) {
                         hits[2 * oi] = make_int4(best_prim, best_geom, __float_as_int(r.tclosest), __float_as_int(bu));
                         hits[2 * oi + 1] = make_int4(__float_as_int(bv), __float_as_int(bw), best_leaf, 0);
@@ -649,17 +654,22 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                 }
                 if (more) {
                     const uint32_t v = cursor + (uint32_t)__popcll(dm & ((1ull << lane) - 1ull));
-                    const uint64_t rnext = wave0 + (uint64_t)(v >> 6) * nthr + (v & 63u);
+                    const uint64_t rnext = ray_of(v);
                     ok = true;
                     if (rnext < n) {
-                        ri = (int)(uint32_t)rnext;
-                        const float4 ra = rays[2 * rnext], rb4 = rays[2 * rnext + 1];
+                        ri = (int)(gather ? perm[rnext] : (uint32_t)rnext);
+                        const float4 ra = rays[2 * (uint64_t)(uint32_t)ri], rb4 = rays[2 * (uint64_t)(uint32_t)ri + 1];
                         r.P[0] = ra.x; r.P[1] = ra.y; r.P[2] = ra.z; r.tclosest = ra.w;
                         const float D[3] = {rb4.x, rb4.y, rb4.z};
                         r.time = rb4.w;
-                        ray_setup(r, D);
-                        kp = pack_perm(r);
-                        ok = ray_plain<MOTION>(r);
+                        // A ray with tmax < 0 (the shading passes' unused shadow slots) culls every entry, since
+                        // no entry distance is below 0: a miss that needs no set-up and no step.
+                        const bool ends = !COUNTERS && ra.w < 0.0f;
+                        if (!ends) {
+                            ray_setup(r, D);
+                            kp = pack_perm(r);
+                            ok = ray_plain<MOTION>(r);
+                        }
                         nodesT = 0; leafsT = 0; trisT = 0; maxDepth = 0;
                         best_geom = -1; best_prim = -1;
                         if (XFORM) best_leaf = -1;
@@ -667,7 +677,7 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
                         in_mesh = false;
                         base = bottom;
                         sp = bottom;
-                        cur = 0;   // the root, whose entry distance is tclosest itself: never culled
+                        cur = ends ? kIdle : 0;   // the root, whose entry distance is tclosest itself: never culled
                     }
                 }
             }
@@ -900,8 +910,10 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     SceneView sv, const float4 *__restrict__ rays, uint64_t n, int4 *__restrict__ hits,                       \
         int32_t *__restrict__ geoms_out, int4 *__restrict__ counters, float *__restrict__ spT,                \
         int32_t *__restrict__ spN, int32_t *__restrict__ err, const uint32_t *__restrict__ n_dev,              \
-        const uint32_t *__restrict__ perm, int refill_min
-#define VGPU_TRACE_ARGS sv, rays, n, hits, geoms_out, counters, spT, spN, err, n_dev, perm, refill_min
+        const uint32_t *__restrict__ perm, int gather, int ray_shift,           \
+        int refill_min
+#define VGPU_TRACE_ARGS \
+    sv, rays, n, hits, geoms_out, counters, spT, spN, err, n_dev, perm, gather, ray_shift, refill_min
 
 template <int BLOCK, int LDS, bool SHADOW, bool MOTION, bool COUNTERS, bool EXT>
 __global__ __launch_bounds__(BLOCK) void k_trace_wide(VGPU_TRACE_PARAMS) {
@@ -932,54 +944,54 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
 template <bool SHADOW, bool EXT>
 hipError_t launch_xform(const SceneView& sv, const TraceLaunch& cfg, const void* rays, uint64_t n, void* hits,
                         int32_t* geoms, float* spT, int32_t* spN, uint64_t spill_threads, int32_t* err, int num_cus,
-                        const uint32_t* n_dev, const uint32_t* perm, hipStream_t stream) {
+                        const uint32_t* n_dev, const uint32_t* perm, bool gather, hipStream_t stream) {
     constexpr int kB = kXformLaunch.block, kL = kXformLaunch.lds_depth;
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
     if (cfg.block != kB || cfg.lds_depth != kL || threads > spill_threads) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_trace_xform<kB, kL, SHADOW, EXT>), dim3((unsigned)(threads / kB)), dim3(kB), 0, stream, sv,
                        (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err, n_dev, perm,
-                       cfg.refill_min);
+                       gather ? 1 : 0, trace_ray_shift(cfg, n, num_cus), cfg.refill_min);
     return hipGetLastError();
 }
 
 template <int BLOCK, int LDS, bool SHADOW, bool MOTION>
 hipError_t launch_cfg(const SceneView& sv, const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,
                       float* spT, int32_t* spN, uint64_t grid, int32_t* err, const uint32_t* n_dev,
-                      const uint32_t* perm, hipStream_t stream, int refill_min) {
+                      const uint32_t* perm, bool gather, hipStream_t stream, int ray_shift, int refill_min) {
     if constexpr (MOTION && LDS <= 12) {
         if (counters)
             hipLaunchKernelGGL((k_trace_wide_m5<BLOCK, LDS, SHADOW, true, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
                                stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)counters, spT, spN, err,
-                               n_dev, perm, refill_min);
+                               n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
         else
             hipLaunchKernelGGL((k_trace_wide_m5<BLOCK, LDS, SHADOW, false, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
                                stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err,
-                               n_dev, perm, refill_min);
+                               n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
         return hipGetLastError();
     }
     if (counters)
         hipLaunchKernelGGL((k_trace_wide<BLOCK, LDS, SHADOW, MOTION, true, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
                            stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)counters, spT, spN, err,
-                           n_dev, perm, refill_min);
+                           n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
     else
         hipLaunchKernelGGL((k_trace_wide<BLOCK, LDS, SHADOW, MOTION, false, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
                            stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err,
-                           n_dev, perm, refill_min);
+                           n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
     return hipGetLastError();
 }
 
 template <int BLOCK, int LDS>
 hipError_t launch_mode(const SceneView& sv, bool shadow, bool motion, const void* rays, uint64_t n, void* hits,
                        int32_t* geoms, int32_t* counters, float* spT, int32_t* spN, uint64_t grid, int32_t* err,
-                       const uint32_t* n_dev, const uint32_t* perm, hipStream_t stream, int refill_min) {
+                       const uint32_t* n_dev, const uint32_t* perm, bool gather, hipStream_t stream, int ray_shift, int refill_min) {
     if (shadow) {
         if (motion)
-            return launch_cfg<BLOCK, LDS, true, true>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, stream, refill_min);
-        return launch_cfg<BLOCK, LDS, true, false>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, stream, refill_min);
+            return launch_cfg<BLOCK, LDS, true, true>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, gather, stream, ray_shift, refill_min);
+        return launch_cfg<BLOCK, LDS, true, false>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, gather, stream, ray_shift, refill_min);
     }
     if (motion)
-        return launch_cfg<BLOCK, LDS, false, true>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, stream, refill_min);
-    return launch_cfg<BLOCK, LDS, false, false>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, stream, refill_min);
+        return launch_cfg<BLOCK, LDS, false, true>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, gather, stream, ray_shift, refill_min);
+    return launch_cfg<BLOCK, LDS, false, false>(sv, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, gather, stream, ray_shift, refill_min);
 }
 
 }  // namespace
@@ -994,26 +1006,35 @@ hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, 
     constexpr int kBM = kExtLaunchMotion.block, kLM = kExtLaunchMotion.lds_depth;
     if (sv.any_xform)
         return launch_xform<false, true>(sv, kXformLaunch, rays, n, hits32, nullptr, spT, spN, spill_threads, err, num_cus,
-                                         n_dev, nullptr, stream);
+                                         n_dev, nullptr, false, stream);
     const TraceLaunch cfg = motion ? kExtLaunchMotion : kExtLaunch;
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
     if (threads > spill_threads) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(threads / cfg.block);
+    const int ray_shift = trace_ray_shift(cfg, n, num_cus);
     if (motion)
         hipLaunchKernelGGL((k_trace_wide<kBM, kLM, false, true, false, true>), dim3(grid), dim3(kBM), 0, stream, sv,
                            (const float4*)rays, n, (int4*)hits32, (int32_t*)nullptr, (int4*)nullptr, spT, spN, err, n_dev,
-                           (const uint32_t*)nullptr, kRefillDefault);
+                           (const uint32_t*)nullptr, 0, ray_shift, kRefillDefault);
     else
         hipLaunchKernelGGL((k_trace_wide<kB, kL, false, false, false, true>), dim3(grid), dim3(kB), 0, stream, sv,
                            (const float4*)rays, n, (int4*)hits32, (int32_t*)nullptr, (int4*)nullptr, spT, spN, err, n_dev,
-                           (const uint32_t*)nullptr, kRefillDefault);
+                           (const uint32_t*)nullptr, 0, ray_shift, kRefillDefault);
     return hipGetLastError();
+}
+
+int trace_ray_shift(const TraceLaunch& cfg, uint64_t n, int num_cus) {
+    const uint64_t waves = (uint64_t)num_cus * (uint64_t)std::min(cfg.waves_per_cu, cfg.spread);
+    int shift = 6;
+    while (shift > 0 && (n >> (shift - 1)) < waves) shift--;
+    return shift;
 }
 
 uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus) {
     const uint64_t resident = (uint64_t)num_cus * (uint64_t)cfg.waves_per_cu * 64ull;
     uint64_t blocks = (resident + cfg.block - 1) / cfg.block;
-    const uint64_t need = (n + cfg.block - 1) / cfg.block;
+    const uint64_t per = (uint64_t)(cfg.block / 64) << trace_ray_shift(cfg, n, num_cus);   // rays per block and round
+    const uint64_t need = (n + per - 1) / per;
     if (blocks > need) blocks = need;
     if (blocks < 1) blocks = 1;
     return blocks * (uint64_t)cfg.block;
@@ -1021,23 +1042,24 @@ uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus) {
 
 hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg, const void* rays, uint64_t n,
                         void* hits, int32_t* geoms, int32_t* counters, float* spT, int32_t* spN, uint64_t spill_threads,
-                        int32_t* err, int num_cus, hipStream_t stream, const uint32_t* n_dev, const uint32_t* perm) {
+                        int32_t* err, int num_cus, hipStream_t stream, const uint32_t* n_dev, const uint32_t* perm, bool gather) {
     if (n == 0) return hipSuccess;
     if (n > 0xffffffffull) return hipErrorInvalidValue;
     if (sv.any_xform) {   // no counters
         if (counters) return hipErrorInvalidValue;
         return shadow ? launch_xform<true, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
-                                                  n_dev, perm, stream)
+                                                  n_dev, perm, gather, stream)
                       : launch_xform<false, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
-                                                   n_dev, perm, stream);
+                                                   n_dev, perm, gather, stream);
     }
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
     if (threads > spill_threads) return hipErrorInvalidValue;
     const uint64_t grid = threads / cfg.block;
+    const int ray_shift = trace_ray_shift(cfg, n, num_cus);
 #define VGPU_CASE(B, L)                                                                                         \
     if (cfg.block == B && cfg.lds_depth == L)                                                                   \
         return launch_mode<B, L>(sv, shadow, motion, rays, n, hits, geoms, counters, spT, spN, grid, err, n_dev, perm, \
-                                 stream, cfg.refill_min);
+                                 gather, stream, ray_shift, cfg.refill_min);
     VGPU_CASE(64, 8) VGPU_CASE(64, 12) VGPU_CASE(64, 16) VGPU_CASE(64, 24) VGPU_CASE(64, 32)
     VGPU_CASE(128, 8) VGPU_CASE(128, 12) VGPU_CASE(128, 16) VGPU_CASE(128, 24) VGPU_CASE(128, 32)
     VGPU_CASE(256, 8) VGPU_CASE(256, 12) VGPU_CASE(256, 16) VGPU_CASE(256, 24) VGPU_CASE(256, 32)
@@ -1105,7 +1127,7 @@ hipError_t launch_trace_noalloc(int device, const SceneView& sv, bool shadow, bo
     float* spT = (float*)(base + 256);
     int32_t* spN = (int32_t*)(base + 256 + per * threads * sizeof(float));
     return launch_trace(sv, shadow, motion, cfg, rays, n, hits, geoms, counters, spT, spN, threads, flag, num_cus,
-                        stream, nullptr, nullptr);
+                        stream, nullptr, nullptr, false);
 }
 
 }  // namespace vgpu

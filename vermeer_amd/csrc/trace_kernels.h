@@ -114,6 +114,7 @@ struct TraceLaunch {
     int lds_depth;      // 8, 12, 16, 24, 32
     int waves_per_cu;   // resident waves per CU used to size the grid
     int refill_min = kRefillDefault;   // idle lanes that make a wavefront take new rays together (1..64)
+    int spread = 16;    // waves per CU that a short launch is spread over (trace_ray_shift)
 };
 
 // Launch shapes of launch_trace_ext (the shading passes' closest-hit traversal) for static and
@@ -125,7 +126,7 @@ constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 
 // Launch shape of the traversals of a scene with transforms (block and LDS depth are its kernel's): the
 // scene's refill threshold in that shape.
-constexpr TraceLaunch kXformLaunch{64, 12, 16};
+constexpr TraceLaunch kXformLaunch{64, 12, 16, kRefillDefault, 8};   // spread: 50,000 rays take 368 us over 8, 442 over 16
 static_assert(kXformLaunch.waves_per_cu <= kExtLaunch.waves_per_cu && kXformLaunch.waves_per_cu <= kExtLaunchMotion.waves_per_cu,
               "the shading passes' spill areas cover it");
 inline TraceLaunch scene_launch(const SceneView& sv, const TraceLaunch& cfg) {
@@ -155,13 +156,14 @@ hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_
 // hold (VGPU_MAX_STACK - lds_depth) entries per launched thread; the launch
 // uses at most spill_threads threads.  n_dev (nullable): a device-resident
 // ray count; the kernel traces min(n, *n_dev) rays (n sizes the grid).  perm (nullable):
-// ray i's results go to slot perm[i] (rays reordered by launch_ray_sort).  cfg: a scene_launch shape.
+// ray i's results go to slot perm[i] (rays reordered by launch_ray_sort); with gather, ray i is the one
+// at slot perm[i] and its results go there (a list of the slots to trace).  cfg: a scene_launch shape.
 // Returns hipSuccess or the launch error.
 hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg,
                         const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,
                         float* spill_T, int32_t* spill_N, uint64_t spill_threads, int32_t* err_flag,
                         int num_cus, hipStream_t stream, const uint32_t* n_dev = nullptr,
-                        const uint32_t* perm = nullptr);
+                        const uint32_t* perm = nullptr, bool gather = false);
 
 // Closest hit with 32-byte records {prim, geom, t, U, V, W, 0, 0} (U, V, W: barycentric weights of the
 // triangle's three vertices), for the shading kernels.  Launch shape kExtLaunch, or kExtLaunchMotion
@@ -169,6 +171,12 @@ hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const Tra
 hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, uint64_t n, void* hits32, float* spill_T,
                             int32_t* spill_N, uint64_t spill_threads, int32_t* err_flag, int num_cus, hipStream_t stream,
                             const uint32_t* n_dev = nullptr);
+
+// Rays that a wavefront takes at a time, as a shift: 64, or fewer when that would leave wavefronts for fewer
+// than cfg.spread per CU.  A short launch lasts as long as its slowest wavefront, and one with fewer rays
+// diverges less, its idle lanes working in the leaf tests: 4096 pinhole rays over the sphere take 45 us
+// instead of 69, 50,000 bounce rays 63 instead of 75, 1024 rays among moving spheres 106 instead of 181.
+int trace_ray_shift(const TraceLaunch& cfg, uint64_t n, int num_cus);
 
 // Threads the launch above will use (so the caller can size the spill area).
 uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus);

@@ -46,6 +46,12 @@ __device__ __forceinline__ int hid_feature(int j, int g, int i) {
 // slots s = 4T + r (T = result tile, r = row in the lane's quad); slots 10, 11 are empty.
 __device__ __forceinline__ int out5_index(int g, int s) { return s < 10 ? 5 * (2 * g + s / 5) + s % 5 : -1; }
 
+// Encoded feature (canonical order: 24 d + 2 f, + 1 for the cosine) held in slot m = 8 j + i of lane group g for
+// k-chunk j of layer 1: group g takes frequencies 3 g .. 3 g + 2 of all six inputs, so a lane's 18 sine and
+// cosine pairs are its own and none is idle; -1: one of the 4 pads.
+constexpr int ENC_SLOTS = 36;
+__device__ __forceinline__ int enc_feature(int g, int m) { return m < ENC_SLOTS ? 24 * (m / 6) + 6 * g + m % 6 : -1; }
+
 __device__ __forceinline__ uint16_t bf16_bits(__bf16 b) { return __builtin_bit_cast(uint16_t, b); }
 __device__ __forceinline__ float bf16_val(__bf16 b) { return (float)b; }
 
@@ -64,8 +70,8 @@ __device__ __forceinline__ bf16x8 frag(const u32x4* s, int f, int lane) {
 __device__ int pack_fwd_index(int f, int lane, int i) {
     const int r = lane & 15, g = lane >> 4;
     if (f < F_L2) {
-        const int o = f / 5, j = f % 5, q = 32 * j + 8 * g + i;
-        return q < NENC ? OW1 + (16 * o + r) * NENC + q : -1;
+        const int o = f / 5, j = f % 5, q = enc_feature(g, 8 * j + i);
+        return q >= 0 ? OW1 + (16 * o + r) * NENC + q : -1;
     }
     if (f < F_L5) {
         const int l = (f - F_L2) / 8, ff = (f - F_L2) % 8, o = ff / 2, j = ff % 2;
@@ -130,31 +136,28 @@ __global__ void k_pack(const float* __restrict__ P, u32x4* __restrict__ ffwd, u3
 
 // ---------------------------------------------------------------- forward pieces
 
-__device__ __forceinline__ float sel6(const float x[6], int d) {
-    return d == 0 ? x[0] : d == 1 ? x[1] : d == 2 ? x[2] : d == 3 ? x[3] : d == 4 ? x[4] : x[5];
-}
-
-// Encoded features 32j + 8g .. +7 (canonical order: 24 d + 2 f (+1 for cos)).
-// sin(pi 2^f x) is evaluated on the exactly reduced argument r = 2^f x - 2 round(2^(f-1) x),
-// in revolutions (r / 2) for the hardware sine.
-__device__ __forceinline__ bf16x8 enc_chunk(const float x[6], int j, int g) {
-    bf16x8 b;
-    const int q0 = 32 * j + 8 * g;
-    if (q0 >= NENC) {
-        for (int i = 0; i < 8; i++) b[i] = (__bf16)0.0f;
-        return b;
-    }
-    const int d = q0 / 24, f0 = (q0 % 24) / 2;
-    const float xd = sel6(x, d);
+// A lane's encoded features in slot order.  sin and cos of pi 2^f x are taken on the exactly reduced argument in
+// revolutions, u - round(u) with u = 2^(f - 1) x.  The lane group sets the frequencies and not the input, so no
+// lane selects its input or skips a chunk.  (Double angles for two of the three octaves saved 1% of 1M queries
+// and moved four times as many activations by a bf16 step.)
+__device__ __forceinline__ void encode(const float x[6], int g, bf16x8 (&e)[5]) {
+    const float scale = __int_as_float((126 + 3 * g) << 23);   // 2^(3 g - 1)
+    float v[40];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float t = ldexpf(xd, f0 + k);
-        const float r = t - 2.0f * rintf(0.5f * t);
-        const float rev = 0.5f * r;
-        b[2 * k] = (__bf16)__builtin_amdgcn_sinf(rev);
-        b[2 * k + 1] = (__bf16)__builtin_amdgcn_cosf(rev);
-    }
-    return b;
+    for (int d = 0; d < 6; d++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const float u = x[d] * (scale * (float)(1 << k));
+            const float r = u - rintf(u);
+            v[6 * d + 2 * k] = __builtin_amdgcn_sinf(r);
+            v[6 * d + 2 * k + 1] = __builtin_amdgcn_cosf(r);
+        }
+#pragma unroll
+    for (int m = ENC_SLOTS; m < 40; m++) v[m] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 5; j++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) e[j][i] = (__bf16)v[8 * j + i];
 }
 
 __device__ __forceinline__ void normalise(const float4& p, const float4& n, const float* bounds, float x[6]) {
@@ -167,17 +170,29 @@ __device__ __forceinline__ void normalise(const float4& p, const float4& n, cons
     x[3] = n.x; x[4] = n.y; x[5] = n.z;
 }
 
+// The biases in LDS: 64 per hidden layer, then the output layer's in the lanes' slot order (12 per lane group).
+constexpr int BIAS_OUT = 4 * NH, BIAS_WORDS = BIAS_OUT + 4 * 12;
+__device__ __forceinline__ float bias_word(const float* P, int w) {
+    if (w < BIAS_OUT) {
+        const int l = w / NH, ob = l == 0 ? OB1 : (l == 1 ? OB2 : (l == 2 ? OB3 : OB4));
+        return P[ob + w % NH];
+    }
+    const int out = out5_index((w - BIAS_OUT) / 12, (w - BIAS_OUT) % 12);
+    return out >= 0 ? P[OB5 + out] : 0.0f;
+}
+
 template <int NT>
 __device__ __forceinline__ void bias_hidden(f32x4 (&acc)[4][NT], const float* b, int g) {
 #pragma unroll
-    for (int o = 0; o < 4; o++)
+    for (int o = 0; o < 4; o++) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(b + 16 * o + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float v = b[16 * o + 4 * g + r];
-#pragma unroll
-            for (int t = 0; t < NT; t++) acc[o][t][r] = v;
-        }
+        for (int t = 0; t < NT; t++) acc[o][t] = v;
+    }
 }
+
+// max(v, 0), 0 for a NaN.
+__device__ __forceinline__ float relu(float v) { return fmaxf(v, 0.0f); }
 
 template <int NT>
 __device__ __forceinline__ void relu_pack(const f32x4 (&acc)[4][NT], bf16x8 (&X)[2][NT]) {
@@ -188,7 +203,7 @@ __device__ __forceinline__ void relu_pack(const f32x4 (&acc)[4][NT], bf16x8 (&X)
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float v = acc[2 * j + (i >> 2)][t][i & 3];
-                X[j][t][i] = (__bf16)(v > 0.0f ? v : 0.0f);
+                X[j][t][i] = (__bf16)relu(v);
             }
 }
 
@@ -210,32 +225,28 @@ template <int NT>
 __device__ __forceinline__ void layer_first(const u32x4* sF, const float* bias, int g, int lane, const float (&x)[NT][6],
                                             f32x4 (&acc)[4][NT]) {
     bias_hidden<NT>(acc, bias, g);
+    bf16x8 b[NT][5];
 #pragma unroll
-    for (int j = 0; j < 5; j++) {
-        bf16x8 b[NT];
+    for (int t = 0; t < NT; t++) encode(x[t], g, b[t]);
 #pragma unroll
-        for (int t = 0; t < NT; t++) b[t] = enc_chunk(x[t], j, g);
+    for (int j = 0; j < 5; j++)
 #pragma unroll
         for (int o = 0; o < 4; o++) {
             const bf16x8 a = frag(sF, F_L1 + 5 * o + j, lane);
 #pragma unroll
-            for (int t = 0; t < NT; t++) acc[o][t] = mfma(a, b[t], acc[o][t]);
+            for (int t = 0; t < NT; t++) acc[o][t] = mfma(a, b[t][j], acc[o][t]);
         }
-    }
 }
 
 template <int NT>
-__device__ __forceinline__ void layer_out(const u32x4* sF, const float* b5, int g, int lane, const bf16x8 (&Xin)[2][NT],
+__device__ __forceinline__ void layer_out(const u32x4* sF, const float* bias, int g, int lane, const bf16x8 (&Xin)[2][NT],
                                           f32x4 (&acc)[3][NT]) {
 #pragma unroll
-    for (int T = 0; T < 3; T++)
+    for (int T = 0; T < 3; T++) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(bias + BIAS_OUT + 12 * g + 4 * T);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int out = out5_index(g, 4 * T + r);
-            const float v = out >= 0 ? b5[out] : 0.0f;
-#pragma unroll
-            for (int t = 0; t < NT; t++) acc[T][t][r] = v;
-        }
+        for (int t = 0; t < NT; t++) acc[T][t] = v;
+    }
 #pragma unroll
     for (int T = 0; T < 3; T++)
 #pragma unroll
@@ -253,20 +264,6 @@ struct LobeD {
     bool kin;
 };
 
-__device__ __forceinline__ void decode_lobe(const float* v, LobeD& L) {
-    const float len = sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    L.ulen = len;
-    if (len > 0.0f) {
-        const float inv = 1.0f / len;
-        L.mu[0] = v[0] * inv; L.mu[1] = v[1] * inv; L.mu[2] = v[2] * inv;
-    } else {
-        L.mu[0] = 0.0f; L.mu[1] = 0.0f; L.mu[2] = 1.0f;
-    }
-    L.kin = v[3] > KAPPA_RAW_MIN && v[3] < KAPPA_RAW_MAX;
-    L.kappa = expf(fminf(fmaxf(v[3], KAPPA_RAW_MIN), KAPPA_RAW_MAX));
-    L.logit = v[4];
-}
-
 __device__ __forceinline__ float quad_max(float v) {
     v = fmaxf(v, __shfl_xor(v, 16));
     return fmaxf(v, __shfl_xor(v, 32));
@@ -274,6 +271,43 @@ __device__ __forceinline__ float quad_max(float v) {
 __device__ __forceinline__ float quad_sum(float v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
+}
+
+// exp(x) for |x| <= 80: x log2 e in two parts, the hardware exp2 on what is left beside the nearest whole number
+// (on the whole argument it was off by 1.3e-7 instead of 8.4e-8).
+__device__ __forceinline__ float exp_mid(float x) {
+    const float L = 1.44269504f, LL = 1.92596299e-8f;          // log2 e = L + LL
+    const float h = x * L, e = rintf(h);
+    const float l = __builtin_fmaf(x, LL, __builtin_fmaf(x, L, -h));
+    return __builtin_ldexpf(__builtin_amdgcn_exp2f((h - e) + l), (int)e);
+}
+
+// A lobe from its five outputs, for inference.  One Newton step on the hardware reciprocal square root stands
+// for a rounded square root and division; squares whose sum leaves the middle of the range take those.
+__device__ __forceinline__ void decode_lobe(const float* v, LobeD& L) {
+    const float q = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+    if (q > 0x1p-96f && q < 0x1p96f) {
+        float r = __builtin_amdgcn_rsqf(q);
+        r = __builtin_fmaf(0.5f * r, __builtin_fmaf(-(q * r), r, 1.0f), r);
+        L.mu[0] = v[0] * r; L.mu[1] = v[1] * r; L.mu[2] = v[2] * r;
+    } else {
+        const float len = sqrtf(q);
+        if (len > 0.0f) {
+            const float inv = 1.0f / len;
+            L.mu[0] = v[0] * inv; L.mu[1] = v[1] * inv; L.mu[2] = v[2] * inv;
+        } else {
+            L.mu[0] = 0.0f; L.mu[1] = 0.0f; L.mu[2] = 1.0f;
+        }
+    }
+    L.kappa = exp_mid(fminf(fmaxf(v[3], KAPPA_RAW_MIN), KAPPA_RAW_MAX));
+    L.logit = v[4];
+}
+// exp of a logit less the largest (never above 0; the rest, NaN too, by the library's function)
+__device__ __forceinline__ float exp_weight(float x) { return x >= -80.0f ? exp_mid(x) : expf(x); }
+// a / z rounded, from iz, the Newton-corrected reciprocal of z
+__device__ __forceinline__ float div_by(float a, float z, float iz) {
+    const float w = a * iz;
+    return __builtin_fmaf(__builtin_fmaf(-z, w, a), iz, w);
 }
 
 // decode_lobe, log_vmf_norm and dlog_norm for the training kernel's loss gradient, on the hardware
@@ -299,32 +333,51 @@ __device__ __forceinline__ float dlog_norm_fast(float k) {
     if (k < 0.05f) return 1.0f - k * (1.0f / 3.0f) + k * k * k * (1.0f / 45.0f);
     return __builtin_amdgcn_rcpf(k) - 2.0f * __builtin_amdgcn_rcpf(expm1f(2.0f * k));
 }
-// log of the vMF normalisation kappa / (2 pi (1 - exp(-2 kappa)))
-__device__ __forceinline__ float log_vmf_norm(float k) {
-    return logf(k) - 1.8378770664093453f - logf(-expm1f(-2.0f * k));
-}
-
-// 1/kappa - 2/(exp(2 kappa) - 1), with its series below 0.05
-__device__ __forceinline__ float dlog_norm(float k) {
-    if (k < 0.05f) return 1.0f - k * (1.0f / 3.0f) + k * k * k * (1.0f / 45.0f);
-    return 1.0f / k - 2.0f / expm1f(2.0f * k);
-}
-
 // ---------------------------------------------------------------- inference
 
+// 1M queries: 87 us of kernel (119 before): every lane has its own encoded features (encode), the biases lie in
+// LDS, the decode needs no full division, square root or exp, and the next queries are fetched ahead.  Two tiles
+// per wave: three and four were no faster.
+// Three waves per SIMD, as the LDS allows; said to the compiler, it also keeps the accumulators in VGPRs (with
+// room for 512 registers it moved every result through an AGPR, 130 of 667 VALU instructions per iteration).
 template <bool RAW>
-__global__ __launch_bounds__(256) void k_infer(Net net, const float4* __restrict__ q, uint64_t n,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_infer(Net net, const float4* __restrict__ q, uint64_t n,
                                                const uint32_t* __restrict__ n_dev, float* __restrict__ out) {
     constexpr int NT = 2;   // 16-query tiles per wave and iteration: 2 keeps three waves per SIMD
     __shared__ u32x4 sF[NF_FWD * 64];
-    for (int k = threadIdx.x; k < NF_FWD * 64; k += 256) sF[k] = reinterpret_cast<const u32x4*>(net.frag_fwd)[k];
+    __shared__ __attribute__((aligned(16))) float sBias[BIAS_WORDS];
+    {
+        // every load issued before the first store: 256 queries took 11.7 us with one load in flight, 8.4 so (the whole step)
+        constexpr int NI = (NF_FWD * 64 + 255) / 256;
+        u32x4 fr[NI];
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+            fr[i] = reinterpret_cast<const u32x4*>(net.frag_fwd)[min((int)threadIdx.x + 256 * i, NF_FWD * 64 - 1)];
+        for (int w = threadIdx.x; w < BIAS_WORDS; w += 256) sBias[w] = bias_word(net.params, w);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int k = (int)threadIdx.x + 256 * i;
+            if (k < NF_FWD * 64) sF[k] = fr[i];
+        }
+    }
     __syncthreads();
     uint64_t nn = n;
     if (n_dev) nn = min(nn, (uint64_t)*n_dev);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
-    const uint64_t nw = (uint64_t)gridDim.x * 4;
-    const float* P = net.params;
-    for (uint64_t base = ((uint64_t)blockIdx.x * 4 + wave) * (16 * NT); base < nn; base += nw * (16 * NT)) {
+    const uint64_t step = (uint64_t)gridDim.x * 4 * (16 * NT);
+    uint64_t base = ((uint64_t)blockIdx.x * 4 + wave) * (16 * NT);
+    // the next iteration's queries are in flight while this one's are evaluated
+    float4 qp[NT], qn[NT];
+    auto fetch = [&](uint64_t first) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const uint64_t i = min(first + 16 * t + c, nn - 1);
+            qp[t] = q[2 * i];
+            qn[t] = q[2 * i + 1];
+        }
+    };
+    if (base < nn) fetch(base);
+    for (; base < nn; base += step) {
         // keeps the weight fragments' LDS reads inside the loop: hoisted, they would pin 200 registers
         __asm__ volatile("" ::: "memory");
         float x[NT][6];
@@ -332,24 +385,21 @@ __global__ __launch_bounds__(256) void k_infer(Net net, const float4* __restrict
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             s[t] = base + 16 * t + c;
-            if (s[t] < nn) {
-                normalise(q[2 * s[t]], q[2 * s[t] + 1], net.bounds, x[t]);
-            } else {
-                for (int k = 0; k < 6; k++) x[t][k] = 0.0f;
-            }
+            normalise(qp[t], qn[t], net.bounds, x[t]);
         }
+        fetch(base + step);
         f32x4 acc[4][NT];
         bf16x8 X[2][NT];
-        layer_first<NT>(sF, P + OB1, g, lane, x, acc);
+        layer_first<NT>(sF, sBias, g, lane, x, acc);
         relu_pack<NT>(acc, X);
-        layer_hidden<NT>(sF, F_L2, P + OB2, g, lane, X, acc);
+        layer_hidden<NT>(sF, F_L2, sBias + 1 * NH, g, lane, X, acc);
         relu_pack<NT>(acc, X);
-        layer_hidden<NT>(sF, F_L3, P + OB3, g, lane, X, acc);
+        layer_hidden<NT>(sF, F_L3, sBias + 2 * NH, g, lane, X, acc);
         relu_pack<NT>(acc, X);
-        layer_hidden<NT>(sF, F_L4, P + OB4, g, lane, X, acc);
+        layer_hidden<NT>(sF, F_L4, sBias + 3 * NH, g, lane, X, acc);
         relu_pack<NT>(acc, X);
         f32x4 o5[3][NT];
-        layer_out<NT>(sF, P + OB5, g, lane, X, o5);
+        layer_out<NT>(sF, sBias, g, lane, X, o5);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             float v[12];
@@ -365,12 +415,13 @@ __global__ __launch_bounds__(256) void k_infer(Net net, const float4* __restrict
                 decode_lobe(v, A);
                 decode_lobe(v + 5, B);
                 const float m = quad_max(fmaxf(A.logit, B.logit));
-                const float ea = expf(A.logit - m), eb = expf(B.logit - m);
-                const float z = quad_sum(ea + eb);
+                const float ea = exp_weight(A.logit - m), eb = exp_weight(B.logit - m);
+                const float z = quad_sum(ea + eb), rz = __builtin_amdgcn_rcpf(z);   // 1 <= z <= 8
+                const float iz = __builtin_fmaf(__builtin_fmaf(-z, rz, 1.0f), rz, rz);
                 if (s[t] < nn) {
                     float* o = out + s[t] * NOUT + 10 * g;
-                    o[0] = A.mu[0]; o[1] = A.mu[1]; o[2] = A.mu[2]; o[3] = A.kappa; o[4] = ea / z;
-                    o[5] = B.mu[0]; o[6] = B.mu[1]; o[7] = B.mu[2]; o[8] = B.kappa; o[9] = eb / z;
+                    o[0] = A.mu[0]; o[1] = A.mu[1]; o[2] = A.mu[2]; o[3] = A.kappa; o[4] = div_by(ea, z, iz);
+                    o[5] = B.mu[0]; o[6] = B.mu[1]; o[7] = B.mu[2]; o[8] = B.kappa; o[9] = div_by(eb, z, iz);
                 }
             }
         }
@@ -452,7 +503,7 @@ constexpr int STG = TRAIN_CHUNK + 8;           // staged row stride, bf16 (272 b
 constexpr size_t FWD_BYTES = (size_t)NF_FWD * 64 * 16, BWD_BYTES = (size_t)NF_BWD * 64 * 16;
 constexpr size_t STAGE_BYTES = (size_t)(NENC + NH) * STG * 2;   // X1 (144 rows) and dY1 (64 rows): the largest
 constexpr size_t SAMPLE_BYTES = (size_t)TRAIN_WG * sizeof(TrainSample);   // the workgroup's batch slots
-constexpr size_t TRAIN_LDS = FWD_BYTES + BWD_BYTES + STAGE_BYTES + SAMPLE_BYTES;
+constexpr size_t TRAIN_LDS = FWD_BYTES + BWD_BYTES + STAGE_BYTES + SAMPLE_BYTES + BIAS_WORDS * sizeof(float);
 static_assert(STAGE_BYTES % 16 == 0 && TRAIN_LDS <= 160 * 1024, "LDS layout");
 
 // Tiles of one layer's dW held by a wave: tiles wave, wave + 8, ... of NOR x NIT.
@@ -538,6 +589,9 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
     uint16_t* Xs = reinterpret_cast<uint16_t*>(lds + (FWD_BYTES + BWD_BYTES) / 16);
     uint16_t* Ys = Xs + NENC * STG;
     TrainSample* sS = reinterpret_cast<TrainSample*>(lds + (FWD_BYTES + BWD_BYTES + STAGE_BYTES) / 16);
+    float* sBias = reinterpret_cast<float*>(sS + TRAIN_WG);
+    // loaded with the fragments below and stored behind them: a store here would wait for its load first
+    const float bias = threadIdx.x < BIAS_WORDS ? bias_word(net.params, threadIdx.x) : 0.0f;
     {
         // the batch slots and both fragment sets (adjacent in LDS), every load issued before the
         // first store so that their latencies overlap
@@ -559,10 +613,10 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
             if (k < NFRAG) lds[k] = fr[i];
         }
     }
+    if (threadIdx.x < BIAS_WORDS) sBias[threadIdx.x] = bias;
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
     const int col = wave * 16 + c;                          // this lane's staged column
-    const float* P = net.params;
     if (wave == 0) {
         float a = 0.0f;
 #pragma unroll
@@ -592,16 +646,16 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
         }
         f32x4 acc[4][NT];
         bf16x8 X2[2][NT], X3[2][NT], X4[2][NT], X5[2][NT];
-        layer_first<NT>(sF, P + OB1, g, lane, x, acc);
+        layer_first<NT>(sF, sBias, g, lane, x, acc);
         relu_pack<NT>(acc, X2);
-        layer_hidden<NT>(sF, F_L2, P + OB2, g, lane, X2, acc);
+        layer_hidden<NT>(sF, F_L2, sBias + 1 * NH, g, lane, X2, acc);
         relu_pack<NT>(acc, X3);
-        layer_hidden<NT>(sF, F_L3, P + OB3, g, lane, X3, acc);
+        layer_hidden<NT>(sF, F_L3, sBias + 2 * NH, g, lane, X3, acc);
         relu_pack<NT>(acc, X4);
-        layer_hidden<NT>(sF, F_L4, P + OB4, g, lane, X4, acc);
+        layer_hidden<NT>(sF, F_L4, sBias + 3 * NH, g, lane, X4, acc);
         relu_pack<NT>(acc, X5);
         f32x4 o5[3][NT];
-        layer_out<NT>(sF, P + OB5, g, lane, X5, o5);
+        layer_out<NT>(sF, sBias, g, lane, X5, o5);
 
         // loss gradient d(-(c/cbar) log q)/d raw for this lane's two lobes, staged as dY5 rows (out5_index)
         bf16x8 G5[2][NT];
@@ -682,14 +736,11 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
         dw_chunk(Xs, Ys, T2, bs2, NH);
         __syncthreads();
         // layer 1: its input is the encoding, recomputed (the forward pass keeps it in no register)
+        {
+            bf16x8 e[5];
+            encode(x[0], g, e);
 #pragma unroll
-        for (int j = 0; j < 5; j++) {
-            const int q0 = 32 * j + 8 * g;
-            if (q0 < NENC) {
-                const bf16x8 b = enc_chunk(x[0], j, g);
-#pragma unroll
-                for (int i = 0; i < 8; i++) Xs[(q0 + i) * STG + col] = bf16_bits(b[i]);
-            }
+            for (int m = 0; m < ENC_SLOTS; m++) Xs[enc_feature(g, m) * STG + col] = bf16_bits(e[m / 8][m % 8]);
         }
         stage_hidden(Ys, D, g, col);
         __syncthreads();
@@ -804,7 +855,7 @@ hipError_t launch_pack(const float* params, uint4* ffwd, uint4* fbwd, hipStream_
 hipError_t launch_infer(const Net& net, const float4* queries, uint64_t n, const uint32_t* n_dev, float* out, bool raw,
                         int num_cus, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    uint64_t blocks = (n + 255) / 256;
+    uint64_t blocks = (n + 127) / 128;   // 32 queries per wave and iteration
     const uint64_t cap = (uint64_t)num_cus * 3;
     if (blocks > cap) blocks = cap;
     if (raw)

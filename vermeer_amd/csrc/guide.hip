@@ -310,7 +310,7 @@ __device__ __forceinline__ float div_by(float a, float z, float iz) {
     return __builtin_fmaf(__builtin_fmaf(-z, w, a), iz, w);
 }
 
-// decode_lobe, log_vmf_norm and dlog_norm for the training kernel's loss gradient, on the hardware
+// The lobe decode, the vMF normalisation and its derivative for the training kernel's loss gradient, on the hardware
 // exp2 / log2 / reciprocal / square-root approximations (about 1 ulp; the gradient is compared
 // with the FP64 oracle at a relative tolerance far above that).
 __device__ __forceinline__ void decode_lobe_fast(const float* v, LobeD& L) {

@@ -169,8 +169,8 @@ int vgpu_pt_create(vgpu_pt** out, vgpu_scene* s, const vgpu_pt_material* materia
     b.rec = nullptr;
     b.plen = nullptr;
     vgpu::TraceLaunch cfg{s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu};
-    const int rc = ensure_spill(s, std::max(vgpu::trace_grid_threads(vgpu::scene_launch(s->view, cfg), np, s->num_cus),
-                                            vgpu::trace_grid_threads(vgpu::kExtLaunch, np, s->num_cus)));
+    const int rc = ensure_spill(s, std::max(vgpu::trace_spill_columns(vgpu::scene_launch(s->view, cfg), np, s->num_cus),
+                                            vgpu::trace_spill_columns(vgpu::kExtLaunch, np, s->num_cus)));
     if (rc) { delete pt; return rc; }
     *out = pt;
     return VGPU_OK;
@@ -267,7 +267,7 @@ int vgpu_pt_pass(vgpu_pt* pt, uint32_t flags, uint32_t pass, double* accum, void
                 HIP_TRY(hipEventRecord(ev[0], st));
                 HIP_TRY(hipEventRecord(ev[1], st));
             }
-            e = vgpu::launch_trace_ext(s->view, false, bb.qray[cur], np, bb.hits, s->d_spT, s->d_spN, s->spill_threads,
+            e = vgpu::launch_trace_ext(s->view, false, bb.qray[cur], np, bb.hits, s->d_spT, s->d_spN, s->spill_columns,
                                        s->d_err, s->num_cus, st, bb.count + cur);
             if (ev[2] && e == hipSuccess) HIP_TRY(hipEventRecord(ev[2], st));
             if (e == hipSuccess) { stage = "hit"; e = vgpu::pt_launch_hit(v, pass, cur, bb, st); }

@@ -462,8 +462,8 @@ int vgpu_render_create(vgpu_render** out, vgpu_scene* s, const vgpu_material* ma
     // size the traversal spill area for the larger (shadow) launch
     vgpu::TraceLaunch L{s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu};
     const vgpu::TraceLaunch ext = s->any_motion ? vgpu::kExtLaunchMotion : vgpu::kExtLaunch;
-    int rc = ensure_spill(s, std::max(vgpu::trace_grid_threads(vgpu::scene_launch(s->view, L), ns, s->num_cus),
-                                      vgpu::trace_grid_threads(ext, np, s->num_cus)));
+    int rc = ensure_spill(s, std::max(vgpu::trace_spill_columns(vgpu::scene_launch(s->view, L), ns, s->num_cus),
+                                      vgpu::trace_spill_columns(ext, np, s->num_cus)));
     if (rc) { delete r; return rc; }
     *out = r;
     return VGPU_OK;
@@ -513,7 +513,7 @@ int vgpu_render_pass(vgpu_render* r, uint32_t flags, const uint64_t* scrambles, 
         for (int level = 0; level <= r->rv.max_level; level++) {
             float4* rin = (level & 1) ? r->d_rays2 : r->d_rays;
             float4* rout = level < r->rv.max_level ? ((level & 1) ? r->d_rays : r->d_rays2) : nullptr;
-            e = vgpu::launch_trace_ext(s->view, s->any_motion, rin, np, r->d_hits32, s->d_spT, s->d_spN, s->spill_threads, s->d_err,
+            e = vgpu::launch_trace_ext(s->view, s->any_motion, rin, np, r->d_hits32, s->d_spT, s->d_spN, s->spill_columns, s->d_err,
                                        s->num_cus, st);
             if (e != hipSuccess) return fail(VGPU_ERR_HIP, "closest hit: %s", hipGetErrorString(e));
             e = vgpu::launch_shade(r->rv, d_scr, iter, level, rin, r->d_hits32, r->d_pix, r->d_slot_rays, r->d_slot_rgb,

@@ -269,15 +269,15 @@ int upload(T** dptr, const std::vector<T>& v) {
     return VGPU_OK;
 }
 
-int ensure_spill(vgpu_scene* s, uint64_t threads) {
-    if (s->d_spT && s->spill_threads >= threads) return VGPU_OK;
+int ensure_spill(vgpu_scene* s, uint64_t columns) {
+    if (s->d_spT && s->spill_columns >= columns) return VGPU_OK;
     if (s->d_spT) { HIP_TRY(hipFree(s->d_spT)); s->d_spT = nullptr; }
     if (s->d_spN) { HIP_TRY(hipFree(s->d_spN)); s->d_spN = nullptr; }
     // size for the smallest LDS depth so later configuration changes never need more
     const uint64_t per = (uint64_t)(VGPU_MAX_STACK - 8);
-    HIP_TRY(hipMalloc((void**)&s->d_spT, per * threads * sizeof(float)));
-    HIP_TRY(hipMalloc((void**)&s->d_spN, per * threads * sizeof(int32_t)));
-    s->spill_threads = threads;
+    HIP_TRY(hipMalloc((void**)&s->d_spT, per * columns * sizeof(float)));
+    HIP_TRY(hipMalloc((void**)&s->d_spN, per * columns * sizeof(int32_t)));
+    s->spill_columns = columns;
     return VGPU_OK;
 }
 
@@ -361,8 +361,7 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
         return fail(VGPU_ERR_ARG, "per-ray counters are not kept for scenes with instances, procs or mesh transforms");
     const vgpu::TraceLaunch L = vgpu::scene_launch(
         s->view, {cfg.block, cfg.lds_stack, cfg.waves_per_cu, cfg.refill > 0 ? cfg.refill : vgpu::kRefillDefault});
-    const uint64_t threads = vgpu::trace_grid_threads(L, n, s->num_cus);
-    int rc = ensure_spill(s, threads);
+    int rc = ensure_spill(s, vgpu::trace_spill_columns(L, n, s->num_cus));
     if (rc) return rc;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     if (s->timing && n > 0) {
@@ -381,7 +380,7 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
     }
     if (ev[1]) HIP_TRY(hipEventRecord(ev[1], st));
     hipError_t e = vgpu::launch_trace(s->view, (flags & VGPU_TRACE_SHADOW) != 0, s->any_motion, L, d_rays, n, d_hits,
-                                      d_geoms, d_counters, s->d_spT, s->d_spN, s->spill_threads, s->d_err, s->num_cus, st,
+                                      d_geoms, d_counters, s->d_spT, s->d_spN, s->spill_columns, s->d_err, s->num_cus, st,
                                       n_dev, perm, list != nullptr);
     if (e != hipSuccess) return fail(VGPU_ERR_HIP, "trace launch: %s", hipGetErrorString(e));
     if (ev[2]) HIP_TRY(hipEventRecord(ev[2], st));
@@ -1104,9 +1103,9 @@ int vgpu_trace_noalloc(vgpu_scene* s, uint32_t flags, const vgpu_ray* d_rays, ui
     // scratch array; never sorted (the sort's buffers grow with n).
     vgpu::TraceLaunch L = vgpu::scene_launch(s->view, {s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu,
                                                        s->cfg.refill > 0 ? s->cfg.refill : vgpu::kRefillDefault});
-    const uint64_t cap = vgpu::noalloc_max_threads(L.lds_depth);
-    while (L.waves_per_cu > 1 && vgpu::trace_grid_threads(L, n, s->num_cus) > cap) L.waves_per_cu--;
-    if (vgpu::trace_grid_threads(L, n, s->num_cus) > cap)
+    const uint64_t cap = vgpu::noalloc_max_columns(L.lds_depth);
+    while (L.waves_per_cu > 1 && vgpu::trace_spill_columns(L, n, s->num_cus) > cap) L.waves_per_cu--;
+    if (vgpu::trace_spill_columns(L, n, s->num_cus) > cap)
         return fail(VGPU_ERR_ARG, "the %llu-byte scratch holds the stack spill of fewer than one wavefront per CU on %d CUs",
                     (unsigned long long)vgpu::kNoAllocScratchBytes, s->num_cus);
     const hipError_t e = vgpu::launch_trace_noalloc(s->device, s->view, (flags & VGPU_TRACE_SHADOW) != 0, s->any_motion, L,

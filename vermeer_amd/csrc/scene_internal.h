@@ -120,7 +120,7 @@ struct vgpu_scene {
     int32_t* d_err = nullptr;
     float* d_spT = nullptr;
     int32_t* d_spN = nullptr;
-    uint64_t spill_threads = 0;
+    uint64_t spill_columns = 0;
     void* d_stage = nullptr;
     size_t stage_bytes = 0;
     vgpu::SceneView view{};
@@ -172,7 +172,7 @@ struct DeviceGuard {
 hipEvent_t timing_event(vgpu_scene* s);
 
 // Ensures the spill area covers `threads` traversal threads.
-int ensure_spill(vgpu_scene* s, uint64_t threads);
+int ensure_spill(vgpu_scene* s, uint64_t columns);
 // Host math of the camera (render.cpp), in the reference's float32 operation order.
 void vec3_normalize(const float* a, float* out);
 void vec3_cross(const float* a, const float* b, float* o);

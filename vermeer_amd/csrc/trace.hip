@@ -587,12 +587,16 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     __shared__ int owner[BLOCK];                  // written by one lane, read by another of its wavefront
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const uint64_t gtid = (uint64_t)blockIdx.x * BLOCK + tid;
-    const uint64_t nthr = (uint64_t)gridDim.x * BLOCK;
-    const uint64_t nwaves = nthr / 64;
+    const uint64_t nwaves = (uint64_t)gridDim.x * (BLOCK / 64);
+    const uint64_t wave = (uint64_t)blockIdx.x * (BLOCK / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     const int bottom = tid * 8;                   // the lane's empty stack: entry i at bottom + i * kEntry
 
-    auto spill = [&](int sp) { return (uint64_t)((uint32_t)sp / kEntry - LDS) * nthr + (uint32_t)gtid; };
+    // A spill column per lane that can own a ray: with ray_shift below 6 the wavefront takes all its rays at once,
+    // into its first 2^ray_shift lanes (trace_spill_columns).
+    auto spill = [&](int sp) {
+        return (uint64_t)((uint32_t)sp / kEntry - LDS) * (nwaves << ray_shift) + (wave << ray_shift) +
+               (uint32_t)(lane & ((1 << ray_shift) - 1));
+    };
     auto push = [&](int sp, float T, int32_t node) {
         if (sp < LDS * kEntry) *reinterpret_cast<uint2*>(reinterpret_cast<char*>(stack_lds) + sp) = make_uint2(__float_as_uint(T), (uint32_t)node);
         else { const uint64_t o = spill(sp); spT[o] = T; spN[o] = node; }
@@ -601,7 +605,6 @@ __device__ __forceinline__ void trace_wide(SceneView sv, const float4* __restric
     if (n_dev) n = min(n, (uint64_t)*n_dev);
     // Rays of this wavefront: v = 0, 1, 2, ... -> ray_of(v), increasing in v: 2^ray_shift consecutive rays, then
     // as many nwaves * 2^ray_shift further on (trace_ray_shift).
-    const uint64_t wave = (uint64_t)blockIdx.x * (BLOCK / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     auto ray_of = [&](uint32_t v) {
         return (((uint64_t)(v >> ray_shift) * nwaves + wave) << ray_shift) + (v & ((1u << ray_shift) - 1u));
     };
@@ -943,11 +946,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
 
 template <bool SHADOW, bool EXT>
 hipError_t launch_xform(const SceneView& sv, const TraceLaunch& cfg, const void* rays, uint64_t n, void* hits,
-                        int32_t* geoms, float* spT, int32_t* spN, uint64_t spill_threads, int32_t* err, int num_cus,
+                        int32_t* geoms, float* spT, int32_t* spN, uint64_t spill_columns, int32_t* err, int num_cus,
                         const uint32_t* n_dev, const uint32_t* perm, bool gather, hipStream_t stream) {
     constexpr int kB = kXformLaunch.block, kL = kXformLaunch.lds_depth;
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
-    if (cfg.block != kB || cfg.lds_depth != kL || threads > spill_threads) return hipErrorInvalidValue;
+    if (cfg.block != kB || cfg.lds_depth != kL || trace_spill_columns(cfg, n, num_cus) > spill_columns) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_trace_xform<kB, kL, SHADOW, EXT>), dim3((unsigned)(threads / kB)), dim3(kB), 0, stream, sv,
                        (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err, n_dev, perm,
                        gather ? 1 : 0, trace_ray_shift(cfg, n, num_cus), cfg.refill_min);
@@ -997,7 +1000,7 @@ hipError_t launch_mode(const SceneView& sv, bool shadow, bool motion, const void
 }  // namespace
 
 hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, uint64_t n, void* hits32, float* spT,
-                            int32_t* spN, uint64_t spill_threads, int32_t* err, int num_cus, hipStream_t stream,
+                            int32_t* spN, uint64_t spill_columns, int32_t* err, int num_cus, hipStream_t stream,
                             const uint32_t* n_dev) {
     if (n == 0) return hipSuccess;
     if (n > 0xffffffffull) return hipErrorInvalidValue;
@@ -1005,11 +1008,11 @@ hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, 
     constexpr int kB = kExtLaunch.block, kL = kExtLaunch.lds_depth;
     constexpr int kBM = kExtLaunchMotion.block, kLM = kExtLaunchMotion.lds_depth;
     if (sv.any_xform)
-        return launch_xform<false, true>(sv, kXformLaunch, rays, n, hits32, nullptr, spT, spN, spill_threads, err, num_cus,
+        return launch_xform<false, true>(sv, kXformLaunch, rays, n, hits32, nullptr, spT, spN, spill_columns, err, num_cus,
                                          n_dev, nullptr, false, stream);
     const TraceLaunch cfg = motion ? kExtLaunchMotion : kExtLaunch;
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
-    if (threads > spill_threads) return hipErrorInvalidValue;
+    if (trace_spill_columns(cfg, n, num_cus) > spill_columns) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(threads / cfg.block);
     const int ray_shift = trace_ray_shift(cfg, n, num_cus);
     if (motion)
@@ -1040,20 +1043,25 @@ uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus) {
     return blocks * (uint64_t)cfg.block;
 }
 
+uint64_t trace_spill_columns(const TraceLaunch& cfg, uint64_t n, int num_cus) {
+    const uint64_t columns = (trace_grid_threads(cfg, n, num_cus) / 64) << trace_ray_shift(cfg, n, num_cus);
+    return (columns + 255) / 256 * 256;
+}
+
 hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg, const void* rays, uint64_t n,
-                        void* hits, int32_t* geoms, int32_t* counters, float* spT, int32_t* spN, uint64_t spill_threads,
+                        void* hits, int32_t* geoms, int32_t* counters, float* spT, int32_t* spN, uint64_t spill_columns,
                         int32_t* err, int num_cus, hipStream_t stream, const uint32_t* n_dev, const uint32_t* perm, bool gather) {
     if (n == 0) return hipSuccess;
     if (n > 0xffffffffull) return hipErrorInvalidValue;
     if (sv.any_xform) {   // no counters
         if (counters) return hipErrorInvalidValue;
-        return shadow ? launch_xform<true, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
+        return shadow ? launch_xform<true, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_columns, err, num_cus,
                                                   n_dev, perm, gather, stream)
-                      : launch_xform<false, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_threads, err, num_cus,
+                      : launch_xform<false, false>(sv, cfg, rays, n, hits, geoms, spT, spN, spill_columns, err, num_cus,
                                                    n_dev, perm, gather, stream);
     }
     const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
-    if (threads > spill_threads) return hipErrorInvalidValue;
+    if (trace_spill_columns(cfg, n, num_cus) > spill_columns) return hipErrorInvalidValue;
     const uint64_t grid = threads / cfg.block;
     const int ray_shift = trace_ray_shift(cfg, n, num_cus);
 #define VGPU_CASE(B, L)                                                                                         \
@@ -1071,8 +1079,8 @@ hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const Tra
 //
 // vgpu_trace_noalloc keeps its traversal spill area in this file-scope array instead of device
 // memory the scene allocates.  Layout: the error flag in the first 256 bytes, then the spill
-// depths T and nodes N, each (VGPU_MAX_STACK - lds) entries per launched thread, depth-major as
-// the Stack struct addresses them.  The array's host-side name is not a device address: host code
+// depths T and nodes N, each (VGPU_MAX_STACK - lds) entries per spill column
+// (trace_spill_columns), depth-major.  The array's host-side name is not a device address: host code
 // uses only the pointer hipGetSymbolAddress returned for the current device.
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -1102,7 +1110,7 @@ hipError_t noalloc_init(int device) {
     return hipSuccess;
 }
 
-uint64_t noalloc_max_threads(int lds_depth) {
+uint64_t noalloc_max_columns(int lds_depth) {
     const uint64_t per = (uint64_t)(VGPU_MAX_STACK - lds_depth) * (sizeof(float) + sizeof(int32_t));
     return (kNoAllocScratchBytes - 256) / per;
 }
@@ -1117,16 +1125,16 @@ hipError_t launch_trace_noalloc(int device, const SceneView& sv, bool shadow, bo
         base = (unsigned char*)g_scratch_ptr[device];
     }
     if (!base) return hipErrorNotInitialized;
-    const uint64_t threads = trace_grid_threads(cfg, n, num_cus);
-    if (threads > noalloc_max_threads(cfg.lds_depth)) return hipErrorInvalidValue;
+    const uint64_t columns = trace_spill_columns(cfg, n, num_cus);
+    if (columns > noalloc_max_columns(cfg.lds_depth)) return hipErrorInvalidValue;
     int32_t* flag = status ? status : (int32_t*)base;
     hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(64), 0, stream, flag);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || n == 0) return e;
     const uint64_t per = (uint64_t)(VGPU_MAX_STACK - cfg.lds_depth);
     float* spT = (float*)(base + 256);
-    int32_t* spN = (int32_t*)(base + 256 + per * threads * sizeof(float));
-    return launch_trace(sv, shadow, motion, cfg, rays, n, hits, geoms, counters, spT, spN, threads, flag, num_cus,
+    int32_t* spN = (int32_t*)(base + 256 + per * columns * sizeof(float));
+    return launch_trace(sv, shadow, motion, cfg, rays, n, hits, geoms, counters, spT, spN, columns, flag, num_cus,
                         stream, nullptr, nullptr, false);
 }
 

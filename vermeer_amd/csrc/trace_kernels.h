@@ -153,15 +153,15 @@ hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_
                            const RaySortBuffers& sb, int num_cus, hipStream_t stream);
 
 // Enqueues one traversal over n rays (device pointers).  spill_T / spill_N
-// hold (VGPU_MAX_STACK - lds_depth) entries per launched thread; the launch
-// uses at most spill_threads threads.  n_dev (nullable): a device-resident
+// hold (VGPU_MAX_STACK - lds_depth) entries per spill column; the launch
+// fails if it needs more than spill_columns.  n_dev (nullable): a device-resident
 // ray count; the kernel traces min(n, *n_dev) rays (n sizes the grid).  perm (nullable):
 // ray i's results go to slot perm[i] (rays reordered by launch_ray_sort); with gather, ray i is the one
 // at slot perm[i] and its results go there (a list of the slots to trace).  cfg: a scene_launch shape.
 // Returns hipSuccess or the launch error.
 hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg,
                         const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,
-                        float* spill_T, int32_t* spill_N, uint64_t spill_threads, int32_t* err_flag,
+                        float* spill_T, int32_t* spill_N, uint64_t spill_columns, int32_t* err_flag,
                         int num_cus, hipStream_t stream, const uint32_t* n_dev = nullptr,
                         const uint32_t* perm = nullptr, bool gather = false);
 
@@ -169,7 +169,7 @@ hipError_t launch_trace(const SceneView& sv, bool shadow, bool motion, const Tra
 // triangle's three vertices), for the shading kernels.  Launch shape kExtLaunch, or kExtLaunchMotion
 // with motion.
 hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, uint64_t n, void* hits32, float* spill_T,
-                            int32_t* spill_N, uint64_t spill_threads, int32_t* err_flag, int num_cus, hipStream_t stream,
+                            int32_t* spill_N, uint64_t spill_columns, int32_t* err_flag, int num_cus, hipStream_t stream,
                             const uint32_t* n_dev = nullptr);
 
 // Rays that a wavefront takes at a time, as a shift: 64, or fewer when that would leave wavefronts for fewer
@@ -177,6 +177,11 @@ hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, 
 // diverges less, its idle lanes working in the leaf tests: 4096 pinhole rays over the sphere take 45 us
 // instead of 69, 50,000 bounce rays 63 instead of 75, 1024 rays among moving spheres 106 instead of 181.
 int trace_ray_shift(const TraceLaunch& cfg, uint64_t n, int num_cus);
+// Spill columns of a launch: a lane that can own a ray has one.  A column per launched thread made the spill area of
+// a short launch four times as large as its rays need, and its allocation is part of a scene's first pass
+// (65,536 pinhole rays: 460 us, now 91).  Rounded up to 256: min(n, resident lanes) rounded is then the same for
+// every shape, so an area sized by one shape serves a launch of as many rays by a shape with no more waves.
+uint64_t trace_spill_columns(const TraceLaunch& cfg, uint64_t n, int num_cus);
 
 // Threads the launch above will use (so the caller can size the spill area).
 uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus);
@@ -188,10 +193,10 @@ constexpr int kNoAllocMaxDevices = 64;
 // Looks the array up on `device`, which must be current; once per device (later calls return at once).
 hipError_t noalloc_init(int device);
 // Threads whose spill columns fit the array at LDS depth lds_depth.
-uint64_t noalloc_max_threads(int lds_depth);
+uint64_t noalloc_max_columns(int lds_depth);
 // Clears the error flag (status, or the array's own flag word when status is NULL) with a kernel,
 // then enqueues launch_trace with the array as its spill area.  The grid of cfg must fit
-// noalloc_max_threads.  hipErrorNotInitialized: noalloc_init has not run on `device`.
+// noalloc_max_columns.  hipErrorNotInitialized: noalloc_init has not run on `device`.
 hipError_t launch_trace_noalloc(int device, const SceneView& sv, bool shadow, bool motion, const TraceLaunch& cfg,
                                 const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,
                                 int32_t* status, int num_cus, hipStream_t stream);

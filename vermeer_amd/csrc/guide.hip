@@ -335,7 +335,7 @@ __device__ __forceinline__ float dlog_norm_fast(float k) {
 }
 // ---------------------------------------------------------------- inference
 
-// 1M queries: 87 us of kernel (119 before): every lane has its own encoded features (encode), the biases lie in
+// 1M queries: 89 us of kernel (119 before; VALU issue takes 61% of the cycles, the matrix units 26%): every lane has its own encoded features (encode), the biases lie in
 // LDS, the decode needs no full division, square root or exp, and the next queries are fetched ahead.  Two tiles
 // per wave: three and four were no faster.
 // Three waves per SIMD, as the LDS allows; said to the compiler, it also keeps the accumulators in VGPRs (with

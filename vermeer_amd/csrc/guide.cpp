@@ -94,7 +94,7 @@ int vgpu_guide_create(vgpu_guide** out, int device, const float* bounds, uint64_
     if (e == hipSuccess) e = hipMalloc(&g->d_params, P4);
     if (e == hipSuccess) e = hipMalloc(&g->d_m, P4);
     if (e == hipSuccess) e = hipMalloc(&g->d_v, P4);
-    if (e == hipSuccess) e = hipMalloc(&g->d_frag_fwd, (size_t)G::NF_FWD * 64 * 16);
+    if (e == hipSuccess) e = hipMalloc(&g->d_frag_fwd, (size_t)(G::NF_FWD + G::NF_ENC) * 64 * 16);
     if (e == hipSuccess) e = hipMalloc(&g->d_frag_bwd, (size_t)G::NF_BWD * 64 * 16);
     if (e == hipSuccess) e = hipMalloc(&g->tb.partial, (size_t)(max_batch / G::TRAIN_WG) * P4);
     if (e == hipSuccess) e = hipMalloc(&g->tb.loss, sizeof(float) * max_batch);

@@ -47,10 +47,17 @@ __device__ __forceinline__ int hid_feature(int j, int g, int i) {
 __device__ __forceinline__ int out5_index(int g, int s) { return s < 10 ? 5 * (2 * g + s / 5) + s % 5 : -1; }
 
 // Encoded feature (canonical order: 24 d + 2 f, + 1 for the cosine) held in slot m = 8 j + i of lane group g for
-// k-chunk j of layer 1: group g takes frequencies 3 g .. 3 g + 2 of all six inputs, so a lane's 18 sine and
-// cosine pairs are its own and none is idle; -1: one of the 4 pads.
+// k-chunk j of layer 1 in inference: group g takes frequencies 3 g .. 3 g + 2 of all six inputs, so a lane's 18
+// sine and cosine pairs are its own and none is idle; -1: one of the 4 pads.  Training keeps the canonical order:
+// another order of layer 1's sum moves some activations by a bf16 step, and Adam carries that on (2.5e-3 of the
+// parameters after eight steps), so a run of training would no longer repeat an earlier one.
 constexpr int ENC_SLOTS = 36;
 __device__ __forceinline__ int enc_feature(int g, int m) { return m < ENC_SLOTS ? 24 * (m / 6) + 6 * g + m % 6 : -1; }
+// Its inverse: the bf16 element of the forward fragments that holds weight w of W1 for inference.
+__device__ __forceinline__ int enc_slot(int w) {
+    const int row = w / NENC, q = w % NENC, g = q % 24 / 6, m = 6 * (q / 24) + q % 6;
+    return ((NF_FWD + 5 * (row / 16) + m / 8) * 64 + 16 * g + row % 16) * 8 + m % 8;
+}
 
 __device__ __forceinline__ uint16_t bf16_bits(__bf16 b) { return __builtin_bit_cast(uint16_t, b); }
 __device__ __forceinline__ float bf16_val(__bf16 b) { return (float)b; }
@@ -66,11 +73,15 @@ __device__ __forceinline__ bf16x8 frag(const u32x4* s, int f, int lane) {
 // ---------------------------------------------------------------- packing
 
 // Parameter held in element i of lane `lane` of forward fragment f (-1: a zero pad).  Every weight
-// of the five layers is held exactly once.
+// of the five layers is held exactly once below NF_FWD; the rest holds layer 1 again, for inference.
 __device__ int pack_fwd_index(int f, int lane, int i) {
     const int r = lane & 15, g = lane >> 4;
     if (f < F_L2) {
-        const int o = f / 5, j = f % 5, q = enc_feature(g, 8 * j + i);
+        const int o = f / 5, j = f % 5, q = 32 * j + 8 * g + i;
+        return q < NENC ? OW1 + (16 * o + r) * NENC + q : -1;
+    }
+    if (f >= NF_FWD) {
+        const int o = (f - NF_FWD) / 5, j = (f - NF_FWD) % 5, q = enc_feature(g, 8 * j + i);
         return q >= 0 ? OW1 + (16 * o + r) * NENC + q : -1;
     }
     if (f < F_L5) {
@@ -107,6 +118,7 @@ __device__ float pack_bwd(const float* P, int f, int lane, int i) {
 
 // Inverse of the packing: slot_fwd[p] / slot_bwd[p] = the bf16 element (index into the fragment
 // array as uint16) that holds parameter p, or -1 (biases; layer 1 has no backward fragment).
+// Inference's second copy of layer 1 is not in the map (enc_slot).
 // Both arrays are -1 on entry.
 __global__ void k_slot_map(int32_t* __restrict__ slot_fwd, int32_t* __restrict__ slot_bwd) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -120,9 +132,10 @@ __global__ void k_slot_map(int32_t* __restrict__ slot_fwd, int32_t* __restrict__
 
 __global__ void k_pack(const float* __restrict__ P, u32x4* __restrict__ ffwd, u32x4* __restrict__ fbwd) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (NF_FWD + NF_BWD) * 64) return;
-    const bool fwd = t < NF_FWD * 64;
-    const int idx = fwd ? t : t - NF_FWD * 64;
+    constexpr int kFwd = (NF_FWD + NF_ENC) * 64;
+    if (t >= kFwd + NF_BWD * 64) return;
+    const bool fwd = t < kFwd;
+    const int idx = fwd ? t : t - kFwd;
     const int f = idx >> 6, lane = idx & 63;
     uint32_t h[8];
     for (int i = 0; i < 8; i++) {
@@ -136,8 +149,34 @@ __global__ void k_pack(const float* __restrict__ P, u32x4* __restrict__ ffwd, u3
 
 // ---------------------------------------------------------------- forward pieces
 
-// A lane's encoded features in slot order.  sin and cos of pi 2^f x are taken on the exactly reduced argument in
-// revolutions, u - round(u) with u = 2^(f - 1) x.  The lane group sets the frequencies and not the input, so no
+__device__ __forceinline__ float sel6(const float x[6], int d) {
+    return d == 0 ? x[0] : d == 1 ? x[1] : d == 2 ? x[2] : d == 3 ? x[3] : d == 4 ? x[4] : x[5];
+}
+
+// Encoded features 32j + 8g .. +7 in canonical order, for training.  sin and cos of pi 2^f x are taken on the
+// exactly reduced argument r = 2^f x - 2 round(2^(f-1) x), in revolutions (r / 2) for the hardware sine.
+__device__ __forceinline__ bf16x8 enc_chunk(const float x[6], int j, int g) {
+    bf16x8 b;
+    const int q0 = 32 * j + 8 * g;
+    if (q0 >= NENC) {
+        for (int i = 0; i < 8; i++) b[i] = (__bf16)0.0f;
+        return b;
+    }
+    const int d = q0 / 24, f0 = (q0 % 24) / 2;
+    const float xd = sel6(x, d);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float t = ldexpf(xd, f0 + k);
+        const float r = t - 2.0f * rintf(0.5f * t);
+        const float rev = 0.5f * r;
+        b[2 * k] = (__bf16)__builtin_amdgcn_sinf(rev);
+        b[2 * k + 1] = (__bf16)__builtin_amdgcn_cosf(rev);
+    }
+    return b;
+}
+
+// The same features in inference's slot order, all of a lane's.  The reduced argument in revolutions is
+// u - round(u) with u = 2^(f - 1) x.  The lane group sets the frequencies and not the input, so no
 // lane selects its input or skips a chunk.  (Double angles for two of the three octaves saved 1% of 1M queries
 // and moved four times as many activations by a bf16 step.)
 __device__ __forceinline__ void encode(const float x[6], int g, bf16x8 (&e)[5]) {
@@ -221,6 +260,25 @@ __device__ __forceinline__ void layer_hidden(const u32x4* sF, int fbase, const f
         }
 }
 
+template <int NT>
+__device__ __forceinline__ void layer_first_train(const u32x4* sF, const float* bias, int g, int lane,
+                                                  const float (&x)[NT][6], f32x4 (&acc)[4][NT]) {
+    bias_hidden<NT>(acc, bias, g);
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+        bf16x8 b[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) b[t] = enc_chunk(x[t], j, g);
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+            const bf16x8 a = frag(sF, F_L1 + 5 * o + j, lane);
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[o][t] = mfma(a, b[t], acc[o][t]);
+        }
+    }
+}
+
+// The same on inference's copy of the weights.
 template <int NT>
 __device__ __forceinline__ void layer_first(const u32x4* sF, const float* bias, int g, int lane, const float (&x)[NT][6],
                                             f32x4 (&acc)[4][NT]) {
@@ -351,8 +409,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         constexpr int NI = (NF_FWD * 64 + 255) / 256;
         u32x4 fr[NI];
 #pragma unroll
-        for (int i = 0; i < NI; i++)
-            fr[i] = reinterpret_cast<const u32x4*>(net.frag_fwd)[min((int)threadIdx.x + 256 * i, NF_FWD * 64 - 1)];
+        for (int i = 0; i < NI; i++) {
+            const int k = min((int)threadIdx.x + 256 * i, NF_FWD * 64 - 1);   // layer 1 from its second copy
+            fr[i] = reinterpret_cast<const u32x4*>(net.frag_fwd)[k < F_L2 * 64 ? NF_FWD * 64 + k : k];
+        }
         for (int w = threadIdx.x; w < BIAS_WORDS; w += 256) sBias[w] = bias_word(net.params, w);
 #pragma unroll
         for (int i = 0; i < NI; i++) {
@@ -646,7 +706,7 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
         }
         f32x4 acc[4][NT];
         bf16x8 X2[2][NT], X3[2][NT], X4[2][NT], X5[2][NT];
-        layer_first<NT>(sF, sBias, g, lane, x, acc);
+        layer_first_train<NT>(sF, sBias, g, lane, x, acc);
         relu_pack<NT>(acc, X2);
         layer_hidden<NT>(sF, F_L2, sBias + 1 * NH, g, lane, X2, acc);
         relu_pack<NT>(acc, X3);
@@ -736,11 +796,14 @@ __global__ __launch_bounds__(512) void k_train(Net net, SampleSource src, TrainB
         dw_chunk(Xs, Ys, T2, bs2, NH);
         __syncthreads();
         // layer 1: its input is the encoding, recomputed (the forward pass keeps it in no register)
-        {
-            bf16x8 e[5];
-            encode(x[0], g, e);
 #pragma unroll
-            for (int m = 0; m < ENC_SLOTS; m++) Xs[enc_feature(g, m) * STG + col] = bf16_bits(e[m / 8][m % 8]);
+        for (int j = 0; j < 5; j++) {
+            const int q0 = 32 * j + 8 * g;
+            if (q0 < NENC) {
+                const bf16x8 b = enc_chunk(x[0], j, g);
+#pragma unroll
+                for (int i = 0; i < 8; i++) Xs[(q0 + i) * STG + col] = bf16_bits(b[i]);
+            }
         }
         stage_hidden(Ys, D, g, col);
         __syncthreads();
@@ -828,6 +891,7 @@ __global__ __launch_bounds__(ADAM_THREADS) void k_adam(
             P[p] = np;
             const uint16_t h = bf16_bits((__bf16)np);
             if (sf >= 0) ffwd[sf] = h;
+            if (p < OB1) ffwd[enc_slot(p - OW1)] = h;
             if (sb >= 0) fbwd[sb] = h;
         }
     }
@@ -847,7 +911,7 @@ hipError_t launch_slot_map(int32_t* slot_fwd, int32_t* slot_bwd, hipStream_t st)
 }
 
 hipError_t launch_pack(const float* params, uint4* ffwd, uint4* fbwd, hipStream_t st) {
-    const int total = (NF_FWD + NF_BWD) * 64;
+    const int total = (NF_FWD + NF_ENC + NF_BWD) * 64;
     hipLaunchKernelGGL(k_pack, dim3((total + 255) / 256), dim3(256), 0, st, params, (u32x4*)ffwd, (u32x4*)fbwd);
     return hipGetLastError();
 }

@@ -21,6 +21,7 @@ static_assert(NPARAM == 24360, "parameter count");
 
 // bf16 operand fragments of the 16x16x32 MFMA, 64 lanes x 16 bytes each.
 constexpr int NF_FWD = 4 * 5 + 3 * 4 * 2 + 3 * 2;   // W1 (4 out tiles x 5 k-chunks), W2..W4, W5 (3 x 2)
+constexpr int NF_ENC = 4 * 5;                       // W1 again, in the order of inference's encoding, behind those
 constexpr int NF_BWD = 4 * 2 * 4;                   // W5^T, W4^T, W3^T, W2^T (4 in tiles x 2 k-chunks)
 constexpr int KSPLIT = 1024;                        // batch granularity (a batch is a multiple of it)
 // Samples per training workgroup: each writes one fp32 partial of every parameter's gradient.
@@ -38,7 +39,7 @@ static_assert(sizeof(TrainSample) == 48, "TrainSample is 48 bytes");
 
 struct Net {
     const float* params;       // fp32 master (NPARAM)
-    const uint4* frag_fwd;     // NF_FWD x 64
+    const uint4* frag_fwd;     // (NF_FWD + NF_ENC) x 64
     const uint4* frag_bwd;     // NF_BWD x 64
     float bounds[6];           // scene box used to normalise positions
 };

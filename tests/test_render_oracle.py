@@ -16,6 +16,7 @@ import oracle
 from vermeer_amd import scenes
 
 REF = "/root/reference"
+HAVE_REF = os.path.isdir(os.path.join(REF, "math"))   # the folder may be there and empty
 
 
 # ------------------------------------------------------------ ldseq (math/ldseq)
@@ -76,7 +77,7 @@ def _parse_go_tables(name):
     return tables
 
 
-@pytest.mark.skipif(not os.path.exists(REF), reason="reference checkout not present")
+@pytest.mark.skipif(not HAVE_REF, reason="reference checkout not present")
 def test_raster_tables_equal_reference_literals():
     fwd_ref = _parse_go_tables("vdcSobolMatrices")
     inv_ref = _parse_go_tables("vdcSobolMatricesInv")
@@ -91,7 +92,7 @@ def test_raster_tables_equal_reference_literals():
 
 # ------------------------------------------------------------ colour
 
-@pytest.mark.skipif(not os.path.exists(REF), reason="reference checkout not present")
+@pytest.mark.skipif(not HAVE_REF, reason="reference checkout not present")
 def test_cie_table_equals_reference_literal():
     text = open(os.path.join(REF, "colour/cie1931_2deg.go")).read()
     ours = oracle.cie_tables()

@@ -406,6 +406,21 @@ __device__ __forceinline__ void ray_to_object(const float* Minv, float* P, float
     for (int k = 0; k < 3; k++) { P[k] = p[k]; D[k] = d[k]; }
 }
 
+// The ray at (px, py, pz) along (dx, dy, dz) moved by the inverse of x's transform at `time`.  A call and not inlined: the
+// decomposed keys, the matrix and its inverse would be allocated beside the traversal's whole state, and the kernels
+// spilled 38 to 116 registers, into the box and leaf steps too (trace_wide's XFORM form; figures at k_trace_xform).
+struct RayPD {
+    float p[3], d[3];
+};
+__device__ __noinline__ RayPD xform_ray(const DevXform* x, const float* xkeys, float time, float px, float py, float pz,
+                                        float dx, float dy, float dz) {
+    float M[16], Minv[16];
+    xform_at(*x, xkeys, time, M, Minv);
+    RayPD r{{px, py, pz}, {dx, dy, dz}};
+    ray_to_object(Minv, r.p, r.d);
+    return r;
+}
+
 // Whether the near/far box tests hold for the ray (box4_near).
 template <bool MOTION>
 __device__ __forceinline__ bool ray_plain(const RayS& r) {
@@ -467,11 +482,10 @@ __device__ __forceinline__ int next_geom_xf(const SceneView& sv, const float4* _
             // the instance's or proc's transform, then the mesh's own
 #pragma unroll 1
             for (int level = x.kind >= kXfInstance ? 0 : 1; level < 2; level++) {
-                const DevXform xl = level == 0 ? x : sv.xforms[w.slot];
-                if (xl.kind == kXfNone) continue;
-                float M[16], Minv[16];
-                xform_at(xl, sv.xkeys, rb.w, M, Minv);
-                ray_to_object(Minv, P, D);
+                const DevXform* xl = sv.xforms + (level == 0 ? gcur : w.slot);
+                if (xl->kind == kXfNone) continue;
+                const RayPD o = xform_ray(xl, sv.xkeys, rb.w, P[0], P[1], P[2], D[0], D[1], D[2]);
+                for (int k = 0; k < 3; k++) { P[k] = o.p[k]; D[k] = o.d[k]; }
             }
         }
         for (int k = 0; k < 3; k++) r.P[k] = P[k];
@@ -526,8 +540,10 @@ __device__ __forceinline__ float lane_f(int addr, float x) {
 __device__ __forceinline__ int lane_i(int addr, int x) { return __builtin_amdgcn_ds_bpermute(addr, x); }
 
 // In scenes with transforms, lanes at the end or the start of a geom wait until kTurnWait times as many
-// wait as hold a node or a leaf: the transform of a moving instance is a thousand instructions.  262,144
-// rays in a room of 60 instances: 712 us when half as many sufficed, 674 at 1, 656 at 2, 646 at 6.
+// wait as hold a node or a leaf: the transform of a moving instance is a thousand instructions.  262,144 rays
+// in a room of 60 instances / 2^20 rays in one of 20, in us: 751 / 1064 when half as many suffice, 706 / 990 at 1,
+// 682 / 917 at 2, 678 / 886 at 3, 671 / 880 at 4, 667 / 878 at 6, 675 / 884 at 8; shadow rays in the first: 568, 522,
+// 496, 506, 510, 516, 527.
 constexpr int kTurnWait = 4;
 
 // What a lane does next, beside node indices (>= 0) and mesh leaves (< kIdle).
@@ -932,10 +948,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
     trace_wide<BLOCK, LDS, SHADOW, true, COUNTERS, EXT>(VGPU_TRACE_ARGS);
 }
 
-// Scenes holding GeomInstances, Procs or meshes with their own Transform.  Four waves per SIMD: the
-// transforms take registers, and their lanes wait for one another (kTurnWait).
-// 262,144 rays in rooms of 60 instances: 988 us, against 1,898 us for one ray per lane with the recursion
-// inside it (the leaf triangles of a lane tested by that lane alone).
+// Scenes holding GeomInstances, Procs or meshes with their own Transform.  Four waves per SIMD: the walk
+// over geoms takes registers, and its lanes wait for one another (kTurnWait).
+// 262,144 rays in a room of 60 instances: 670 us of kernel, 12 registers spilled.  With the transform inlined
+// (xform_ray) 73 were and the kernel took 1061 us, 875 without spills at three waves per SIMD; one ray per lane with
+// the recursion inside it (the leaf triangles of a lane tested by that lane alone) took 1868.
 template <int BLOCK, int LDS, bool SHADOW, bool EXT>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_trace_xform(VGPU_TRACE_PARAMS) {
     trace_wide<BLOCK, LDS, SHADOW, true, false, EXT, true>(VGPU_TRACE_ARGS);

@@ -461,7 +461,9 @@ typedef struct vgpu_trace_config {
     int32_t waves_per_cu; /* resident-grid sizing: workgroups = CUs * waves_per_cu * 64 / block */
     int32_t sort;         /* 0: trace in the given order; k in 1..6: first reorder the rays by bucket =
                            * (Morton cell of the origin in a 2^k-per-axis grid over the scene box) x
-                           * (direction octant); results still land in the callers' order */
+                           * (direction octant); results still land in the callers' order.  Applies to vgpu_trace
+                           * and to the shadow rays of render and path passes; a pass's closest-hit rays are
+                           * traced as they come, vgpu_trace_noalloc never sorts */
     int32_t refill;       /* 1..64: a wavefront's finished lanes wait until this many are idle, then take
                            * new rays together (ray set-up runs once for them); 0: the default, 48 */
 } vgpu_trace_config;

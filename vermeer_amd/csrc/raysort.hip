@@ -61,8 +61,9 @@ __global__ void k_sort_clear(uint32_t* __restrict__ hist, uint32_t nb) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) hist[i] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_sort_keys(const float4* __restrict__ rays, uint64_t n,
-                                                   const uint32_t* __restrict__ n_dev, float3 lo, float3 scale,
+// list (nullable): ray i is the one at slot list[i].
+__global__ __launch_bounds__(256) void k_sort_keys(const float4* __restrict__ rays, const uint32_t* __restrict__ list,
+                                                   uint64_t n, const uint32_t* __restrict__ n_dev, float3 lo, float3 scale,
                                                    int bits, uint32_t* __restrict__ keys, uint32_t* __restrict__ hist) {
     if (n_dev) n = min(n, (uint64_t)*n_dev);
     const float cmax = (float)((1 << bits) - 1);
@@ -73,7 +74,8 @@ __global__ __launch_bounds__(256) void k_sort_keys(const float4* __restrict__ ra
         const bool act = i < n;
         uint32_t key = 0;
         if (act) {
-            const float4 a = rays[2 * i], b = rays[2 * i + 1];
+            const uint64_t j = list ? list[i] : i;
+            const float4 a = rays[2 * j], b = rays[2 * j + 1];
             const uint32_t qx = (uint32_t)fminf(fmaxf((a.x - lo.x) * scale.x, 0.0f), cmax);
             const uint32_t qy = (uint32_t)fminf(fmaxf((a.y - lo.y) * scale.y, 0.0f), cmax);
             const uint32_t qz = (uint32_t)fminf(fmaxf((a.z - lo.z) * scale.z, 0.0f), cmax);
@@ -134,8 +136,8 @@ __global__ __launch_bounds__(1024) void k_scan_top(uint32_t* __restrict__ bsum, 
     }
 }
 
-__global__ __launch_bounds__(256) void k_sort_scatter(const float4* __restrict__ rays, uint64_t n,
-                                                      const uint32_t* __restrict__ n_dev,
+__global__ __launch_bounds__(256) void k_sort_scatter(const float4* __restrict__ rays, const uint32_t* __restrict__ list,
+                                                      uint64_t n, const uint32_t* __restrict__ n_dev,
                                                       const uint32_t* __restrict__ keys, uint32_t* __restrict__ offs,
                                                       const uint32_t* __restrict__ bsum, float4* __restrict__ out,
                                                       uint32_t* __restrict__ perm) {
@@ -148,9 +150,10 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const float4* __restrict__
         const uint32_t rank = wave_count(offs, key, act);
         if (act) {
             const uint32_t pos = rank + bsum[key / SCAN_BLOCK];
-            out[2 * (uint64_t)pos] = rays[2 * i];
-            out[2 * (uint64_t)pos + 1] = rays[2 * i + 1];
-            perm[pos] = (uint32_t)i;
+            const uint64_t j = list ? list[i] : i;
+            out[2 * (uint64_t)pos] = rays[2 * j];
+            out[2 * (uint64_t)pos + 1] = rays[2 * j + 1];
+            perm[pos] = (uint32_t)j;
         }
     }
 }
@@ -162,7 +165,7 @@ uint32_t ray_sort_buckets(int bits) { return 1u << (3 * bits + 3); }
 uint32_t ray_sort_scan_blocks(int bits) { return (ray_sort_buckets(bits) + SCAN_BLOCK - 1) / SCAN_BLOCK; }
 
 hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_t n, const uint32_t* n_dev,
-                           const RaySortBuffers& sb, int num_cus, hipStream_t st) {
+                           const RaySortBuffers& sb, int num_cus, hipStream_t st, const uint32_t* list) {
     if (bits < 1 || bits > 6 || n > sb.capacity || n > 0xffffffffull) return hipErrorInvalidValue;
     if (n == 0) return hipSuccess;
     const uint32_t nb = ray_sort_buckets(bits), nblk = ray_sort_scan_blocks(bits);
@@ -177,11 +180,11 @@ hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_
     if (g > gmax) g = gmax;
     hipLaunchKernelGGL(k_sort_clear, dim3((nb + 255) / 256 < 4096 ? (nb + 255) / 256 : 4096), dim3(256), 0, st,
                        sb.hist, nb);
-    hipLaunchKernelGGL(k_sort_keys, dim3((unsigned)g), dim3(256), 0, st, (const float4*)rays, n, n_dev, lo, sc, bits,
+    hipLaunchKernelGGL(k_sort_keys, dim3((unsigned)g), dim3(256), 0, st, (const float4*)rays, list, n, n_dev, lo, sc, bits,
                        sb.keys, sb.hist);
     hipLaunchKernelGGL(k_scan_block, dim3(nblk), dim3(256), 0, st, sb.hist, nb, sb.bsum);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, sb.bsum, nblk);
-    hipLaunchKernelGGL(k_sort_scatter, dim3((unsigned)g), dim3(256), 0, st, (const float4*)rays, n, n_dev, sb.keys,
+    hipLaunchKernelGGL(k_sort_scatter, dim3((unsigned)g), dim3(256), 0, st, (const float4*)rays, list, n, n_dev, sb.keys,
                        sb.hist, sb.bsum, sb.rays, sb.perm);
     return hipGetLastError();
 }

@@ -370,10 +370,10 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
         HIP_TRY(hipEventRecord(ev[0], st));
     }
     const uint32_t* perm = list;
-    if (cfg.sort > 0 && !list) {
+    if (cfg.sort > 0) {
         if (n > 0xffffffffull) return fail(VGPU_ERR_ARG, "ray sorting handles at most 2^32-1 rays per call");
         if ((rc = ensure_sort(s, n))) return rc;
-        hipError_t e = vgpu::launch_ray_sort(s->box, cfg.sort, d_rays, n, n_dev, s->sort, s->num_cus, st);
+        hipError_t e = vgpu::launch_ray_sort(s->box, cfg.sort, d_rays, n, n_dev, s->sort, s->num_cus, st, list);
         if (e != hipSuccess) return fail(VGPU_ERR_HIP, "ray sort launch: %s", hipGetErrorString(e));
         d_rays = s->sort.rays;
         perm = s->sort.perm;
@@ -381,7 +381,7 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
     if (ev[1]) HIP_TRY(hipEventRecord(ev[1], st));
     hipError_t e = vgpu::launch_trace(s->view, (flags & VGPU_TRACE_SHADOW) != 0, s->any_motion, L, d_rays, n, d_hits,
                                       d_geoms, d_counters, s->d_spT, s->d_spN, s->spill_columns, s->d_err, s->num_cus, st,
-                                      n_dev, perm, list != nullptr);
+                                      n_dev, perm, list && perm == list);
     if (e != hipSuccess) return fail(VGPU_ERR_HIP, "trace launch: %s", hipGetErrorString(e));
     if (ev[2]) HIP_TRY(hipEventRecord(ev[2], st));
     return VGPU_OK;

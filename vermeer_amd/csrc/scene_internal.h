@@ -203,7 +203,7 @@ struct GraphCache {
 };
 // Enqueues one traversal (device pointers) with configuration cfg.  n_dev (nullable): device-resident
 // count of rays to trace, at most n.  list (nullable): the slots of d_rays and d_hits to trace, in order
-// (they are not sorted).
+// unless cfg sorts them.
 int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n, void* d_hits, int32_t* d_geoms,
                   int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev = nullptr, const uint32_t* list = nullptr);
 

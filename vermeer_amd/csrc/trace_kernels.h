@@ -148,9 +148,10 @@ struct RaySortBuffers {
 uint32_t ray_sort_buckets(int bits);
 uint32_t ray_sort_scan_blocks(int bits);
 // Sorts min(n, *n_dev) rays into sb.rays / sb.perm by (Morton cell of the origin in a 2^bits grid over
-// box = lo xyz, hi xyz) x (direction octant); bits in [1,6].
+// box = lo xyz, hi xyz) x (direction octant); bits in [1,6].  list (nullable): ray i is the one at slot list[i], and
+// sb.perm holds slots.
 hipError_t launch_ray_sort(const float* box, int bits, const void* rays, uint64_t n, const uint32_t* n_dev,
-                           const RaySortBuffers& sb, int num_cus, hipStream_t stream);
+                           const RaySortBuffers& sb, int num_cus, hipStream_t stream, const uint32_t* list = nullptr);
 
 // Enqueues one traversal over n rays (device pointers).  spill_T / spill_N
 // hold (VGPU_MAX_STACK - lds_depth) entries per spill column; the launch

@@ -453,8 +453,10 @@ int vgpu_scene_timing(vgpu_scene* scene, float* trace_ms, float* sort_ms, int32_
 
 /* Traversal launch configuration (the autotuner's knobs).  Until the caller
  * sets one (or runs the autotuner), vgpu_scene_commit picks block 64, LDS
- * stack 12, 20 waves per CU, no sort for a static scene, and 64 / 8 / 20 /
- * no sort for a scene with motion keys. */
+ * stack 12, 20 waves per CU, no sort for a static scene, 64 / 8 / 20 / no sort
+ * for a scene with motion keys and 64 / 12 / 16 / no sort for one with instances,
+ * procs or mesh transforms.  The last kind is always traced with block 64 and LDS
+ * stack 12, whatever block and lds_stack say. */
 typedef struct vgpu_trace_config {
     int32_t block;        /* threads per workgroup: 64, 128 or 256 */
     int32_t lds_stack;    /* stack entries per ray held in LDS: 8, 12, 16, 24 or 32; the rest spill to HBM */
@@ -475,7 +477,8 @@ int vgpu_scene_get_trace_config(const vgpu_scene* scene, vgpu_trace_config* cfg)
  * waves per CU in {8, 16, 20, 24, 32} x sort in {0, 4, 5, 6}, the sort
  * included in the time) on the given rays
  * (device pointers, n rays), then the refill threshold (16, 32, 40, 48, 56, 64)
- * in the fastest of those, and keeps the fastest.  The results of a trace never
+ * in the fastest of those, and keeps the fastest (in a scene with transforms only the
+ * candidates of its block and LDS depth).  The results of a trace never
  * depend on its configuration.  best_out (nullable) receives the chosen
  * configuration; ms_out (nullable) its time. */
 int vgpu_scene_autotune(vgpu_scene* scene, uint32_t flags, const vgpu_ray* d_rays, uint64_t n,

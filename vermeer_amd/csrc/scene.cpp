@@ -811,9 +811,14 @@ int vgpu_scene_commit(vgpu_scene* s) {
         }
     }
     s->any_motion = maxKeys > 1;
-    // Default launch shape unless the caller chose one: both kernels hold five waves per SIMD, so 20 waves
-    // per CU, with the LDS stack that measured fastest (figures at kExtLaunch and k_trace_wide_m5).
-    if (!s->cfg_set) s->cfg = s->any_motion ? vgpu_trace_config{64, 8, 20, 0, 0} : vgpu_trace_config{64, 12, 20, 0, 0};
+    bool any_xform = false;
+    for (auto& m : s->meshes) any_xform = any_xform || m.kind != vgpu::kXfNone;
+    // Default launch shape unless the caller chose one: the static and the motion kernel hold five waves per
+    // SIMD, so 20 waves per CU, with the LDS stack that measured fastest (figures at kExtLaunch and
+    // k_trace_wide_m5); scenes with transforms have one shape, of which the caller sets the waves.
+    if (!s->cfg_set)
+        s->cfg = any_xform ? vgpu_trace_config{vgpu::kXformLaunch.block, vgpu::kXformLaunch.lds_depth, vgpu::kXformLaunch.waves_per_cu, 0, 0}
+                           : (s->any_motion ? vgpu_trace_config{64, 8, 20, 0, 0} : vgpu_trace_config{64, 12, 20, 0, 0});
 
     // Flatten into the device layout.
     std::vector<vgpu::DevNode> dnodes;
@@ -954,10 +959,8 @@ int vgpu_scene_commit(vgpu_scene* s) {
     }
     // Transforms per slot (xform.h records; one key precomputed with its inverse)
     {
-        bool any = false;
-        for (auto& m : s->meshes) any = any || m.kind != vgpu::kXfNone;
-        s->view.any_xform = any ? 1 : 0;
-        if (any) {
+        s->view.any_xform = any_xform ? 1 : 0;
+        if (any_xform) {
             std::vector<int32_t> slot_of(nall);
             for (int slot = 0; slot < nall; slot++) slot_of[s->order[slot]] = slot;
             std::vector<vgpu::DevXform> dx(nall);
@@ -1219,6 +1222,8 @@ int vgpu_scene_autotune(vgpu_scene* s, uint32_t flags, const vgpu_ray* d_rays, u
                 for (int w : waves) {
                     const vgpu_trace_config c{b, l, w, so, 0};
                     if (rc || check_config(c)) continue;
+                    // a scene with transforms has one block and LDS depth: the other candidates are the same launch
+                    if (s->view.any_xform && (b != vgpu::kXformLaunch.block || l != vgpu::kXformLaunch.lds_depth)) continue;
                     rc = time_config(c);
                 }
     // second stage: the refill threshold in the fastest shape

@@ -124,14 +124,17 @@ struct TraceLaunch {
 constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 
-// Launch shape of the traversals of a scene with transforms (block and LDS depth are its kernel's): the
-// scene's refill threshold in that shape.
-constexpr TraceLaunch kXformLaunch{64, 12, 16, kRefillDefault, 8};   // spread: 50,000 rays take 368 us over 8, 442 over 16
+// Launch shape of the traversals of a scene with transforms: block and LDS depth are its kernel's, waves per CU and
+// refill threshold the scene's (these waves where the caller chose none, and in launch_trace_ext).
+// Spread over 4 / 8 / 16 waves per CU: 5,003 rays take 328 / 268 / 261 us, 50,000 take 471 / 472 / 475, 120,001 take
+// 533 / 533 / 573.
+constexpr TraceLaunch kXformLaunch{64, 12, 16, kRefillDefault, 8};
 static_assert(kXformLaunch.waves_per_cu <= kExtLaunch.waves_per_cu && kXformLaunch.waves_per_cu <= kExtLaunchMotion.waves_per_cu,
               "the shading passes' spill areas cover it");
 inline TraceLaunch scene_launch(const SceneView& sv, const TraceLaunch& cfg) {
     if (!sv.any_xform) return cfg;
     TraceLaunch l = kXformLaunch;
+    l.waves_per_cu = cfg.waves_per_cu;
     l.refill_min = cfg.refill_min;
     return l;
 }

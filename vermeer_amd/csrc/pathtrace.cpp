@@ -245,7 +245,7 @@ int vgpu_pt_pass(vgpu_pt* pt, uint32_t flags, uint32_t pass, double* accum, void
     const bool graph = (flags & VGPU_GRAPH) != 0;
     if (graph && host) return fail(VGPU_ERR_ARG, "VGPU_GRAPH needs VGPU_TRACE_DEVICE_PTRS");
     if (graph && s->timing) return fail(VGPU_ERR_STATE, "VGPU_GRAPH with kernel timing enabled");
-    if (graph && s->cfg.sort > 0) { const int rc = ensure_sort(s, np); if (rc) return rc; }
+    { const int rc = ensure_trace(s, np); if (rc) return rc; }
     // The pass's launches, on the caller's stream or on the capture stream of the pass's graph.
     auto enqueue = [&](hipStream_t st) -> int {
         vgpu::PTView v = pt->v;

@@ -505,7 +505,7 @@ int vgpu_render_pass(vgpu_render* r, uint32_t flags, const uint64_t* scrambles, 
     const bool graph = (flags & VGPU_GRAPH) != 0;
     if (graph && host) return fail(VGPU_ERR_ARG, "VGPU_GRAPH needs VGPU_TRACE_DEVICE_PTRS");
     if (graph && s->timing) return fail(VGPU_ERR_STATE, "VGPU_GRAPH with kernel timing enabled");
-    if (graph && s->cfg.sort > 0) { const int rc = ensure_sort(s, ns); if (rc) return rc; }
+    if (r->rv.groups > 0) { const int rc = ensure_trace(s, ns); if (rc) return rc; }
     uint64_t shadow_count = 0;
     // The pass's launches, on the caller's stream or on the capture stream of the pass's graph.
     auto enqueue = [&](hipStream_t st) -> int {

@@ -281,6 +281,15 @@ int ensure_spill(vgpu_scene* s, uint64_t columns) {
     return VGPU_OK;
 }
 
+vgpu::TraceLaunch trace_shape(const vgpu_scene* s, const vgpu_trace_config& cfg) {
+    return vgpu::scene_launch(s->view, {cfg.block, cfg.lds_stack, cfg.waves_per_cu, cfg.refill > 0 ? cfg.refill : vgpu::kRefillDefault});
+}
+
+int ensure_trace(vgpu_scene* s, uint64_t n) {
+    const int rc = ensure_spill(s, vgpu::trace_spill_columns(trace_shape(s, s->cfg), n, s->num_cus));
+    return rc || s->cfg.sort == 0 ? rc : ensure_sort(s, n);
+}
+
 int check_config(const vgpu_trace_config& c) {
     if (c.block != 64 && c.block != 128 && c.block != 256) return fail(VGPU_ERR_ARG, "block must be 64, 128 or 256");
     if (c.lds_stack != 8 && c.lds_stack != 12 && c.lds_stack != 16 && c.lds_stack != 24 && c.lds_stack != 32)
@@ -359,8 +368,7 @@ int enqueue_trace(vgpu_scene* s, uint32_t flags, const void* d_rays, uint64_t n,
                   int32_t* d_counters, hipStream_t st, const vgpu_trace_config& cfg, const uint32_t* n_dev, const uint32_t* list) {
     if (d_counters && s->view.any_xform)
         return fail(VGPU_ERR_ARG, "per-ray counters are not kept for scenes with instances, procs or mesh transforms");
-    const vgpu::TraceLaunch L = vgpu::scene_launch(
-        s->view, {cfg.block, cfg.lds_stack, cfg.waves_per_cu, cfg.refill > 0 ? cfg.refill : vgpu::kRefillDefault});
+    const vgpu::TraceLaunch L = trace_shape(s, cfg);
     int rc = ensure_spill(s, vgpu::trace_spill_columns(L, n, s->num_cus));
     if (rc) return rc;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
@@ -1104,8 +1112,7 @@ int vgpu_trace_noalloc(vgpu_scene* s, uint32_t flags, const vgpu_ray* d_rays, ui
     DeviceGuard dg(s->device);
     // The scene's launch shape with fewer resident waves where its spill columns would not fit the
     // scratch array; never sorted (the sort's buffers grow with n).
-    vgpu::TraceLaunch L = vgpu::scene_launch(s->view, {s->cfg.block, s->cfg.lds_stack, s->cfg.waves_per_cu,
-                                                       s->cfg.refill > 0 ? s->cfg.refill : vgpu::kRefillDefault});
+    vgpu::TraceLaunch L = trace_shape(s, s->cfg);
     const uint64_t cap = vgpu::noalloc_max_columns(L.lds_depth);
     while (L.waves_per_cu > 1 && vgpu::trace_spill_columns(L, n, s->num_cus) > cap) L.waves_per_cu--;
     if (vgpu::trace_spill_columns(L, n, s->num_cus) > cap)

@@ -171,8 +171,15 @@ struct DeviceGuard {
 // NULL when the runtime cannot create one.
 hipEvent_t timing_event(vgpu_scene* s);
 
-// Ensures the spill area covers `threads` traversal threads.
+// Ensures the spill area holds `columns` spill columns (trace_spill_columns).
 int ensure_spill(vgpu_scene* s, uint64_t columns);
+// The launch shape of a configuration on the scene.
+vgpu::TraceLaunch trace_shape(const vgpu_scene* s, const vgpu_trace_config& cfg);
+// Ensures what enqueue_trace of n rays allocates, spill area and sort buffers, with the scene's configuration as it is
+// now.  A pass does so before its first launch: its closest-hit launches hold the spill area's address, and a
+// capture records no allocation, so neither may change within the pass (the caller may have raised waves_per_cu since
+// the pass's object was created).
+int ensure_trace(vgpu_scene* s, uint64_t n);
 // Host math of the camera (render.cpp), in the reference's float32 operation order.
 void vec3_normalize(const float* a, float* out);
 void vec3_cross(const float* a, const float* b, float* o);

@@ -271,6 +271,7 @@ int upload(T** dptr, const std::vector<T>& v) {
 
 int ensure_spill(vgpu_scene* s, uint64_t columns) {
     if (s->d_spT && s->spill_columns >= columns) return VGPU_OK;
+    s->spill_columns = 0;   // until both arrays are there: one allocation may fail
     if (s->d_spT) { HIP_TRY(hipFree(s->d_spT)); s->d_spT = nullptr; }
     if (s->d_spN) { HIP_TRY(hipFree(s->d_spN)); s->d_spN = nullptr; }
     // size for the smallest LDS depth so later configuration changes never need more

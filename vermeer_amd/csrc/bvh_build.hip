@@ -885,12 +885,13 @@ __global__ void k_leaf_boxes(const GElem* E, const int2* leaves, int n, float* o
 }
 
 // Moves subtree s's nodes from the scratch area (offset src[s], in the order they were found) to their
-// pre-order place from dst[s] on, renumbering child nodes.
+// pre-order place from dst[s] on, renumbering child nodes.  A block per subtree along x: the grid's other axes end at
+// 65,535, which 38 million elements can pass (about 590 a subtree where the ranges above 2048 split evenly).
 __global__ void k_place(const vgpu_qbvh_node* scratch, const int* pre_all, const int* src, const int* dst,
                         const int* counts, vgpu_qbvh_node* out) {
-    const int s = blockIdx.y;
+    const int s = blockIdx.x;
     const int* pre = pre_all + src[s];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < counts[s]; i += gridDim.x * blockDim.x) {
+    for (int i = threadIdx.x; i < counts[s]; i += blockDim.x) {
         vgpu_qbvh_node nd = scratch[src[s] + i];
         for (int c = 0; c < 4; c++)
             if (nd.children[c] >= 0) nd.children[c] = dst[s] + pre[nd.children[c]];
@@ -1360,7 +1361,7 @@ int build_qbvh_gpu(float* boxes, float* centroids, int32_t* idx, int32_t n, int3
         BUILD_TRY(d_dst.alloc(nsub));
         BUILD_TRY(hipMemcpyAsync(d_src.p, src.data(), nsub * sizeof(int), hipMemcpyHostToDevice, st));
         BUILD_TRY(hipMemcpyAsync(d_dst.p, sub_dst.data(), nsub * sizeof(int), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_place, dim3(8, nsub), dim3(256), 0, st, d_scratch.p, d_pre.p, d_src.p, d_dst.p,
+        hipLaunchKernelGGL(k_place, dim3(nsub), dim3(256), 0, st, d_scratch.p, d_pre.p, d_src.p, d_dst.p,
                            d_counts.p, d_nodes.p);
         BUILD_TRY(hipGetLastError());
     }

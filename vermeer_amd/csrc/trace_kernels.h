@@ -121,6 +121,9 @@ struct TraceLaunch {
 // motion scenes; callers size the spill area for the larger grid.  The static kernel holds 88 VGPRs, five
 // waves per SIMD: a grid of 20 waves per CU fills them and leaves no workgroup waiting (2.1M bounce rays,
 // block 64: 725 us at 20 waves per CU, 786 at 16; block 128: 749 at 20, 780 at 24).
+// The motion shape runs the four-wave kernel: a pass over the moving spheres takes 843 us at 512^2, 1171 with five
+// segments at 320 x 199 and 2035 at 1024^2, in the five-wave kernel's shape (64, 8, 20) 864, 1215 and 2081 (64, 16, 16:
+// 841, 1159 and 2053).
 constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 

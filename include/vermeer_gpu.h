@@ -453,7 +453,7 @@ int vgpu_scene_timing(vgpu_scene* scene, float* trace_ms, float* sort_ms, int32_
 
 /* Traversal launch configuration (the autotuner's knobs).  Until the caller
  * sets one (or runs the autotuner), vgpu_scene_commit picks block 64, LDS
- * stack 12, 20 waves per CU, no sort for a static scene, 64 / 8 / 20 / no sort
+ * stack 12, 20 waves per CU, no sort for a static scene, 256 / 16 / 16 / no sort
  * for a scene with motion keys and 64 / 12 / 16 / no sort for one with instances,
  * procs or mesh transforms.  The last kind is always traced with block 64 and LDS
  * stack 12, whatever block and lds_stack say. */

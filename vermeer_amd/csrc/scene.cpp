@@ -822,12 +822,11 @@ int vgpu_scene_commit(vgpu_scene* s) {
     s->any_motion = maxKeys > 1;
     bool any_xform = false;
     for (auto& m : s->meshes) any_xform = any_xform || m.kind != vgpu::kXfNone;
-    // Default launch shape unless the caller chose one: the static and the motion kernel hold five waves per
-    // SIMD, so 20 waves per CU, with the LDS stack that measured fastest (figures at kExtLaunch and
-    // k_trace_wide_m5); scenes with transforms have one shape, of which the caller sets the waves.
+    // Default launch shape unless the caller chose one, the shading passes' one (figures at kExtLaunch and
+    // kExtLaunchMotion); scenes with transforms have one shape, of which the caller sets the waves.
+    auto default_shape = [](const vgpu::TraceLaunch& l) { return vgpu_trace_config{l.block, l.lds_depth, l.waves_per_cu, 0, 0}; };
     if (!s->cfg_set)
-        s->cfg = any_xform ? vgpu_trace_config{vgpu::kXformLaunch.block, vgpu::kXformLaunch.lds_depth, vgpu::kXformLaunch.waves_per_cu, 0, 0}
-                           : (s->any_motion ? vgpu_trace_config{64, 8, 20, 0, 0} : vgpu_trace_config{64, 12, 20, 0, 0});
+        s->cfg = any_xform ? default_shape(vgpu::kXformLaunch) : default_shape(s->any_motion ? vgpu::kExtLaunchMotion : vgpu::kExtLaunch);
 
     // Flatten into the device layout.
     std::vector<vgpu::DevNode> dnodes;

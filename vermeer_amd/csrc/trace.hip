@@ -939,9 +939,10 @@ __global__ __launch_bounds__(BLOCK) void k_trace_wide(VGPU_TRACE_PARAMS) {
     trace_wide<BLOCK, LDS, SHADOW, MOTION, COUNTERS, EXT>(VGPU_TRACE_ARGS);
 }
 
-// Motion scenes with a short LDS stack (8 or 12 entries): the box and triangle interpolation leave the
-// plain kernel above 100 VGPRs, four waves per SIMD.  Held to 96 (a few dwords of spill), five waves fit;
-// 1M camera rays among 2000 moving spheres take 650 us at 64 / 8 / 20 against 738 us with a grid of four.
+// Motion scenes with a short LDS stack (8 or 12 entries), where the caller chose one: the box and triangle
+// interpolation leave the plain kernel at 112 VGPRs, four waves per SIMD.  Held to 96 (four spilled), five waves fit; 1M
+// camera rays among 2000 moving spheres take 687 us at 64 / 8 / 20, the plain kernel on that grid 778 (but 617 on one
+// of 16 waves per CU, as kExtLaunchMotion's is).
 template <int BLOCK, int LDS, bool SHADOW, bool COUNTERS, bool EXT>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_wide_m5(VGPU_TRACE_PARAMS) {
     static_assert(LDS <= 12, "the five-wave motion kernel is built for short LDS stacks");

@@ -117,13 +117,15 @@ struct TraceLaunch {
     int spread = 16;    // waves per CU that a short launch is spread over (trace_ray_shift)
 };
 
-// Launch shapes of launch_trace_ext (the shading passes' closest-hit traversal) for static and
-// motion scenes; callers size the spill area for the larger grid.  The static kernel holds 88 VGPRs, five
-// waves per SIMD: a grid of 20 waves per CU fills them and leaves no workgroup waiting (2.1M bounce rays,
-// block 64: 725 us at 20 waves per CU, 786 at 16; block 128: 749 at 20, 780 at 24).
-// The motion shape runs the four-wave kernel: a pass over the moving spheres takes 843 us at 512^2, 1171 with five
-// segments at 320 x 199 and 2035 at 1024^2, in the five-wave kernel's shape (64, 8, 20) 864, 1215 and 2081 (64, 16, 16:
-// 841, 1159 and 2053).
+// Launch shapes of static and motion scenes: of launch_trace_ext (the shading passes' closest-hit traversal; callers
+// size the spill area for the larger grid) and of every other traversal where the caller chose none.
+// The static kernel holds 86 to 88 VGPRs, five waves per SIMD: a grid of 20 waves per CU fills them and leaves no
+// workgroup waiting (2.1M bounce rays, block 64: 706 us at 20 waves per CU, 743 at 16, 898 at 24; block 128: 703 at 20,
+// 910 at 24).
+// The motion shape runs the plain kernel (112 VGPRs, four waves per SIMD) and not k_trace_wide_m5, whose five waves
+// cost spills.  Among moving spheres, at 256 / 16 / 16 against 64 / 8 / 20, in us: 1M camera rays 591 against 687, 1M shadow
+// rays from them 533 against 633, 1M uniform shadow rays 758 against 1010 (967 in the kernel before its phases),
+// 20,011 uniform rays 130 against 176, 1,024 rays 59 against 76; a pass over 512^2 pixels 843 against 864.
 constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 

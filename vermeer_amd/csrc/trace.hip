@@ -939,16 +939,6 @@ __global__ __launch_bounds__(BLOCK) void k_trace_wide(VGPU_TRACE_PARAMS) {
     trace_wide<BLOCK, LDS, SHADOW, MOTION, COUNTERS, EXT>(VGPU_TRACE_ARGS);
 }
 
-// Motion scenes with a short LDS stack (8 or 12 entries), where the caller chose one: the box and triangle
-// interpolation leave the plain kernel at 112 VGPRs, four waves per SIMD.  Held to 96 (four spilled), five waves fit; 1M
-// camera rays among 2000 moving spheres take 687 us at 64 / 8 / 20, the plain kernel on that grid 778 (but 617 on one
-// of 16 waves per CU, as kExtLaunchMotion's is).
-template <int BLOCK, int LDS, bool SHADOW, bool COUNTERS, bool EXT>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_wide_m5(VGPU_TRACE_PARAMS) {
-    static_assert(LDS <= 12, "the five-wave motion kernel is built for short LDS stacks");
-    trace_wide<BLOCK, LDS, SHADOW, true, COUNTERS, EXT>(VGPU_TRACE_ARGS);
-}
-
 // Scenes holding GeomInstances, Procs or meshes with their own Transform.  Four waves per SIMD: the walk
 // over geoms takes registers, and its lanes wait for one another (kTurnWait).
 // 262,144 rays in a room of 60 instances: 670 us of kernel, 12 registers spilled.  With the transform inlined
@@ -979,17 +969,6 @@ template <int BLOCK, int LDS, bool SHADOW, bool MOTION>
 hipError_t launch_cfg(const SceneView& sv, const void* rays, uint64_t n, void* hits, int32_t* geoms, int32_t* counters,
                       float* spT, int32_t* spN, uint64_t grid, int32_t* err, const uint32_t* n_dev,
                       const uint32_t* perm, bool gather, hipStream_t stream, int ray_shift, int refill_min) {
-    if constexpr (MOTION && LDS <= 12) {
-        if (counters)
-            hipLaunchKernelGGL((k_trace_wide_m5<BLOCK, LDS, SHADOW, true, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
-                               stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)counters, spT, spN, err,
-                               n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
-        else
-            hipLaunchKernelGGL((k_trace_wide_m5<BLOCK, LDS, SHADOW, false, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
-                               stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)nullptr, spT, spN, err,
-                               n_dev, perm, gather ? 1 : 0, ray_shift, refill_min);
-        return hipGetLastError();
-    }
     if (counters)
         hipLaunchKernelGGL((k_trace_wide<BLOCK, LDS, SHADOW, MOTION, true, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
                            stream, sv, (const float4*)rays, n, (int4*)hits, geoms, (int4*)counters, spT, spN, err,

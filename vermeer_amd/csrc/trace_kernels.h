@@ -122,10 +122,10 @@ struct TraceLaunch {
 // The static kernel holds 86 to 88 VGPRs, five waves per SIMD: a grid of 20 waves per CU fills them and leaves no
 // workgroup waiting (2.1M bounce rays, block 64: 706 us at 20 waves per CU, 743 at 16, 898 at 24; block 128: 703 at 20,
 // 910 at 24).
-// The motion shape runs the plain kernel (112 VGPRs, four waves per SIMD) and not k_trace_wide_m5, whose five waves
-// cost spills.  Among moving spheres, at 256 / 16 / 16 against 64 / 8 / 20, in us: 1M camera rays 591 against 687, 1M shadow
-// rays from them 533 against 633, 1M uniform shadow rays 758 against 1010 (967 in the kernel before its phases),
-// 20,011 uniform rays 130 against 176, 1,024 rays 59 against 76; a pass over 512^2 pixels 843 against 864.
+// The motion kernel holds 112 VGPRs, four waves per SIMD.  Held to 96 (four spilled, and their reloads lie in the loop) it
+// fitted five, and was slower.  Among moving spheres, this shape against five waves at 64 / 8 / 20, in us: 1M camera rays
+// 591 against 687, 1M shadow rays from them 533 against 633, 1M uniform shadow rays 758 against 1010, 20,011 uniform
+// rays 130 against 176, 1,024 rays 59 against 76; a pass over 512^2 pixels 843 against 864.
 constexpr TraceLaunch kExtLaunch{64, 12, 20};
 constexpr TraceLaunch kExtLaunchMotion{256, 16, 16};
 

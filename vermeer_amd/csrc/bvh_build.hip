@@ -175,8 +175,8 @@ __device__ __forceinline__ uint32_t bin_join(int w, uint32_t x, uint32_t y) {
 // A wavefront's bins in LDS: COPIES copies, lane l adding to copy l % COPIES, since atomics on one address are
 // served one after another (about 8 cycles a lane).  Eight for the chunks of the device-wide splits (293 chunks
 // of 1024 elements: 25 us with one copy, 18 with eight), one for the subtrees, whose ranges are too short to
-// pay for more (147 subtrees: 220 us with one, 245 with eight).  Eight boxes per lane in registers cost 130
-// instructions an element and 288 shuffles a fold.
+// pay for more (k_subtree over 300,001 triangles: 220 us with one, 245 with eight, measured before its last permutation
+// stayed in registers).  Eight boxes per lane in registers cost 130 instructions an element and 288 shuffles a fold.
 constexpr int kBinStride = kBinWords + 1;   // the odd stride spreads the copies over the banks
 template <int COPIES>
 struct WaveBins {
@@ -446,8 +446,9 @@ __device__ void complete_node(SubLds& L, int me, vgpu_qbvh_node* nodes, float* r
 // root is complete (or the build is given up), which some wavefront always reaches, since a published node
 // waits for no other.  Finding order puts parents before children; the numbers follow from the subtree sizes.
 // One wavefront per subtree splitting in global memory, with eight bin boxes per lane folded through
-// shuffles, took 2270 us for the 147 subtrees of 300,001 triangles (a chain of 270 nodes at 8 us each);
-// this takes 220 us.
+// shuffles, took 2270 us for the 340 subtrees (882 elements and 39 nodes each on average) of 300,001 triangles of the
+// icosphere field; this takes 208 us.  What bounds it: SubLds fills a CU (141,100 bytes of 160 K), so on 256 CUs the 340
+// workgroups run in two rounds, and a subtree's nodes wait for one another near its root.
 __global__ __launch_bounds__(kSubThreads) void k_subtree(GElem* E_all, const int2* roots, vgpu_qbvh_node* nodes_all,
                                                          int* pre_all, int* counts, float* root_boxes, int leafMax,
                                                          int* err) {

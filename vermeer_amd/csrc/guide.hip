@@ -331,8 +331,8 @@ __device__ __forceinline__ float quad_sum(float v) {
     return v + __shfl_xor(v, 32);
 }
 
-// exp(x) for |x| <= 80: x log2 e in two parts, the hardware exp2 on what is left beside the nearest whole number
-// (on the whole argument it was off by 1.3e-7 instead of 8.4e-8).
+// exp(x) for |x| <= 80: Cody and Waite's reduction with x log2 e in two parts, the hardware exp2 on what is left beside
+// the nearest whole number (on the whole argument it was off by 1.3e-7 instead of 8.4e-8).
 __device__ __forceinline__ float exp_mid(float x) {
     const float L = 1.44269504f, LL = 1.92596299e-8f;          // log2 e = L + LL
     const float h = x * L, e = rintf(h);
@@ -340,7 +340,7 @@ __device__ __forceinline__ float exp_mid(float x) {
     return __builtin_ldexpf(__builtin_amdgcn_exp2f((h - e) + l), (int)e);
 }
 
-// A lobe from its five outputs, for inference.  One Newton step on the hardware reciprocal square root stands
+// A lobe from its five outputs, for inference.  One Newton-Raphson step on the hardware reciprocal square root stands
 // for a rounded square root and division; squares whose sum leaves the middle of the range take those.
 __device__ __forceinline__ void decode_lobe(const float* v, LobeD& L) {
     const float q = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
@@ -362,7 +362,7 @@ __device__ __forceinline__ void decode_lobe(const float* v, LobeD& L) {
 }
 // exp of a logit less the largest (never above 0; the rest, NaN too, by the library's function)
 __device__ __forceinline__ float exp_weight(float x) { return x >= -80.0f ? exp_mid(x) : expf(x); }
-// a / z rounded, from iz, the Newton-corrected reciprocal of z
+// a / z rounded, from iz, the Newton-corrected reciprocal of z: the quotient corrected by its remainder (Markstein)
 __device__ __forceinline__ float div_by(float a, float z, float iz) {
     const float w = a * iz;
     return __builtin_fmaf(__builtin_fmaf(-z, w, a), iz, w);
@@ -393,9 +393,9 @@ __device__ __forceinline__ float dlog_norm_fast(float k) {
 }
 // ---------------------------------------------------------------- inference
 
-// 1M queries: 89 us of kernel (119 before; VALU issue takes 61% of the cycles, the matrix units 26%): every lane has its own encoded features (encode), the biases lie in
-// LDS, the decode needs no full division, square root or exp, and the next queries are fetched ahead.  Two tiles
-// per wave: three and four were no faster.
+// 1M queries: 90 us of kernel (119 before; VALU issue takes 60% of the cycles, the matrix units 26%): every lane has
+// its own encoded features (encode), the biases lie in LDS, the decode needs no full division, square root or exp, and
+// the next queries are fetched ahead.  Two tiles per wave: three and four were no faster.
 // Three waves per SIMD, as the LDS allows; said to the compiler, it also keeps the accumulators in VGPRs (with
 // room for 512 registers it moved every result through an AGPR, 130 of 667 VALU instructions per iteration).
 template <bool RAW>

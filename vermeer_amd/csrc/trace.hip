@@ -16,8 +16,8 @@
 // The traversal stack (the reference's RenderTask.Traversal.Stack, shared by
 // both levels, core/ray.go:153-162) lives in LDS for its first LDS entries,
 // laid out lane-minor ([depth][lane]) so lanes never conflict on a bank;
-// deeper entries spill to a per-thread HBM region, also lane-minor so that
-// lanes at equal depth coalesce.
+// deeper entries spill to HBM, a column per lane that can own a ray
+// (trace_spill_columns), also lane-minor so that lanes at equal depth coalesce.
 //
 // Compiled with -ffp-contract=off: every float operation rounds as the
 // reference's unfused SSE code does.
@@ -553,9 +553,9 @@ constexpr int kIdle = -2;   // no ray, or its traversal has ended
 // The wavefront tests the leaves its lanes hold once kLeafRatio times as many lanes hold a leaf as hold a
 // node: few waiting leaves cost less than a node step with idle lanes while most lanes hold nodes, more as
 // the node lanes run out.  Measured on the icosphere field (2.1M bounce rays) / the 1M-triangle room (one
-// plain 1024^2 pass) / the box of spheres (320 x 199, depth 5), in us: ratio 3: 703 / 8282 / 1780, 5: 705 /
-// 8448 / 1799, 8: 704 / 8713 / 1823; a fixed count of 2 lanes: 725 / 9044 / 1880, 4: 726 / 8564 / 1890, 10:
-// 743 / 8211 / 2030.
+// plain 1024^2 pass) / the box of spheres (320 x 199, depth 5), in us: ratio 2: 709 / 7930 / 1606, 3: 705 / 8009 /
+// 1615, 5: 714 / 8184 / 1634, 8: 708 / 8429 / 1659; a fixed count of 2 lanes: 732 / 9046 / 1667, 4: 730 / 8468 /
+// 1638, 10: 743 / 8144 / 1705.  Moving spheres (1M camera rays): 586 at 2, 592 at 3, 599 at 5.
 constexpr int kLeafRatio = 3;
 
 // The traversal, one ray per lane.  A lane holds the node it visits next, a leaf of triangles it has
@@ -565,7 +565,7 @@ constexpr int kLeafRatio = 3;
 // is the reference's, whatever the other lanes do.
 //
 // What bounds it is VALU issue: 2.1M bounce rays in the icosphere field took 4.4e8 VALU instructions, 80%
-// of the issue slots of 902 us, when every turn ran both phases; now 3.0e8 and 65% of 703 us (2.98
+// of the issue slots of 902 us, when every turn ran both phases; now 2.85e8 and 66% of 705 us (2.97
 // Grays/s), the rest waiting for nodes and triangles beyond L2.  Hence the forms below: near and far planes
 // by address instead of sorted pairs (box4_near), stack positions as byte offsets summed from hit flags,
 // one 8-byte LDS entry per push, DPP scans, the workers' results handed to the owners instead of a second

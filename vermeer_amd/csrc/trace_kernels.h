@@ -183,8 +183,8 @@ hipError_t launch_trace_ext(const SceneView& sv, bool motion, const void* rays, 
 
 // Rays that a wavefront takes at a time, as a shift: 64, or fewer when that would leave wavefronts for fewer
 // than cfg.spread per CU.  A short launch lasts as long as its slowest wavefront, and one with fewer rays
-// diverges less, its idle lanes working in the leaf tests: 4096 pinhole rays over the sphere take 45 us
-// instead of 69, 50,000 bounce rays 63 instead of 75, 1024 rays among moving spheres 106 instead of 181.
+// diverges less, its idle lanes working in the leaf tests: 4096 pinhole rays over the sphere take 47 us
+// instead of 72, 50,000 bounce rays in the field 86 instead of 101, 1024 rays among moving spheres 59 instead of 107.
 int trace_ray_shift(const TraceLaunch& cfg, uint64_t n, int num_cus);
 // Spill columns of a launch: a lane that can own a ray has one.  A column per launched thread made the spill area of
 // a short launch four times as large as its rays need, and its allocation is part of a scene's first pass
@@ -192,7 +192,7 @@ int trace_ray_shift(const TraceLaunch& cfg, uint64_t n, int num_cus);
 // every shape, so an area sized by one shape serves a launch of as many rays by a shape with no more waves.
 uint64_t trace_spill_columns(const TraceLaunch& cfg, uint64_t n, int num_cus);
 
-// Threads the launch above will use (so the caller can size the spill area).
+// Threads of a launch.
 uint64_t trace_grid_threads(const TraceLaunch& cfg, uint64_t n, int num_cus);
 
 // Allocation-free traversal (vgpu_trace_noalloc): the spill area and error flag live in a
@@ -201,7 +201,7 @@ constexpr uint64_t kNoAllocScratchBytes = 128ull << 20;
 constexpr int kNoAllocMaxDevices = 64;
 // Looks the array up on `device`, which must be current; once per device (later calls return at once).
 hipError_t noalloc_init(int device);
-// Threads whose spill columns fit the array at LDS depth lds_depth.
+// Spill columns that fit the array at LDS depth lds_depth.
 uint64_t noalloc_max_columns(int lds_depth);
 // Clears the error flag (status, or the array's own flag word when status is NULL) with a kernel,
 // then enqueues launch_trace with the array as its spill area.  The grid of cfg must fit
